@@ -1,0 +1,102 @@
+"""The persistent lanes' leaf and intersection queues at their edges, through the C-ABI against
+the oracle: every geometry mode, leaves of 1 to 3 records (a node test can yield 24), ray counts
+around the 64-lane wavefront, equal hits of several instances and rays with a negative tmin."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def G():
+    import gpu_util
+    return gpu_util
+
+
+@pytest.fixture(scope="module")
+def curves():
+    import scenes
+    return scenes.dense_ball_curves(nstrands=300)
+
+
+def _add(S, oracle, G, ctx, mode, curves, leaf_size=0, transform=None):
+    """One instance of `curves` in a mode: into the oracle scene, and as a BLAS."""
+    import scenes
+    import vkhrt_amd as V
+    if mode == "mesh":
+        import torch
+        verts, idx = scenes.uv_sphere(11.0, 24, 48)
+        S.add_mesh(verts, idx, transform=transform)
+        dv, di = G.dev(verts), G.dev(idx)
+        b = V.BottomLevelAccelerationStructure(ctx, V.GEOMETRY_TRIANGLES, dv.data_ptr(), idx.shape[0],
+                                               indices_ptr=di.data_ptr(), vertex_count=verts.shape[0],
+                                               leaf_size=leaf_size, transform=transform, stream=G.stream_ptr())
+        torch.cuda.synchronize()
+        return b
+    if mode.startswith("phantom"):
+        point = mode == "phantom"
+        S.add(oracle.MODE_PHANTOM, curves, per_point=point, transform=transform)
+        return G.build_blas(ctx, V.GEOMETRY_PHANTOM_CURVES, curves, per_point=point, leaf_size=leaf_size,
+                            transform=transform)
+    lines = scenes.lines_from_curves(curves, 4)
+    if mode == "lss":
+        prims = oracle.generate_lss(lines)
+        S.add(oracle.MODE_LSS, prims, transform=transform)
+        return G.build_blas(ctx, V.GEOMETRY_LSS, prims, leaf_size=leaf_size, transform=transform)
+    S.add(oracle.MODE_DOTS, lines, per_point=True, transform=transform)
+    return G.build_blas(ctx, V.GEOMETRY_DOTS, lines, per_point=True, leaf_size=leaf_size, transform=transform)
+
+
+@pytest.mark.parametrize("count", [1, 63, 64, 65, 4097])
+@pytest.mark.parametrize("modes,leaf", [(("phantom",), 3), (("lss",), 1), (("lss",), 3), (("dots",), 2), (("mesh",), 3),
+                                        (("phantom", "mesh"), 2), (("phantom", "phantom const", "lss", "dots", "mesh"), 3)])
+def test_lanes_match_oracle(gpu_ctx, G, oracle, curves, modes, leaf, count):
+    import scenes
+    import vkhrt_amd as V
+    S = oracle.Scene()
+    tlas = V.TopLevelAccelerationStructure(gpu_ctx, [_add(S, oracle, G, gpu_ctx, m, curves, leaf) for m in modes])
+    rays = scenes.targeted_rays(curves, count, seed=31, dist=(1.0, 60.0))
+    assert (S.trace(rays)["prim"] != 0xFFFFFFFF).sum() * 4 > count or count < 64
+    G.compare_hits(G.trace(gpu_ctx, tlas, rays), S.trace(rays), f"{modes} x {count}")
+    g = G.trace(gpu_ctx, tlas, rays, flags=V.TRACE_TERMINATE_ON_FIRST_HIT)
+    r = S.trace(rays, flags=oracle.F_ANY_HIT)
+    assert np.array_equal(g["prim"] == 0xFFFFFFFF, r["prim"] == 0xFFFFFFFF)
+    polish = S.trace(rays, flags=oracle.F_POLISH)
+    G.compare_hits(G.trace(gpu_ctx, tlas, rays, flags=V.TRACE_FP64_POLISH), polish, f"{modes} x {count}, polished")
+
+
+@pytest.mark.parametrize("copies", [2, 17])
+@pytest.mark.parametrize("mode", ["phantom", "lss", "dots", "mesh"])
+def test_equal_hits_of_instances(gpu_ctx, G, oracle, curves, mode, copies):
+    """The same geometry several times over: equal t goes to the lowest instance (up to 16
+    instances are staged in LDS, more are not), with another mode's instance among them."""
+    import scenes
+    import vkhrt_amd as V
+    other = "mesh" if mode != "mesh" else "lss"
+    far = np.array([1, 0, 0, 40.0, 0, 1, 0, 0, 0, 0, 1, 0], np.float32)
+    for extra in (False, True):
+        S = oracle.Scene()
+        blases = [_add(S, oracle, G, gpu_ctx, other, curves, transform=far)] if extra else []
+        blases += [_add(S, oracle, G, gpu_ctx, mode, curves) for _ in range(copies)]
+        tlas = V.TopLevelAccelerationStructure(gpu_ctx, blases)
+        rays = scenes.targeted_rays(curves, 1500, seed=32, dist=(1.0, 60.0))
+        ref = S.trace(rays)
+        assert set(np.unique(ref["inst"])) >= {int(extra)}
+        G.compare_hits(G.trace(gpu_ctx, tlas, rays), ref, f"{copies} x {mode}")
+
+
+@pytest.mark.parametrize("mode", ["lss", "dots", "mesh", "phantom"])
+def test_negative_tmin(gpu_ctx, G, oracle, curves, mode):
+    """Hits behind the origin (t < 0) order like the others: rays from inside the hair whose
+    interval starts 40 units behind them."""
+    import scenes
+    import vkhrt_amd as V
+    S = oracle.Scene()
+    tlas = V.TopLevelAccelerationStructure(gpu_ctx, [_add(S, oracle, G, gpu_ctx, mode, curves)])
+    rays = scenes.targeted_rays(curves, 3000, seed=33, dist=(-25.0, 25.0))
+    rays[:, 3] = -40.0
+    rays[:, 7] = 30.0
+    ref = S.trace(rays)
+    if mode != "phantom":  # a phantom hit lies in front of the origin
+        assert (ref["t"][ref["prim"] != 0xFFFFFFFF] < 0).sum() > 100
+    G.compare_hits(G.trace(gpu_ctx, tlas, rays), ref, f"{mode}, negative tmin")

@@ -13,7 +13,8 @@ LIB = os.path.join(HERE, "libvkhrt.so")
 OBJ_COUNT = os.path.join(HERE, "_build_count")
 LIB_COUNT = os.path.join(HERE, "libvkhrt_count.so")
 SOURCES = ["api.cpp", "asset.cpp", "noalloc.cpp", "bvh_build.hip", "geometry.hip", "voxel.hip", "trace.hip", "trace_phantom_const.hip",
-           "trace_phantom_point.hip", "trace_lss.hip", "trace_dots.hip", "trace_tris.hip", "trace_mixed.hip", "mlp.hip"]
+           "trace_phantom_point.hip", "trace_lss.hip", "trace_dots.hip", "trace_tris.hip", "trace_mixed.hip", "trace_multi.hip",
+           "mlp.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 

@@ -199,9 +199,14 @@ uint64_t blas_id_range(const vkhrt_blas* b) {
     return b->records;
 }
 
-// Kernel variant for a TLAS and the polish flag.
-int trace_variant(const vkhrt_tlas* t, bool polish) {
+// Kernel variant for a TLAS and the polish flag. A TLAS of several BVH modes takes the persistent
+// lanes where they run (`lanes`); voxel instances have no BVH to walk, and leaf slots past the
+// queue encoding keep one thread per ray.
+int trace_variant(const vkhrt_tlas* t, bool polish, bool lanes) {
     int v = t->variant;
+    if (v == vk::kVarMixed && lanes && t->polish_ok &&
+        std::find(t->modes.begin(), t->modes.end(), uint32_t(VKHRT_GEOMETRY_VOXELS)) == t->modes.end())
+        v = vk::kVarMulti;
     if (polish && (v == vk::kVarPhConst || v == vk::kVarPhPoint)) ++v;
     return v;
 }
@@ -1220,7 +1225,7 @@ int trace_launch(vkhrt_context* c, const vkhrt_tlas* t, const vkhrt_ray* rays, u
     }
     Timer tm(c, st, timed ? "trace_rays" : nullptr);
     hipError_t e = vk::launch_trace_rays(tp, reinterpret_cast<const float*>(rays), count,
-                                         reinterpret_cast<vk::HitRec*>(hits), nullptr, trace_variant(t, polish),
+                                         reinterpret_cast<vk::HitRec*>(hits), nullptr, trace_variant(t, polish, tp.work != nullptr),
                                          stack_kind_for(c, t), st);
     if (e == hipSuccess && accurate)
         e = vk::launch_accurate_hits(tp, reinterpret_cast<const float*>(rays), count, reinterpret_cast<vk::HitRec*>(hits),
@@ -1364,7 +1369,7 @@ int vkhrt_render(vkhrt_context* c, const vkhrt_tlas* t, const vkhrt_camera* cam,
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     if (c->profiling)
         for (auto& x : ev) hipEventCreate(&x);
-    hipError_t e = vk::launch_render(rp, trace_variant(t, (d->flags & VKHRT_RENDER_FP64_POLISH) != 0),
+    hipError_t e = vk::launch_render(rp, trace_variant(t, (d->flags & VKHRT_RENDER_FP64_POLISH) != 0, rp.tp.work != nullptr),
                                      stack_kind_for(c, t), st, c->profiling ? ev : nullptr);
     if (c->profiling) {
         c->pending.push_back(PendingTiming{"render_primary", ev[0], ev[1]});
@@ -1532,7 +1537,7 @@ int vkhrt_render_batch(vkhrt_context* c, const vkhrt_tlas* t, const vkhrt_view* 
     bp.order = c->b_order;
     bp.squeue = c->b_squeue;
     bp.counters = c->b_counters;
-    const int variant = trace_variant(t, polish), stack = stack_kind_for(c, t);
+    const int variant = trace_variant(t, polish, true), stack = stack_kind_for(c, t);
 
     hipEvent_t ev[2] = {nullptr, nullptr};
     if (c->profiling) {

@@ -191,7 +191,7 @@ __global__ __launch_bounds__(kAppendBlock) void k_batch_primary(BatchParams bp) 
 // Closest hit of the depth-b queue: hit record per queue slot (and the merge key when
 // grazing roots are deferred to the FP64 polish).
 template <class G, int STACK, int IM>
-__global__ __launch_bounds__(kTraceBlock) void k_batch_trace(BatchParams bp, uint32_t b) {
+__global__ __launch_bounds__(kTraceBlock, lanes_waves(STACK)) void k_batch_trace(BatchParams bp, uint32_t b) {
     __shared__ uint2 stk[STACK * kTraceBlock];
     const uint32_t* q = depth_queue(bp, b);
     persistent_lanes<G, false, STACK, IM>(
@@ -209,13 +209,13 @@ __global__ __launch_bounds__(kTraceBlock) void k_batch_trace(BatchParams bp, uin
             HitRec h;
             finish_hit(bp.tp, o, d, best, h);
             bp.hits[qi] = h;
-            if (G::kPolish) bp.tp.keys[qi] = best_key(bp.tp, best);
+            if (G::kPolish || (G::kMixed && bp.tp.keys)) bp.tp.keys[qi] = best_key(bp.tp, best);
         },
         bp.counters + batch_xcd(b, 0));
 }
 
-// Mixed-mode TLASes (per-instance geometry dispatch): one lane per queue slot, the queue length
-// read on the device; the grid covers every path.
+// TLASes with voxel instances (per-instance geometry dispatch): one lane per queue slot, the queue
+// length read on the device; the grid covers every path.
 template <class G, int STACK>
 __global__ __launch_bounds__(kTraceBlock) void k_batch_trace_flat(BatchParams bp, uint32_t b) {
     __shared__ uint2 stk[STACK * kTraceBlock];
@@ -384,7 +384,7 @@ __global__ __launch_bounds__(kAppendBlock) void k_batch_shade(BatchParams bp, ui
 
 // Shadow rays of depth b (any hit): visibility into nee.w.
 template <class G, int STACK, int IM>
-__global__ __launch_bounds__(kTraceBlock) void k_batch_shadow(BatchParams bp, uint32_t b) {
+__global__ __launch_bounds__(kTraceBlock, lanes_waves(STACK)) void k_batch_shadow(BatchParams bp, uint32_t b) {
     __shared__ uint2 stk[STACK * kTraceBlock];
     const SrcBatchShadow src{bp.squeue, bp.ray};
     persistent_lanes<G, true, STACK, IM>(
@@ -454,6 +454,7 @@ hipError_t launch_batch_variant(const BatchParams& bp0, hipStream_t st) {
         hipLaunchKernelGGL(k_zero, dim3((kBatchCounterWords + 255) / 256), dim3(256), 0, st, bp0.counters,
                            kBatchCounterWords);
         const int im = instance_mode(bp0.tp.ninst);  // how the traversal reaches the BLAS fields
+        constexpr int kOne = G::kMixed ? kInstFew : kInstOne;  // several modes come with several instances
         hipLaunchKernelGGL(k_batch_primary, all, ab, 0, st, bp0);
         for (uint32_t b = 0; b <= bp0.bounces; ++b) {
             BatchParams bp = bp0;
@@ -464,12 +465,12 @@ hipError_t launch_batch_variant(const BatchParams& bp0, hipStream_t st) {
                 hipLaunchKernelGGL(k_batch_ray_scatter, strided, ab, 0, st, bp, b);
             }
             bp.tp.defer_count = bp0.counters + bc(b, kBcDefer);
-            if constexpr (G::kMixed)
+            if constexpr (!G::kCompact)
                 hipLaunchKernelGGL((k_batch_trace_flat<G, STACK>), dim3((total + kTraceBlock - 1) / kTraceBlock), tb, 0,
                                    st, bp, b);
             else if (im == kInstOne)
-                hipLaunchKernelGGL((k_batch_trace<G, STACK, kInstOne>),
-                                   persistent_grid(k_batch_trace<G, STACK, kInstOne>, bp.tp.blocks_per_cu), tb, 0, st, bp, b);
+                hipLaunchKernelGGL((k_batch_trace<G, STACK, kOne>),
+                                   persistent_grid(k_batch_trace<G, STACK, kOne>, bp.tp.blocks_per_cu), tb, 0, st, bp, b);
             else if (im == kInstFew)
                 hipLaunchKernelGGL((k_batch_trace<G, STACK, kInstFew>),
                                    persistent_grid(k_batch_trace<G, STACK, kInstFew>, bp.tp.blocks_per_cu), tb, 0, st, bp, b);
@@ -489,12 +490,12 @@ hipError_t launch_batch_variant(const BatchParams& bp0, hipStream_t st) {
             }
             hipLaunchKernelGGL(k_batch_shade, strided, ab, 0, st, bp, b);
             bp.tp.defer_count = bp0.counters + bc(b, kBcDeferShadow);
-            if constexpr (G::kMixed)
+            if constexpr (!G::kCompact)
                 hipLaunchKernelGGL((k_batch_shadow_flat<G, STACK>), dim3((total + kTraceBlock - 1) / kTraceBlock), tb, 0,
                                    st, bp, b);
             else if (im == kInstOne)
-                hipLaunchKernelGGL((k_batch_shadow<G, STACK, kInstOne>),
-                                   persistent_grid(k_batch_shadow<G, STACK, kInstOne>, bp.tp.blocks_per_cu), tb, 0, st, bp,
+                hipLaunchKernelGGL((k_batch_shadow<G, STACK, kOne>),
+                                   persistent_grid(k_batch_shadow<G, STACK, kOne>, bp.tp.blocks_per_cu), tb, 0, st, bp,
                                    b);
             else if (im == kInstFew)
                 hipLaunchKernelGGL((k_batch_shadow<G, STACK, kInstFew>),

@@ -162,7 +162,8 @@ struct RenderParams {
 };
 
 // Compile-time geometry variants of the traversal kernels. A TLAS whose instances share
-// one mode uses the matching specialized kernels; mixed TLASes use kVarMixed.
+// one mode uses the matching specialized kernels; one that mixes BVH modes kVarMulti (the
+// persistent lanes), one with voxel instances kVarMixed (one thread per ray).
 enum TraceVariant {
     kVarPhConst = 0,
     kVarPhConstPolish = 1,
@@ -171,7 +172,8 @@ enum TraceVariant {
     kVarLss = 4,
     kVarDots = 5,
     kVarMixed = 6,
-    kVarTris = 7
+    kVarTris = 7,
+    kVarMulti = 8
 };
 
 // ---- batched path tracing: many views of one TLAS in one wavefront pipeline

@@ -12,7 +12,8 @@
 
 namespace vk {
 
-enum RadiusModeDev { kRadiusConstant = 0, kRadiusPerPoint = 1 };
+// kRadiusRuntime: the model is an argument (TLASes whose phantom BLASes may differ in it)
+enum RadiusModeDev { kRadiusConstant = 0, kRadiusPerPoint = 1, kRadiusRuntime = -1 };
 
 struct RayFrame {
     f3 o, d;      // ray in the primitive's space
@@ -132,7 +133,8 @@ struct PhantomHit {
 // FP64 polish handling inside Prhi: off, evaluated in place, or deferred (the FP32 pass
 // stops at the first side that would enter the FP64 continuation and flags the curve; a
 // later kernel re-runs the full Prhi with kPolishInline for flagged ray/curve pairs).
-enum PolishMode { kPolishOff = 0, kPolishInline = 1, kPolishDefer = 2 };
+// kPolishRuntime: deferred or off by an argument.
+enum PolishMode { kPolishOff = 0, kPolishInline = 1, kPolishDefer = 2, kPolishRuntime = 3 };
 
 // One side of the Prhi iteration (hair_intersection.rint:46-116) on an RCC-space curve.
 template <class V, class R>
@@ -228,9 +230,10 @@ __device__ __forceinline__ bool prhi_polish_f64(f3 of, f3 df, const float4* cv, 
 // `rmax` is the curve's early-out cylinder radius (:21-22), precomputed per curve at build
 // time with the same arithmetic. CULL = false skips that test for callers that ran it already.
 template <int RMODE, int PMODE, bool CULL = true>
-__device__ __forceinline__ bool prhi(const RayFrame& F, const float4* cv, float rmax, float const_r, PhantomHit& out) {
+__device__ __forceinline__ bool prhi(const RayFrame& F, const float4* cv, float rmax, float const_r, PhantomHit& out,
+                                     int rt_radius_mode = 0, bool rt_defer = false) {
     out.deferred = false;
-    constexpr int radius_mode = RMODE;
+    const int radius_mode = RMODE == kRadiusRuntime ? rt_radius_mode : RMODE;
     const f3 p0 = f3{cv[0].x, cv[0].y, cv[0].z}, p1 = f3{cv[1].x, cv[1].y, cv[1].z};
     const f3 p2 = f3{cv[2].x, cv[2].y, cv[2].z}, p3 = f3{cv[3].x, cv[3].y, cv[3].z};
     // early out (:24-33)
@@ -257,7 +260,11 @@ __device__ __forceinline__ bool prhi(const RayFrame& F, const float4* cv, float 
                 return true;
             }
         } else if (PMODE != kPolishOff && st == 3 && t >= 0.0f && t <= 1.0f && fabsf(last) < 0.05f) {
-            if (PMODE == kPolishDefer) {
+            if (PMODE == kPolishRuntime && !rt_defer) {
+                tStart = 1.0f - tStart;
+                continue;
+            }
+            if (PMODE == kPolishDefer || PMODE == kPolishRuntime) {
                 out.deferred = true;
                 return false;
             }

@@ -35,6 +35,7 @@ VKHRT_DECLARE_VARIANT(PhPointPolish)
 VKHRT_DECLARE_VARIANT(LssG)
 VKHRT_DECLARE_VARIANT(DotsG)
 VKHRT_DECLARE_VARIANT(TrisG)
+VKHRT_DECLARE_VARIANT(GeoMulti)
 VKHRT_DECLARE_VARIANT(GeoMixed)
 
 namespace {
@@ -71,6 +72,7 @@ hipError_t launch_batch(const BatchParams& bp, int variant, int stack_kind, hipS
         case kVarLss: return batch_stack<LssG>(bp, stack_kind, st);
         case kVarDots: return batch_stack<DotsG>(bp, stack_kind, st);
         case kVarTris: return batch_stack<TrisG>(bp, stack_kind, st);
+        case kVarMulti: return batch_stack<GeoMulti>(bp, stack_kind, st);
         default: return batch_stack<GeoMixed>(bp, stack_kind, st);
     }
 }
@@ -85,6 +87,7 @@ hipError_t launch_trace_rays(const TraceParams& tp, const float* rays, uint32_t 
         case kVarLss: return trace_stack<LssG>(tp, rays, n, hits, stats, stack_kind, st);
         case kVarDots: return trace_stack<DotsG>(tp, rays, n, hits, stats, stack_kind, st);
         case kVarTris: return trace_stack<TrisG>(tp, rays, n, hits, stats, stack_kind, st);
+        case kVarMulti: return trace_stack<GeoMulti>(tp, rays, n, hits, stats, stack_kind, st);
         default: return trace_stack<GeoMixed>(tp, rays, n, hits, stats, stack_kind, st);
     }
 }
@@ -98,6 +101,7 @@ hipError_t launch_render(const RenderParams& rp, int variant, int stack_kind, hi
         case kVarLss: return render_stack<LssG>(rp, stack_kind, st, ev);
         case kVarDots: return render_stack<DotsG>(rp, stack_kind, st, ev);
         case kVarTris: return render_stack<TrisG>(rp, stack_kind, st, ev);
+        case kVarMulti: return render_stack<GeoMulti>(rp, stack_kind, st, ev);
         default: return render_stack<GeoMixed>(rp, stack_kind, st, ev);
     }
 }

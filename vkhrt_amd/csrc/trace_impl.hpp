@@ -24,13 +24,20 @@ namespace vk {
 // Geometry variant of a traversal kernel.
 template <int MODE_, int RMODE_, bool POLISH_>
 struct Geo {
-    static constexpr bool kMixed = false;
+    static constexpr bool kMixed = false, kCompact = true;
     static constexpr int kMode = MODE_, kRMode = RMODE_;
     static constexpr bool kPolish = POLISH_;
 };
-// Instances of different modes in one TLAS: runtime dispatch per instance.
+// Instances of different modes in one TLAS, the mode read per instance. GeoMulti: BVH instances
+// only, walked by the compacted persistent lanes. GeoMixed: any instances (voxel grids have no
+// BVH), one thread per ray with trace_world's dispatch.
+struct GeoMulti {
+    static constexpr bool kMixed = true, kCompact = true;
+    static constexpr int kMode = -1, kRMode = 0;
+    static constexpr bool kPolish = false;
+};
 struct GeoMixed {
-    static constexpr bool kMixed = true;
+    static constexpr bool kMixed = true, kCompact = false;
     static constexpr int kMode = -1, kRMode = 0;
     static constexpr bool kPolish = false;
 };
@@ -945,115 +952,51 @@ struct WorkClaim {
     }
 };
 
-// Persistent wavefronts with per-lane refill: every iteration each active lane performs one
-// walker step; lanes whose ray finished take new work from a global counter (one atomic per
-// wave per refill), so a wavefront is not held back by its slowest ray. src(r, id, o, d, tmin,
-// tmax) produces work item r and names its ray `id` (the index results and deferred-polish
-// entries use); snk(id, o, d, best) consumes the result (called by the lanes that finish in
-// the same iteration, so it may use wave ballots).
-template <class G, bool ANY, int STACK, int IM, class Src, class Snk>
-__device__ __forceinline__ void persistent_generic(const TraceParams& tp, WorkClaim& work, uint2* lds, Src&& src,
-                                                   Snk&& snk) {
-    BlasDev b1{};  // one instance: as in persistent_compact (a few: read per lane here)
-    if constexpr (IM == kInstOne) b1 = wave_uniform(tp.inst[0].blas);
-    static_assert(!G::kMixed, "persistent kernels serve single-mode TLASes");
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint64_t lt = (1ull << lane) - 1ull;
-    Walker<G::kMode, G::kRMode, G::kPolish, ANY, STACK> W;
-    Best best;
-    f3 ow = f3{0, 0, 0}, dw = f3{0, 0, 0};
-    float tmin = 0.0f, tmax = 0.0f;
-    uint32_t idx = 0, inst = 0;
-    bool active = false, need_inst = false;
-    for (;;) {
-        if (!work.exhausted) {
-            const uint64_t idle = __ballot(!active);
-            if (idle && (__popcll(idle) >= tp.refill_min || idle == __ballot(true))) {
-                const uint32_t r = work.claim(idle, __popcll(idle & lt));
-                if (!active) {
-                    if (r < work.total) {
-                        src(r, idx, ow, dw, tmin, tmax);
-                        best.t = tmax;
-                        best.inst = 0xFFFFFFFFu;
-                        best.pid = 0xFFFFFFFFu;
-                        best.slot = 0xFFFFFFFFu;
-                        best.u = best.a = best.b = best.c = 0.0f;
-                        best.extra = 0;
-                        inst = 0;
-                        need_inst = true;
-                        active = true;
-                    }
-                }
-            }
-        }
-        if (!__ballot(active)) break;
-        bool finish = false;
-        if (active && need_inst) {
-            // next instance whose world box the ray overlaps (top_level_acceleration_structure.cpp:23-43)
-            while (inst < tp.ninst) {
-                const InstanceDev& I = tp.inst[inst];
-                if (I.blas.nprims != 0 && ray_box(ow, dw, I.lo, I.hi, tmin, best.t)) break;
-                ++inst;
-            }
-            if (inst >= tp.ninst) {
-                finish = true;
-            } else {
-                const InstanceDev& I = tp.inst[inst];
-                f3 oo = ow, dd = dw;
-                if (!I.identity) {
-                    oo = xform_pt(I.inv, ow);
-                    dd = xform_dir(I.inv, dw);
-                }
-                W.begin(oo, dd);
-                need_inst = false;
-            }
-        }
-        // up to tp.steps_per_iter traversal steps before the refill and finish bookkeeping again
-        const uint32_t nsteps = tp.steps_per_iter > 1u ? tp.steps_per_iter : 1u;
-        for (uint32_t si = 0; si < nsteps; ++si) {
-            const bool walk = active && !need_inst && !finish;
-            if (si > 0u && !__ballot(walk)) break;
-            if (walk) {
-                const int r = W.step(IM == kInstOne ? b1 : tp.inst[inst].blas, tmin, inst, best, lds, nullptr, tp, idx);
-                if (r == kStepError) {
-                    atomicAdd(&tp.status[0], 1u);
-                    finish = true;
-                } else if (r == kStepHit) {
-                    finish = true;
-                } else if (r == kStepDone) {
-                    ++inst;
-                    need_inst = true;
-                }
-            }
-        }
-        if (active && finish) {
-            snk(idx, ow, dw, best);
-            active = false;
-        }
-    }
-}
-
-// ------------------------------------------------------------------ compacted phantom lanes
-// Phantom persistent loop with wave-level compaction of the intersection work. Lanes run one
-// traversal step per iteration: a node test, or one leaf record through the capped-cylinder
-// early-out (hair_intersection.rint:24-33). A (lane, leaf slot) pair that survives the
-// early-out is appended to a per-wave queue in LDS. When the queue holds 64 pairs, or no
-// lane can traverse, every lane of the wave takes one pair and runs the rest of Prhi on the
-// owner's ray (read with cross-lane permutes), so the iteration loop runs on full
-// wavefronts instead of on the few lanes that happen to sit at a leaf. Results merge into the
-// owner's LDS slot by a 64-bit atomicMin on (t, instance, primitive): that minimum is unique,
-// so the closest hit and its tie rule do not depend on the processing order. A lane does not
-// move to its next instance, finish or take a new ray while pairs of its ray are queued.
-constexpr uint32_t kCompactQueue = 128;    // per wave: < 64 left after a round + <= 64 appended per step
+// ------------------------------------------------------------------ compacted persistent lanes
+// Persistent loop with per-lane refill and wave-level compaction of the leaf work. Walking lanes
+// only test nodes; the (lane, leaf slot) pairs that a node test yields are appended to a per-wave
+// leaf queue in LDS. When that queue holds 64 pairs, or no lane can walk, every lane of the wave
+// takes one pair and tests the record against its owner's ray (read with cross-lane permutes):
+// the whole intersection for LSS, DOTS and triangles, the capped-cylinder early-out
+// (hair_intersection.rint:24-33) for phantom curves. The phantom pairs that survive go on to a
+// second queue, whose rounds run the rest of Prhi the same way. So neither the record tests nor
+// the iteration run for the few lanes that happen to sit at a leaf while the others wait: a leaf
+// hit is yielded by about every fifth node test, so nearly every step of a 64-lane wave had one.
+// 1080p frames of 100k strands, us, before (phantom: early-out tests inside the steps; LSS and
+// DOTS: whole tests inside the steps; several modes: one thread per ray) and now: phantom 1650 ->
+// 1426 (accurate), LSS 1306 -> 758, DOTS 1411 -> 789, hair on a mesh 6457 -> 1650; bound by the
+// VALU work of the node tests.
+// Results merge into the owner's LDS slot by a 64-bit atomicMin on (t, primitive) of the current
+// instance: that minimum is unique, so the closest hit and its tie rule do not depend on the
+// processing order. A lane does not move to its next instance, finish or take a new ray while
+// pairs of its ray are queued.
+constexpr uint32_t kCompactQueue = 128;    // per wave: < 64 left after a round + <= 64 appended per leaf round
+constexpr uint32_t kLeafQueue = 128;       // per wave: < 64 left after a round + <= 64 appended per step
+// Low word of a lane's key: no hit yet; a hit of an earlier instance (equal t of a later one
+// loses); else 1 + the primitive id of a hit of the current instance.
 constexpr uint32_t kNoHitLow = 0xFFFFFFFFu;
+constexpr uint32_t kEarlierLow = 0u;
 constexpr uint32_t kCompactIterationCap = 1u << 24;
+constexpr uint32_t kWalkerOne = 1u << 16;  // s_cnt: queued pairs in the low half, helper lanes in the high half
+
+// float <-> unsigned with the float order (t may be negative for rays with a negative tmin)
+__device__ __forceinline__ uint32_t t_ord(float f) {
+    const uint32_t b = __float_as_uint(f);
+    return b ^ ((b & 0x80000000u) ? 0xFFFFFFFFu : 0x80000000u);
+}
+__device__ __forceinline__ float ord_t(uint32_t u) {
+    return __uint_as_float(u ^ ((u & 0x80000000u) ? 0x80000000u : 0xFFFFFFFFu));
+}
+__device__ __forceinline__ unsigned long long lane_key(float t, uint32_t low) {
+    return (static_cast<unsigned long long>(t_ord(t)) << 32) | low;
+}
 
 template <int STACK>
 struct CWalker {
     f3 o, d, inv;
     uint32_t oct;
     uint2 cur;  // current group: x = child_base, y = imask | remaining hit bits (octant order) << 8
-    uint32_t node, pbase, pmask;
+    uint32_t node, pbase, pmask;  // pmask: leaf records of the last node not yet queued
     int sp, sb;  // the stack is a deque: push / pop at sp, other lanes take entries at sb
     bool have_node;
 
@@ -1084,36 +1027,29 @@ struct CWalker {
         have_node = false;
     }
 
-    // One step: one pending leaf record through the early-out, or one node test; then, when
-    // no record of the node is pending, the next node is selected. `cand` receives the leaf
-    // slot that passed the early-out (0xFFFFFFFF if none); it is valid with any return value.
-    __device__ __forceinline__ int step(const BlasDev& B, float tmin, float tcur, uint2* lds, uint32_t& cand) {
-        cand = 0xFFFFFFFFu;
-        if (pmask) {
-            const uint32_t slot = pbase + uint32_t(__ffs(pmask) - 1);
-            pmask &= pmask - 1;
-            const auto* pr = gmem(B.prims + size_t(slot) * 4);
-            const float4 a = pr[0], b = pr[3];
-            if (ray_cylinder(o, d, f3{a.x, a.y, a.z}, f3{b.x, b.y, b.z}, gmem(B.aux)[slot])) cand = slot;
-        } else if (have_node) {
-            if (node >= B.nnodes) return kStepError;  // malformed structure: report, never read out of bounds
-            uint32_t hits, pm, child_base, imask, pb;
-            node_visit(B.nodes, node, o, inv, oct, tmin, tcur, hits, pm, child_base, imask, pb);
-            if (pm && pb + (32u - __clz(pm)) > B.nprims) return kStepError;
-            pbase = pb;
-            pmask = pm;
-            have_node = false;
-            if (hits) {
-                const uint2 g = make_uint2(child_base, imask | (hits << 8));
-                if (cur.y >> 8) {
-                    if (sp >= STACK) return kStepError;
-                    lds[sp * kTraceBlock] = cur;
-                    ++sp;
-                }
-                cur = g;
+    // Tests the selected node: its leaf records hit go to pmask, its internal children hit become
+    // the current group (the former one is pushed).
+    __device__ __forceinline__ int visit(const BlasDev& B, float tmin, float tcur, uint2* lds) {
+        if (node >= B.nnodes) return kStepError;  // malformed structure: report, never read out of bounds
+        uint32_t hits, pm, child_base, imask, pb;
+        node_visit(B.nodes, node, o, inv, oct, tmin, tcur, hits, pm, child_base, imask, pb);
+        if (pm && pb + (32u - __clz(pm)) > B.nprims) return kStepError;
+        pbase = pb;
+        pmask = pm;
+        have_node = false;
+        if (hits) {
+            if (cur.y >> 8) {
+                if (sp >= STACK) return kStepError;
+                lds[sp * kTraceBlock] = cur;
+                ++sp;
             }
+            cur = make_uint2(child_base, imask | (hits << 8));
         }
-        if (pmask || have_node) return kStepMore;
+        return kStepMore;
+    }
+
+    // Selects the next node of the walk (kStepDone when none is left).
+    __device__ __forceinline__ int next(uint2* lds) {
         if ((cur.y >> 8) == 0) {
             if (sp == sb) return kStepDone;
             --sp;
@@ -1130,6 +1066,59 @@ struct CWalker {
         return kStepMore;
     }
 };
+
+// One leaf record of a mode other than phantom against a ray: the hit within [tmin, tmax] with
+// its primitive id and payload (LSS: u and the normal; DOTS, triangles: two barycentrics, the
+// record's slot and the triangle of a DOTS piece). A piece's nearest triangle wins, the lower
+// one on equal t.
+__device__ __forceinline__ bool leaf_intersect(int mode, const BlasDev& B, uint32_t slot, f3 o, f3 d, float tmin,
+                                               float tmax, float& t, uint32_t& pid, float4& pay) {
+    bool hit = false;
+    if (mode == kLss) {
+        const auto* pr = gmem(B.prims + size_t(slot) * 2);
+        const float4 a = pr[0], b = pr[1];
+        LssHit lh;
+        if (lss_intersect(o, d, f3{a.x, a.y, a.z}, fabsf(a.w), f3{b.x, b.y, b.z}, b.w, !signbit(a.w), tmin, tmax, lh)) {
+            hit = true;
+            t = lh.t;
+            pid = gmem(B.prim_ids)[slot];
+            pay = make_float4(lh.u, lh.n.x, lh.n.y, lh.n.z);
+        }
+    } else if (mode == kTriangles) {
+        const auto* pr = gmem(B.prims + size_t(slot) * 3);
+        const float4 a = pr[0], b = pr[1], c = pr[2];
+        float b1, b2;
+        if (tri_intersect(make_tri_ray(d), o, f3{a.x, a.y, a.z}, f3{b.x, b.y, b.z}, f3{c.x, c.y, c.z}, tmin, tmax, t, b1,
+                          b2)) {
+            hit = true;
+            pid = gmem(B.prim_ids)[slot];
+            pay = make_float4(b1, b2, __uint_as_float(slot), 0.0f);
+        }
+    } else {
+        const auto* pr = gmem(B.prims + size_t(slot) * 4);
+        const float4 P[4] = {pr[0], pr[1], pr[2], pr[3]};
+        const TriRay TR = make_tri_ray(d);
+        float bt = tmax;
+        uint32_t btri = 0;
+#pragma unroll
+        for (int tri = 0; tri < 4; ++tri) {
+            f3 v0, v1, v2;
+            dots_tri(P, tri >> 1, tri & 1, v0, v1, v2);
+            float tt, b1, b2;
+            if (tri_intersect(TR, o, v0, v1, v2, tmin, bt, tt, b1, b2) && (!hit || tt < bt)) {
+                hit = true;
+                bt = tt;
+                btri = uint32_t(tri);
+                pay = make_float4(b1, b2, __uint_as_float(slot), __uint_as_float(btri));
+            }
+        }
+        if (hit) {
+            t = bt;
+            pid = gmem(B.prim_ids)[slot] * 4u + btri;
+        }
+    }
+    return hit;
+}
 
 template <class G, bool ANY, int STACK, int IM, class Src, class Snk>
 __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkClaim& work, uint2* lds, Src&& src,
@@ -1154,29 +1143,37 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
         else
             return tp.inst[i].blas;
     };
-    static_assert(G::kMode == kPhantom, "compacted lanes serve the phantom intersector");
-    __shared__ uint32_t s_queue[(kTraceBlock / 64) * kCompactQueue];
-    __shared__ unsigned long long s_key[kTraceBlock];  // best (t, instance, primitive) of the lane's ray
-    __shared__ float4 s_pay[kTraceBlock];              // its u and ray-centric normal vector
-    __shared__ uint32_t s_pol[kTraceBlock];            // its polished flag
-    __shared__ uint32_t s_cnt[kTraceBlock];            // pairs of the lane's ray still queued
-    __shared__ uint32_t s_walk[kTraceBlock];           // other lanes walking subtrees of the lane's ray
-    __shared__ uint32_t s_xfer[kTraceBlock];           // donor lane by rank (subtree hand-over)
+    static_assert(!G::kMixed || G::kCompact, "compacted lanes serve BVH instances");
+    constexpr bool kHasPhantom = G::kMixed || G::kMode == kPhantom;
+    constexpr uint32_t kWaves = kTraceBlock / 64;
+    __shared__ uint32_t s_leaf[kWaves * kLeafQueue];     // leaf queue: slots
+    __shared__ uint8_t s_leaf_lane[kWaves * kLeafQueue]; // ... and the lane whose ray they belong to
+    __shared__ uint32_t s_queue[kHasPhantom ? kWaves * kCompactQueue : 1];  // phantom pairs past the early-out
+    __shared__ unsigned long long s_key[kTraceBlock];  // best (t, primitive) of the lane's ray
+    __shared__ float4 s_pay[kTraceBlock];              // its u and normal / barycentrics and record
+    __shared__ uint32_t s_cnt[kTraceBlock];            // pairs of the lane's ray still queued (low half),
+                                                       // other lanes walking its subtrees (high half)
+    __shared__ uint8_t s_xfer[kTraceBlock];            // donor lane by rank (subtree hand-over)
     // kTrav: walking its own ray; kHelp: walking a subtree of the ray of lane `home`; kWait: own
     // walk done, waiting for queued pairs and helpers of its ray
     enum { kIdle = 0, kInst = 1, kTrav = 2, kWait = 3, kHelp = 4 };
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wbase = threadIdx.x & ~63u;
     const uint64_t lt = (1ull << lane) - 1ull;
-    uint32_t* queue = s_queue + (threadIdx.x >> 6) * kCompactQueue;
+    uint32_t* leaf = s_leaf + (threadIdx.x >> 6) * kLeafQueue;
+    uint8_t* leaf_lane = s_leaf_lane + (threadIdx.x >> 6) * kLeafQueue;
+    uint32_t* queue = s_queue + (kHasPhantom ? (threadIdx.x >> 6) * kCompactQueue : 0u);
     CWalker<STACK> W;
     W.o = W.d = f3{0.0f, 0.0f, 0.0f};
+    W.pmask = 0;
+    W.have_node = false;
     f3 ow = f3{0, 0, 0}, dw = f3{0, 0, 0};
     float tmin = 0.0f, tmax = 0.0f, tcur = 0.0f;
     uint32_t idx = 0, inst = 0, home = lane;
+    uint32_t binst = 0, bpid = 0;  // best hit of the instances before the current one
     int state = kIdle;
     bool ray_done = false;
-    uint32_t qn = 0;         // wave-uniform queue length
+    uint32_t ln = 0, qn = 0;  // wave-uniform lengths of the leaf queue and the Prhi queue
 #ifdef VKHRT_WORK_COUNTERS
     unsigned long long wc[14] = {};  // WorkCounter sums of this wave (wave-uniform)
     unsigned long long t_it = clock64(), t_mid = t_it;
@@ -1195,6 +1192,19 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
 #define VK_WC_MARK() ((void)0)
 #define VK_WC_END(kind) ((void)0)
 #endif
+    // After a round: the lanes' limits, and the end of any-hit rays that found one.
+    auto merged = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (state != kIdle) {
+            const unsigned long long kk = s_key[wbase + home];
+            tcur = ord_t(uint32_t(kk >> 32));
+            if (ANY && state != kHelp && uint32_t(kk) != kNoHitLow && !ray_done) {
+                ray_done = true;
+                state = kWait;
+            }
+        }
+    };
     // Every wave leaves the loop: a normal frame takes ~10^4 iterations per wave; past the cap
     // the wave reports an error (status[0]) and stops, leaving its rays unwritten.
     for (uint32_t guard = 0;; ++guard) {
@@ -1204,14 +1214,18 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
             break;
         }
         // (a) a waiting lane whose pairs are all merged moves to its next instance or finishes
-        if (state == kWait && s_cnt[threadIdx.x] == 0u && s_walk[threadIdx.x] == 0u) {
-            if (ray_done) {
-                state = kInst;
-                inst = tp.ninst;  // finish below
-            } else {
-                ++inst;
-                state = kInst;
+        if (state == kWait && s_cnt[threadIdx.x] == 0u) {
+            if constexpr (IM != kInstOne) {
+                const unsigned long long kk = s_key[threadIdx.x];
+                const uint32_t lo = uint32_t(kk);
+                if (lo != kNoHitLow && lo != kEarlierLow) {
+                    binst = inst;
+                    bpid = lo - 1u;
+                    s_key[threadIdx.x] = kk & ~0xFFFFFFFFull;  // low word kEarlierLow
+                }
             }
+            inst = ray_done ? tp.ninst : inst + 1u;
+            state = kInst;
         }
         // (b) refill idle lanes from the work counters
         if (!work.exhausted) {
@@ -1222,11 +1236,8 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
                     if (r < work.total) {
                         src(r, idx, ow, dw, tmin, tmax);
                         tcur = tmax;
-                        s_key[threadIdx.x] =
-                            (static_cast<unsigned long long>(__float_as_uint(tmax)) << 32) | kNoHitLow;
-                        s_pol[threadIdx.x] = 0u;
+                        s_key[threadIdx.x] = lane_key(tmax, kNoHitLow);
                         s_cnt[threadIdx.x] = 0u;
-                        s_walk[threadIdx.x] = 0u;
                         home = lane;
                         inst = 0;
                         ray_done = false;
@@ -1250,29 +1261,26 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
                 const uint32_t lo = uint32_t(kk);
                 Best best;
                 best.slot = 0xFFFFFFFFu;
+                best.extra = 0u;
                 if (lo == kNoHitLow) {
                     best.t = tmax;
                     best.inst = best.pid = 0xFFFFFFFFu;
                     best.u = best.a = best.b = best.c = 0.0f;
-                    best.extra = 0u;
                 } else {
                     const float4 pay = s_pay[threadIdx.x];
-                    best.t = __uint_as_float(uint32_t(kk >> 32));
-                    if constexpr (IM == kInstOne) {
-                        best.inst = 0;
-                    } else if constexpr (IM == kInstFew) {
-                        uint32_t k = 0;
-                        for (uint32_t j = 1; j < tp.ninst; ++j) k = few[j].gbase <= lo ? j : k;
-                        best.inst = k;
-                    } else {
-                        best.inst = gid_instance(tp.inst, tp.ninst, lo);
-                    }
-                    best.pid = lo - blas(best.inst).gbase;
+                    best.t = ord_t(uint32_t(kk >> 32));
+                    best.inst = IM == kInstOne ? 0u : binst;
+                    best.pid = IM == kInstOne ? lo - 1u : bpid;
                     best.u = pay.x;
                     best.a = pay.y;
                     best.b = pay.z;
                     best.c = pay.w;
-                    best.extra = s_pol[threadIdx.x];
+                    if constexpr (G::kMixed || G::kMode == kDots || G::kMode == kTriangles) {
+                        best.slot = __float_as_uint(pay.z);  // read for DOTS and triangle hits only
+                        best.extra = __float_as_uint(pay.w);
+                        if constexpr (G::kMixed)
+                            if (const uint32_t mode = blas(best.inst).mode; mode != kDots) best.extra = 0u;
+                    }
                 }
                 snk(idx, ow, dw, best);
                 state = kIdle;
@@ -1303,7 +1311,7 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
             if (dm && im) {
                 const uint32_t n = min(uint32_t(__popcll(dm)), uint32_t(__popcll(im)));
                 const uint32_t kd = __popcll(dm & lt), ki = __popcll(im & lt);
-                if (give && kd < n) s_xfer[wbase + kd] = lane;
+                if (give && kd < n) s_xfer[wbase + kd] = uint8_t(lane);
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 __builtin_amdgcn_wave_barrier();
                 const bool take = state == kIdle && ki < n;
@@ -1320,8 +1328,8 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
                     home = ghome;
                     inst = ginst;
                     tmin = gtmin;
-                    tcur = __uint_as_float(uint32_t(s_key[wbase + home] >> 32));
-                    atomicAdd(&s_walk[wbase + home], 1u);
+                    tcur = ord_t(uint32_t(s_key[wbase + home] >> 32));
+                    atomicAdd(&s_cnt[wbase + home], kWalkerOne);
                     state = kHelp;
                 }
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -1336,111 +1344,174 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
             if (work.exhausted) break;
             continue;
         }
-        // (d) intersection round on up to 64 queued pairs, one per lane
         VK_WC_MARK();
-        if (qn >= 64u || (qn != 0u && !__ballot(state == kTrav || state == kHelp))) {
-            const uint32_t m = qn < 64u ? qn : 64u;
-            VK_WC(kWcRounds, 1);
-            VK_WC(kWcRoundLanes, m);
-            const uint32_t e = lane < m ? queue[qn - m + lane] : 0u;
-            const int owner = int(e >> kCompactSlotBits);
-            const uint32_t slot = e & ((1u << kCompactSlotBits) - 1u);
+        const bool stuck = !__ballot(state == kTrav || state == kHelp);
+        // (d) Prhi round on up to 64 pairs past the early-out, one per lane (also when nothing
+        // else is left to do)
+        if constexpr (kHasPhantom) {
+            if (qn >= 64u || (stuck && ln == 0u && qn != 0u)) {
+                const uint32_t m = qn < 64u ? qn : 64u;
+                VK_WC(kWcRounds, 1);
+                VK_WC(kWcRoundLanes, m);
+                const uint32_t e = lane < m ? queue[qn - m + lane] : 0u;
+                const int owner = int(e >> kCompactSlotBits);
+                const uint32_t slot = e & ((1u << kCompactSlotBits) - 1u);
+                const f3 po = f3{__shfl(W.o.x, owner), __shfl(W.o.y, owner), __shfl(W.o.z, owner)};
+                const f3 pd = f3{__shfl(W.d.x, owner), __shfl(W.d.y, owner), __shfl(W.d.z, owner)};
+                const float ptmin = __shfl(tmin, owner), ptmax = __shfl(tmax, owner);
+                const uint32_t pinst = __shfl(inst, owner), pidx = __shfl(idx, owner);
+                const uint32_t os = wbase + uint32_t(owner);
+                unsigned long long k = ~0ull;
+                PhantomHit ph;
+                bool hit = false;
+                if (lane < m) {
+                    const bool skip = ANY && uint32_t(s_key[os]) != kNoHitLow;  // already occluded
+                    if (!skip) {
+                        const BlasDev& B = blas(pinst);
+                        RayFrame F;
+                        make_frame(po, pd, F);
+                        const auto* pr = gmem(B.prims + size_t(slot) * 4);
+                        float4 cv[4] = {pr[0], pr[1], pr[2], pr[3]};
+                        if constexpr (G::kMixed)
+                            hit = prhi<kRadiusRuntime, kPolishRuntime, false>(F, cv, 0.0f, B.radius, ph, B.radius_mode,
+                                                                              tp.defer != nullptr);
+                        else
+                            hit = prhi<G::kRMode, G::kPolish ? kPolishDefer : kPolishOff, false>(F, cv, 0.0f, B.radius, ph);
+                        if ((G::kMixed || G::kPolish) && ph.deferred) {
+                            // this curve needs the FP64 continuation: queue (ray, instance, slot)
+                            const uint32_t q = atomicAdd(tp.defer_count, 1u);
+                            if (q < tp.defer_cap)
+                                tp.defer[q] = make_uint4(pidx, pinst, slot, 0u);
+                            else
+                                atomicAdd(&tp.status[1], 1u);
+                        }
+                        hit = hit && ph.t >= ptmin && ph.t <= ptmax;
+                        if (hit) {
+                            k = lane_key(ph.t, gmem(B.prim_ids)[slot] + 1u);
+                            atomicMin(&s_key[os], k);
+                        }
+                    }
+                    atomicSub(&s_cnt[os], 1u);
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                // the unique winner for this owner writes the payload
+                if (hit && s_key[os] == k) s_pay[os] = make_float4(ph.u, ph.ncx, ph.ncy, ph.nsz);
+                qn -= m;
+                merged();
+                VK_WC_END(kWcCyclesRounds);
+                continue;
+            }
+        }
+        // (e) leaf round on up to 64 records, one per lane
+        if (ln >= 64u || (stuck && ln != 0u)) {
+            const uint32_t m = ln < 64u ? ln : 64u;
+            VK_WC(kWcLeafTests, m);
+            const uint32_t slot = lane < m ? leaf[ln - m + lane] : 0u;
+            const int owner = lane < m ? int(leaf_lane[ln - m + lane]) : 0;
             const f3 po = f3{__shfl(W.o.x, owner), __shfl(W.o.y, owner), __shfl(W.o.z, owner)};
             const f3 pd = f3{__shfl(W.d.x, owner), __shfl(W.d.y, owner), __shfl(W.d.z, owner)};
-            const float ptmin = __shfl(tmin, owner), ptmax = __shfl(tmax, owner);
-            const uint32_t pinst = __shfl(inst, owner), pidx = __shfl(idx, owner);
+            const uint32_t pinst = __shfl(inst, owner);
             const uint32_t os = wbase + uint32_t(owner);
+            bool cand = false, hit = false;
             unsigned long long k = ~0ull;
-            PhantomHit ph;
-            bool hit = false;
+            float4 pay = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            float ptmin = 0.0f;
+            if constexpr (G::kMixed || G::kMode != kPhantom) ptmin = __shfl(tmin, owner);
             if (lane < m) {
-                const bool skip = ANY && uint32_t(s_key[os]) != kNoHitLow;  // already occluded
+                const unsigned long long kk = s_key[os];
+                const bool skip = ANY && uint32_t(kk) != kNoHitLow;  // already occluded
                 if (!skip) {
                     const BlasDev& B = blas(pinst);
-                    RayFrame F;
-                    make_frame(po, pd, F);
-                    const auto* pr = gmem(B.prims + size_t(slot) * 4);
-                    float4 cv[4] = {pr[0], pr[1], pr[2], pr[3]};
-                    hit = prhi<G::kRMode, G::kPolish ? kPolishDefer : kPolishOff, false>(F, cv, 0.0f, B.radius, ph);
-                    if (G::kPolish && ph.deferred) {
-                        // this curve needs the FP64 continuation: queue (ray, instance, slot)
-                        const uint32_t q = atomicAdd(tp.defer_count, 1u);
-                        if (q < tp.defer_cap)
-                            tp.defer[q] = make_uint4(pidx, pinst, slot, 0u);
-                        else
-                            atomicAdd(&tp.status[1], 1u);
-                    }
-                    hit = hit && ph.t >= ptmin && ph.t <= ptmax;
-                    if (hit) {
-                        k = pack_key(ph.t, B.gbase + B.prim_ids[slot]);
-                        atomicMin(&s_key[os], k);
+                    const int mode = G::kMixed ? int(B.mode) : G::kMode;
+                    if (kHasPhantom && mode == kPhantom) {
+                        const auto* pr = gmem(B.prims + size_t(slot) * 4);
+                        const float4 a = pr[0], b = pr[3];
+                        cand = ray_cylinder(po, pd, f3{a.x, a.y, a.z}, f3{b.x, b.y, b.z}, gmem(B.aux)[slot]);
+                    } else if (G::kMixed || G::kMode != kPhantom) {
+                        float t = 0.0f;
+                        uint32_t pid = 0;
+                        hit = leaf_intersect(mode, B, slot, po, pd, ptmin, ord_t(uint32_t(kk >> 32)), t, pid, pay);
+                        if (hit) {
+                            k = lane_key(t, pid + 1u);
+                            atomicMin(&s_key[os], k);
+                        }
                     }
                 }
-                atomicSub(&s_cnt[os], 1u);
+                if (!cand) atomicSub(&s_cnt[os], 1u);  // a survivor stays counted in the Prhi queue
             }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            if (hit && s_key[os] == k) {  // the unique winner for this owner writes the payload
-                s_pay[os] = make_float4(ph.u, ph.ncx, ph.ncy, ph.nsz);
-                s_pol[os] = ph.polished ? 1u : 0u;
+            if constexpr (kHasPhantom) {
+                const uint64_t cm = __ballot(cand);
+                if (cand) queue[qn + __popcll(cm & lt)] = (uint32_t(owner) << kCompactSlotBits) | slot;
+                qn += __popcll(cm);
+                VK_WC(kWcPairs, __popcll(cm));
             }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            qn -= m;
-            if (state != kIdle) {
-                const unsigned long long kk = s_key[wbase + home];
-                tcur = __uint_as_float(uint32_t(kk >> 32));
-                if (ANY && state != kHelp && uint32_t(kk) != kNoHitLow && !ray_done) {
-                    ray_done = true;
-                    state = kWait;
-                }
+            ln -= m;
+            if constexpr (G::kMixed || G::kMode != kPhantom) {
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                if (hit && s_key[os] == k) s_pay[os] = pay;
+                merged();
+            } else {
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
             }
-            VK_WC_END(kWcCyclesRounds);
+            VK_WC_END(kWcCyclesSteps);
             continue;
         }
-        // (e) traversal steps, one per traversing lane each; survivors of the early-out are queued.
+        // (f) traversal steps, one node test per walking lane each; the leaf records hit are queued.
         // tp.steps_per_iter > 1 runs up to that many steps before the bookkeeping above comes
-        // round again, while the queue can take a full step of pairs and some lane still walks.
-        // (Stopping early once refill_min lanes have stopped walking measured no better.)
+        // round again, while the leaf queue can take a full step and some lane still walks.
         const uint32_t nsteps = tp.steps_per_iter > 1u ? tp.steps_per_iter : 1u;
         for (uint32_t si = 0; si < nsteps; ++si) {
-            if (si > 0u && (qn >= 64u || !__ballot(state == kTrav || state == kHelp))) break;
+            if (si > 0u && (ln >= 64u || !__ballot(state == kTrav || state == kHelp))) break;
 #ifdef VKHRT_WORK_COUNTERS
             {
                 const bool wk = state == kTrav || state == kHelp;
-                VK_WC(kWcNodeTests, __popcll(__ballot(wk && W.pmask == 0u && W.have_node)));
-                VK_WC(kWcLeafTests, __popcll(__ballot(wk && W.pmask != 0u)));
+                VK_WC(kWcNodeTests, __popcll(__ballot(wk && W.have_node)));
                 VK_WC(kWcStepLanes, __popcll(__ballot(wk)));
             }
 #endif
-            uint32_t cand = 0xFFFFFFFFu;
             if (state == kHelp && ANY && uint32_t(s_key[wbase + home]) != kNoHitLow) {
-                atomicSub(&s_walk[wbase + home], 1u);  // the ray is occluded already
+                atomicSub(&s_cnt[wbase + home], kWalkerOne);  // the ray is occluded already
+                W.pmask = 0;
                 state = kIdle;
-            } else if (state == kTrav || state == kHelp) {
-                const int r = W.step(blas(inst), tmin, tcur, lds, cand);
-                if (r == kStepError) atomicAdd(&tp.status[0], 1u);
+            }
+            bool walk = state == kTrav || state == kHelp;
+            int r = kStepMore;
+            if (walk && W.have_node) r = W.visit(blas(inst), tmin, tcur, lds);
+            // one record per lane and pass joins the leaf queue while a full pass fits; a lane whose
+            // records did not all fit keeps them pending and walks on when they are queued
+            uint32_t added = 0;
+            for (;;) {
+                const bool app = walk && r == kStepMore && W.pmask != 0u;
+                const uint64_t am = __ballot(app);
+                if (am == 0 || ln + uint32_t(__popcll(am)) > kLeafQueue) break;
+                if (app) {
+                    const uint32_t at = ln + __popcll(am & lt);
+                    leaf[at] = W.pbase + uint32_t(__ffs(W.pmask) - 1);
+                    leaf_lane[at] = uint8_t(home);
+                    W.pmask &= W.pmask - 1u;
+                    ++added;
+                }
+                ln += __popcll(am);
+            }
+            if (added) atomicAdd(&s_cnt[wbase + home], added);
+            if (walk && r == kStepMore && W.pmask == 0u) r = W.next(lds);
+            if (walk && r != kStepMore) {
+                if (r == kStepError) {
+                    atomicAdd(&tp.status[0], 1u);
+                    W.pmask = 0;
+                }
                 if (state == kHelp) {
-                    if (r == kStepError || r == kStepDone) {
-                        atomicSub(&s_walk[wbase + home], 1u);
-                        state = kIdle;
-                    }
-                } else if (r == kStepError) {
-                    ray_done = true;
-                    state = kWait;
-                } else if (r == kStepDone) {
+                    atomicSub(&s_cnt[wbase + home], kWalkerOne);
+                    state = kIdle;
+                } else {
+                    if (r == kStepError) ray_done = true;
                     state = kWait;
                 }
             }
-            const bool app = cand != 0xFFFFFFFFu;
-            const uint64_t am = __ballot(app);
-            if (app) {
-                queue[qn + __popcll(am & lt)] = (home << kCompactSlotBits) | cand;
-                atomicAdd(&s_cnt[wbase + home], 1u);
-            }
-            qn += __popcll(am);
             VK_WC(kWcSteps, 1);
-            VK_WC(kWcPairs, __popcll(am));
             VK_WC_END(kWcCyclesSteps);
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
@@ -1458,8 +1529,12 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
 #undef VK_WC_END
 }
 
-// Persistent loop for one geometry variant: compacted intersection rounds for phantom curves
-// (the expensive, iterative test), the per-lane loop for LSS and DOTS.
+// Waves per SIMD the persistent kernels are held to: the LDS of four 256-thread blocks (36.6-38.7 KB
+// each) fits a CU with stacks of up to 12 entries, so the registers have to stay at 128 there (left
+// alone some variants take 131-150 and run three waves).
+constexpr int lanes_waves(int stack) { return stack <= 12 ? 4 : 1; }
+
+// Persistent loop for one geometry variant.
 template <class G, bool ANY, int STACK, int IM = kInstMany, class Src, class Snk>
 __device__ __forceinline__ void persistent_lanes(const TraceParams& tp, uint32_t total, uint32_t* counter, uint2* lds,
                                                  Src&& src, Snk&& snk, uint32_t* xcd = nullptr) {
@@ -1472,14 +1547,11 @@ __device__ __forceinline__ void persistent_lanes(const TraceParams& tp, uint32_t
         __syncthreads();
     }
     WorkClaim work(counter, xcd, chunk, total, &s_dry);
-    if constexpr (G::kMode == kPhantom)
-        persistent_compact<G, ANY, STACK, IM>(tp, work, lds, src, snk);
-    else
-        persistent_generic<G, ANY, STACK, IM>(tp, work, lds, src, snk);
+    persistent_compact<G, ANY, STACK, IM>(tp, work, lds, src, snk);
 }
 
 template <class G, bool ANY, int STACK, int IM>
-__global__ __launch_bounds__(kTraceBlock) void k_trace_rays_persistent(TraceParams tp, const float* __restrict__ rays,
+__global__ __launch_bounds__(kTraceBlock, lanes_waves(STACK)) void k_trace_rays_persistent(TraceParams tp, const float* __restrict__ rays,
                                                                        uint32_t n, HitRec* __restrict__ hits,
                                                                        uint32_t* __restrict__ counter) {
     __shared__ uint2 stk[STACK * kTraceBlock];
@@ -1498,7 +1570,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_trace_rays_persistent(TracePara
             HitRec h;
             finish_hit(tp, o, d, best, h);
             hits[i] = h;
-            if (G::kPolish) tp.keys[i] = best_key(tp, best);
+            if (G::kPolish || (G::kMixed && tp.keys)) tp.keys[i] = best_key(tp, best);
         },
         tp.xcd_work);
 }
@@ -1836,7 +1908,7 @@ __global__ __launch_bounds__(kAppendBlock) void k_render_live(RenderParams rp) {
 }
 
 template <class G, int STACK, int IM>
-__global__ __launch_bounds__(kTraceBlock) void k_render_primary_defer(RenderParams rp) {
+__global__ __launch_bounds__(kTraceBlock, lanes_waves(STACK)) void k_render_primary_defer(RenderParams rp) {
     __shared__ uint2 stk[STACK * kTraceBlock];
     persistent_lanes<G, false, STACK, IM>(
         rp.tp, rp.counters[6], rp.counters + 1, stk + threadIdx.x,
@@ -1851,7 +1923,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_render_primary_defer(RenderPara
             HitRec h;
             finish_hit(rp.tp, o, d, best, h);
             rp.hitrec[pix] = h;
-            if (G::kPolish) rp.tp.keys[pix] = best_key(rp.tp, best);
+            if (G::kPolish || (G::kMixed && rp.tp.keys)) rp.tp.keys[pix] = best_key(rp.tp, best);
         },
         rp.counters + kXcdCounters);
 }
@@ -1939,7 +2011,7 @@ __global__ __launch_bounds__(kAppendBlock) void k_render_classify(RenderParams r
 
 // Pass 3: shadow rays (FP32, any hit) -> per-pixel visibility.
 template <class G, int STACK, int IM>
-__global__ __launch_bounds__(kTraceBlock) void k_render_shadow_defer(RenderParams rp, const uint32_t* queue,
+__global__ __launch_bounds__(kTraceBlock, lanes_waves(STACK)) void k_render_shadow_defer(RenderParams rp, const uint32_t* queue,
                                                                      const uint32_t* count, uint32_t* work,
                                                                      uint32_t skip_upto) {
     __shared__ uint2 stk[STACK * kTraceBlock];
@@ -2361,8 +2433,8 @@ __global__ __launch_bounds__(64) void k_render_shadow_groups(RenderParams rp, co
 #endif
 }
 
-// The same two traversal passes for TLASes that mix geometry modes: one thread per queued
-// ray, trace_world's per-instance dispatch (with the FP64 polish candidates of phantom
+// The same two traversal passes for TLASes with voxel instances (and those whose merge keys do not
+// fit): one thread per queued ray, trace_world's per-instance dispatch (with the FP64 polish candidates of phantom
 // instances deferred like the persistent kernels'); the queue lengths are read on the device.
 template <class G, int STACK>
 __global__ __launch_bounds__(kTraceBlock) void k_render_primary_flat(RenderParams rp) {
@@ -2486,24 +2558,26 @@ hipError_t launch_trace_pass(const TraceParams& tp, const float* rays, uint32_t 
                              bool any, hipStream_t st) {
     using namespace trace_detail;
     uint2* stats = nullptr;
-    if constexpr (!G::kMixed) {
+    if constexpr (G::kCompact) {
         if (tp.work) {
             hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, st, tp.work, 1u);
             if (tp.xcd_chunk && tp.xcd_work)
                 hipLaunchKernelGGL(k_zero, dim3(8 * kXcdStride / 64), dim3(64), 0, st, tp.xcd_work, 8u * kXcdStride);
             // one-instance TLASes take kernels that read the BLAS fields once
-            const bool one = instance_mode(tp.ninst) == kInstOne;
+            // (a TLAS of several modes has several instances)
+            const bool one = !G::kMixed && instance_mode(tp.ninst) == kInstOne;
+            constexpr int kOne = G::kMixed ? kInstMany : kInstOne;
             if (any && one)
-                hipLaunchKernelGGL((k_trace_rays_persistent<G, true, STACK, kInstOne>),
-                                   persistent_grid(k_trace_rays_persistent<G, true, STACK, kInstOne>, tp.blocks_per_cu), block, 0,
+                hipLaunchKernelGGL((k_trace_rays_persistent<G, true, STACK, kOne>),
+                                   persistent_grid(k_trace_rays_persistent<G, true, STACK, kOne>, tp.blocks_per_cu), block, 0,
                                    st, tp, rays, n, hits, tp.work);
             else if (any)
                 hipLaunchKernelGGL((k_trace_rays_persistent<G, true, STACK, kInstMany>),
                                    persistent_grid(k_trace_rays_persistent<G, true, STACK, kInstMany>, tp.blocks_per_cu), block, 0,
                                    st, tp, rays, n, hits, tp.work);
             else if (one)
-                hipLaunchKernelGGL((k_trace_rays_persistent<G, false, STACK, kInstOne>),
-                                   persistent_grid(k_trace_rays_persistent<G, false, STACK, kInstOne>, tp.blocks_per_cu), block,
+                hipLaunchKernelGGL((k_trace_rays_persistent<G, false, STACK, kOne>),
+                                   persistent_grid(k_trace_rays_persistent<G, false, STACK, kOne>, tp.blocks_per_cu), block,
                                    0, st, tp, rays, n, hits, tp.work);
             else
                 hipLaunchKernelGGL((k_trace_rays_persistent<G, false, STACK, kInstMany>),
@@ -2512,11 +2586,15 @@ hipError_t launch_trace_pass(const TraceParams& tp, const float* rays, uint32_t 
             return hipGetLastError();
         }
     }
-    if (any)
-        hipLaunchKernelGGL((k_trace_rays<G, true, STACK, false>), grid, block, 0, st, tp, rays, n, hits, stats);
-    else
-        hipLaunchKernelGGL((k_trace_rays<G, false, STACK, false>), grid, block, 0, st, tp, rays, n, hits, stats);
-    return hipGetLastError();
+    if constexpr (G::kMixed && G::kCompact) {
+        return hipErrorNotSupported;  // the host picks GeoMixed where the persistent lanes are off
+    } else {
+        if (any)
+            hipLaunchKernelGGL((k_trace_rays<G, true, STACK, false>), grid, block, 0, st, tp, rays, n, hits, stats);
+        else
+            hipLaunchKernelGGL((k_trace_rays<G, false, STACK, false>), grid, block, 0, st, tp, rays, n, hits, stats);
+        return hipGetLastError();
+    }
 }
 
 // The neural fallback's lane-group walker: rp.group_lanes (8, 16, 32 or 64; 16 otherwise) lanes per ray.
@@ -2556,8 +2634,8 @@ hipError_t launch_render_variant(const RenderParams& rp, hipStream_t st, hipEven
             // Deferred pipeline: the traversal kernels only record hits (their sinks stay
             // small because a lane finishing any ray makes the whole wave run the sink);
             // shading, the shadow queue and the optional deferred FP64 polish run as passes.
-            // A TLAS of one geometry mode traverses with persistent lanes, a mixed TLAS with one
-            // thread per queued ray.
+            // BVH instances are traversed with persistent lanes, a TLAS with voxel instances with
+            // one thread per queued ray.
             const TraceParams& tp = rp.tp;
             const dim3 pgrid(1024);
             hipLaunchKernelGGL(k_render_live, dim3((rp.cam.work + kAppendBlock * kAppendItems - 1) / (kAppendBlock * kAppendItems)), dim3(kAppendBlock),
@@ -2567,11 +2645,12 @@ hipError_t launch_render_variant(const RenderParams& rp, hipStream_t st, hipEven
             // one-instance TLASes take kernels that read the BLAS fields once, TLASes of up to
             // kFewInstances instances kernels that stage them in LDS
             const int im = instance_mode(tp.ninst);
-            if constexpr (G::kMixed)
+            constexpr int kOne = G::kMixed ? kInstFew : kInstOne;
+            if constexpr (!G::kCompact)
                 hipLaunchKernelGGL((k_render_primary_flat<G, STACK>), grid, block, 0, st, rp);
             else if (im == kInstOne)
-                hipLaunchKernelGGL((k_render_primary_defer<G, STACK, kInstOne>),
-                                   persistent_grid(k_render_primary_defer<G, STACK, kInstOne>, tp.blocks_per_cu), block, 0,
+                hipLaunchKernelGGL((k_render_primary_defer<G, STACK, kOne>),
+                                   persistent_grid(k_render_primary_defer<G, STACK, kOne>, tp.blocks_per_cu), block, 0,
                                    st, rp);
             else if (im == kInstFew)
                 hipLaunchKernelGGL((k_render_primary_defer<G, STACK, kInstFew>),
@@ -2638,11 +2717,11 @@ hipError_t launch_render_variant(const RenderParams& rp, hipStream_t st, hipEven
                             if (e != hipSuccess) return e;
                         }
                     }
-                    if constexpr (G::kMixed)
+                    if constexpr (!G::kCompact)
                         hipLaunchKernelGGL((k_render_shadow_flat<G, STACK>), sgrid, block, 0, st, rp, squeue, scount);
                     else if (im == kInstOne)
-                        hipLaunchKernelGGL((k_render_shadow_defer<G, STACK, kInstOne>),
-                                           persistent_grid(k_render_shadow_defer<G, STACK, kInstOne>, tp.blocks_per_cu),
+                        hipLaunchKernelGGL((k_render_shadow_defer<G, STACK, kOne>),
+                                           persistent_grid(k_render_shadow_defer<G, STACK, kOne>, tp.blocks_per_cu),
                                            block, 0, st, rp, squeue, scount, rp.counters + 2, skip);
                     else if (im == kInstFew)
                         hipLaunchKernelGGL((k_render_shadow_defer<G, STACK, kInstFew>),
@@ -2667,7 +2746,9 @@ hipError_t launch_render_variant(const RenderParams& rp, hipStream_t st, hipEven
             return hipGetLastError();
         }
     }
-    // one thread per pixel (mixed-mode TLASes, or persistence switched off)
+    // one thread per pixel (persistence switched off)
+    if constexpr (G::kMixed && G::kCompact) return hipErrorNotSupported;  // the host picks GeoMixed here
+    else {
     if (ev) hipEventRecord(ev[0], st);
     hipLaunchKernelGGL((k_render_primary<G, STACK>), grid, block, 0, st, rp);
     if (ev) hipEventRecord(ev[1], st);
@@ -2680,6 +2761,7 @@ hipError_t launch_render_variant(const RenderParams& rp, hipStream_t st, hipEven
     }
     if (ev) hipEventRecord(ev[3], st);
     return hipGetLastError();
+    }
 }
 
 }  // namespace vk
