@@ -7,10 +7,11 @@
 //   2. 63-bit Morton codes of box centroids
 //   3. stable LSD radix sort of (key, index), 8 bits per pass: LDS histogram, one-block
 //      scan, LDS-ranked stable scatter (wave ballots rank equal digits)
-//   4. Karras (HPG 2012) binary radix tree, one thread per internal node
-//   5. bottom-up box refit in level-synchronous rounds (one launch per tree level)
+//   4. boxes of the aligned power-of-two runs of the sorted order
+//   5. Karras (HPG 2012) binary radix tree, one thread per internal node, each node's box
+//      combined from those runs
 //   6. top-down collapse to 8-wide nodes, one level per launch, by one of two rules:
-//      SAH: the refit rounds also compute, for every binary node, the least SAH cost
+//      SAH: level-synchronous rounds compute, for every binary node, the least SAH cost
 //      of covering its subtree with at most j child slots (j = 1..width), and each wide node is
 //      opened along those choices (Ylitie, Karras, Laine, HPG 2017);
 //      greedy (default, fewer node visits per ray on hair): each binary subtree is opened by
@@ -20,6 +21,8 @@
 //      power-of-two scales (outward rounding)
 //   7. gather primitive records into leaf order
 #include <hip/hip_runtime.h>
+
+#include <stddef.h>
 
 #include <algorithm>
 #include <string>
@@ -319,7 +322,92 @@ __global__ void k_rs_scatter(const uint64_t* __restrict__ kin, const uint32_t* _
     }
 }
 
+// ------------------------------------------------------------------ boxes of sorted ranges
+struct Box {
+    float lo[3], hi[3];
+};
+__device__ __forceinline__ void grow(Box& a, const Box& b) {
+    for (int k = 0; k < 3; ++k) {
+        a.lo[k] = fminf(a.lo[k], b.lo[k]);
+        a.hi[k] = fmaxf(a.hi[k], b.hi[k]);
+    }
+}
+
+// Boxes of the aligned power-of-two runs of the sorted primitives: entry l of level k is the box of
+// the sorted primitives [l << k, (l + 1) << k); runs that reach past the end are left out. Every
+// binary node covers a range of the sorted order, so its box follows from at most two entries per
+// level, without its children's boxes: no node waits for another and no launch per tree level is
+// needed. (min and max do not depend on the order, so the boxes are those of a bottom-up refit.)
+// 3.2M curves: 134 us here and 194 us for the tree with its boxes, where the tree and 32 refit
+// rounds took 102 + 455 us and a wait for every 8 rounds.
+constexpr int kBoxLevels = 32;
+struct BoxTree {
+    Box* box;
+    size_t off[kBoxLevels];  // first entry of each level
+};
+constexpr int kBoxPass = 7;  // levels made per launch: a wave's 64 lanes hold 2 entries each
+
+__device__ __forceinline__ Box range_box(const BoxTree& T, uint32_t first, uint32_t last) {
+    Box r;
+    for (int k = 0; k < 3; ++k) {
+        r.lo[k] = INFINITY;
+        r.hi[k] = -INFINITY;
+    }
+    uint32_t l = first, e = last + 1;
+    for (int k = 0; l < e; ++k) {
+        const Box* b = T.box + T.off[k];
+        if (l & 1u) grow(r, b[l++]);
+        if (e & 1u) grow(r, b[--e]);
+        l >>= 1;
+        e >>= 1;
+    }
+    return r;
+}
+
+// Levels level + 1 .. level + 7 from level `level`; the first launch (level 0) also gathers level 0,
+// the primitive boxes in sorted order.
+__global__ __launch_bounds__(kBlock) void k_box_levels(BoxTree T, uint32_t n, int level, const uint32_t* __restrict__ vals,
+                                                       const float4* __restrict__ blo, const float4* __restrict__ bhi) {
+    const uint32_t count = n >> level;  // entries of the input level
+    const uint32_t i = (blockIdx.x * kBlock + threadIdx.x) * 2u;
+    Box b[2];
+    for (uint32_t h = 0; h < 2; ++h) {
+        if (i + h < count) {
+            if (level == 0) {
+                const uint32_t p = vals[i + h];
+                const float4 lo = blo[p], hi = bhi[p];
+                b[h] = Box{{lo.x, lo.y, lo.z}, {hi.x, hi.y, hi.z}};
+                T.box[T.off[0] + i + h] = b[h];
+            } else {
+                b[h] = T.box[T.off[level] + i + h];
+            }
+        } else {
+            b[h] = Box{{INFINITY, INFINITY, INFINITY}, {-INFINITY, -INFINITY, -INFINITY}};
+        }
+    }
+    grow(b[0], b[1]);
+    for (int k = 1; k <= kBoxPass; ++k) {
+        const int lv = level + k;
+        if (lv >= kBoxLevels || (n >> lv) == 0) break;
+        const uint32_t l = i >> k;
+        if ((threadIdx.x & ((1u << (k - 1)) - 1u)) == 0u && l < (n >> lv)) T.box[T.off[lv] + l] = b[0];
+        if (k == kBoxPass) break;
+        Box o;
+        for (int c = 0; c < 3; ++c) {
+            o.lo[c] = __shfl_xor(b[0].lo[c], 1 << (k - 1));
+            o.hi[c] = __shfl_xor(b[0].hi[c], 1 << (k - 1));
+        }
+        grow(b[0], o);
+    }
+}
+
 // ------------------------------------------------------------------ Karras LBVH
+struct BinNode {
+    Box box;
+    uint32_t child[2];  // internal index, or kLeafFlag | sorted index
+    uint32_t first, count;  // its range of the sorted order
+};
+
 __device__ __forceinline__ int delta(const uint64_t* k, int n, int i, int j) {
     if (j < 0 || j >= n) return -1;
     uint64_t a = k[i], b = k[j];
@@ -327,8 +415,8 @@ __device__ __forceinline__ int delta(const uint64_t* k, int n, int i, int j) {
     return __clzll(a ^ b);
 }
 
-__global__ void k_karras(const uint64_t* __restrict__ keys, int n, uint2* __restrict__ child,
-                         uint2* __restrict__ range, uint32_t* __restrict__ parent_int, uint32_t* __restrict__ parent_leaf) {
+__global__ __launch_bounds__(kBlock) void k_karras(const uint64_t* __restrict__ keys, int n, BoxTree T,
+                                                   BinNode* __restrict__ bin) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n - 1) return;
     int d = (delta(keys, n, i, i + 1) - delta(keys, n, i, i - 1)) > 0 ? 1 : -1;
@@ -347,32 +435,13 @@ __global__ void k_karras(const uint64_t* __restrict__ keys, int n, uint2* __rest
     } while (t > 1);
     int gamma = i + s * d + min(d, 0);
     int lo = min(i, j), hi = max(i, j);
-    uint32_t left = (lo == gamma) ? (kLeafFlag | uint32_t(gamma)) : uint32_t(gamma);
-    uint32_t right = (hi == gamma + 1) ? (kLeafFlag | uint32_t(gamma + 1)) : uint32_t(gamma + 1);
-    child[i] = make_uint2(left, right);
-    range[i] = make_uint2(uint32_t(lo), uint32_t(hi));
-    if (left & kLeafFlag) parent_leaf[left & ~kLeafFlag] = uint32_t(i); else parent_int[left] = uint32_t(i);
-    if (right & kLeafFlag) parent_leaf[right & ~kLeafFlag] = uint32_t(i); else parent_int[right] = uint32_t(i);
-    if (i == 0) parent_int[0] = 0xFFFFFFFFu;
-}
-
-__device__ __forceinline__ void child_box(uint32_t ref, const float4* blo, const float4* bhi, const uint32_t* vals,
-                                          const float* nlo, const float* nhi, float lo[3], float hi[3]) {
-    if (ref & kLeafFlag) {
-        uint32_t p = vals[ref & ~kLeafFlag];
-        float4 a = blo[p], b = bhi[p];
-        lo[0] = a.x;
-        lo[1] = a.y;
-        lo[2] = a.z;
-        hi[0] = b.x;
-        hi[1] = b.y;
-        hi[2] = b.z;
-    } else {
-        for (int k = 0; k < 3; ++k) {
-            lo[k] = nlo[ref * 3 + k];
-            hi[k] = nhi[ref * 3 + k];
-        }
-    }
+    BinNode b;
+    b.child[0] = (lo == gamma) ? (kLeafFlag | uint32_t(gamma)) : uint32_t(gamma);
+    b.child[1] = (hi == gamma + 1) ? (kLeafFlag | uint32_t(gamma + 1)) : uint32_t(gamma + 1);
+    b.first = uint32_t(lo);
+    b.count = uint32_t(hi - lo + 1);
+    b.box = range_box(T, uint32_t(lo), uint32_t(hi));
+    bin[i] = b;
 }
 
 __device__ __forceinline__ float box_area(const float lo[3], const float hi[3]) {
@@ -396,26 +465,23 @@ struct SahCost {
 };
 struct SahParams {
     SahCost* cost;  // null: greedy collapse
-    const uint2* range;
     int leaf_max, width;
     float c_node, c_prim;
 };
 
-__device__ __forceinline__ float sah_child(const SahParams& sp, uint32_t ref, int j, const float lo[3],
-                                           const float hi[3]) {
-    return (ref & kLeafFlag) ? box_area(lo, hi) * sp.c_prim : sp.cost[ref].c[j - 1];
-}
-
-__device__ __forceinline__ void sah_node(const SahParams& sp, int i, uint2 c, const float lo[3], const float hi[3],
-                                         const float alo[3], const float ahi[3], const float blo[3],
-                                         const float bhi[3]) {
+__device__ __forceinline__ void sah_node(const SahParams& sp, int i, const BinNode& b, const Box* leaf_box) {
     const int W = sp.width;
     float cl[8], cr[8], dist[9];
     uint8_t dk[9];
+    auto side = [&](uint32_t ref, int j) {
+        if (!(ref & kLeafFlag)) return sp.cost[ref].c[j - 1];
+        const Box& q = leaf_box[ref & ~kLeafFlag];
+        return box_area(q.lo, q.hi) * sp.c_prim;
+    };
 #pragma unroll
     for (int j = 1; j <= 8; ++j) {
-        cl[j - 1] = j <= W ? sah_child(sp, c.x, j, alo, ahi) : 0.0f;
-        cr[j - 1] = j <= W ? sah_child(sp, c.y, j, blo, bhi) : 0.0f;
+        cl[j - 1] = j <= W ? side(b.child[0], j) : 0.0f;
+        cr[j - 1] = j <= W ? side(b.child[1], j) : 0.0f;
     }
     for (int j = 2; j <= W; ++j) {
         float best = INFINITY;
@@ -430,9 +496,8 @@ __device__ __forceinline__ void sah_node(const SahParams& sp, int i, uint2 c, co
         dist[j] = best;
         dk[j] = bk;
     }
-    const float A = box_area(lo, hi);
-    const uint2 rg = sp.range[i];
-    const uint32_t cnt = rg.y - rg.x + 1;
+    const float A = box_area(b.box.lo, b.box.hi);
+    const uint32_t cnt = b.count;
     const float c_leaf = cnt <= uint32_t(sp.leaf_max) ? A * float(cnt) * sp.c_prim : INFINITY;
     const float c_int = A * sp.c_node + dist[W];
     SahCost out;
@@ -452,46 +517,21 @@ __device__ __forceinline__ void sah_node(const SahParams& sp, int i, uint2 c, co
     sp.cost[i] = out;
 }
 
-// Level-synchronous refit, one round per launch: an internal node whose children were
-// finished in earlier rounds (leaves always are) gets its box and records the round. Rounds =
-// tree height. The kernel boundary makes the children's boxes visible, so the rounds need no
-// atomics or fences (a per-node climb needs agent-scope release/acquire pairs, which write back
-// and invalidate L2 across the XCDs at every step).
-// With SAH costs requested, the round also computes the node's costs from its children's.
-__global__ void k_refit_round(int nint, const uint2* __restrict__ child, const uint32_t* __restrict__ vals,
-                              const float4* __restrict__ blo, const float4* __restrict__ bhi, float* __restrict__ nlo,
-                              float* __restrict__ nhi, uint32_t* __restrict__ done, uint32_t round, SahParams sp) {
+// SAH costs, one round per launch: an internal node whose children were finished in earlier rounds
+// (leaves always are) gets its costs and records the round. Rounds = tree height. The kernel
+// boundary makes the children's costs visible, so the rounds need no atomics or fences.
+__global__ void k_sah_round(int nint, const BinNode* __restrict__ bin, const Box* __restrict__ leaf_box,
+                            uint32_t* __restrict__ done, uint32_t round, SahParams sp) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nint || done[i]) return;
-    const uint2 c = child[i];
-    const bool ra = (c.x & kLeafFlag) || (done[c.x] != 0u && done[c.x] < round);
-    const bool rb = (c.y & kLeafFlag) || (done[c.y] != 0u && done[c.y] < round);
-    if (!(ra && rb)) return;
-    float alo[3], ahi[3], blo3[3], bhi3[3];
-    child_box(c.x, blo, bhi, vals, nlo, nhi, alo, ahi);
-    child_box(c.y, blo, bhi, vals, nlo, nhi, blo3, bhi3);
-    float lo[3], hi[3];
-    for (int k = 0; k < 3; ++k) {
-        lo[k] = fminf(alo[k], blo3[k]);
-        hi[k] = fmaxf(ahi[k], bhi3[k]);
-        nlo[i * 3 + k] = lo[k];
-        nhi[i * 3 + k] = hi[k];
-    }
-    if (sp.cost) sah_node(sp, i, c, lo, hi, alo, ahi, blo3, bhi3);
+    const BinNode b = bin[i];
+    for (int k = 0; k < 2; ++k)
+        if (!(b.child[k] & kLeafFlag) && (done[b.child[k]] == 0u || done[b.child[k]] >= round)) return;
+    sah_node(sp, i, b, leaf_box);
     done[i] = round;
 }
 
 // ------------------------------------------------------------------ collapse to 8-wide
-struct Task {
-    uint32_t bref;   // binary node (internal index or kLeafFlag | sorted index)
-    uint32_t wnode;  // wide node to fill
-};
-
-__device__ __forceinline__ float area(const float lo[3], const float hi[3]) {
-    float dx = hi[0] - lo[0], dy = hi[1] - lo[1], dz = hi[2] - lo[2];
-    return dx * dy + dy * dz + dz * dx;
-}
-
 __device__ __forceinline__ uint32_t fexp_for(float extent) {
     // smallest power of two s with 255 * s >= extent; returns the biased exponent byte
     float x = extent / 255.0f;
@@ -502,223 +542,267 @@ __device__ __forceinline__ uint32_t fexp_for(float extent) {
     return uint32_t(max(1, min(254, b)));
 }
 
-__global__ void k_collapse(const Task* __restrict__ tin, const uint32_t* __restrict__ ntin, Task* __restrict__ tout,
-                           uint32_t* __restrict__ ntout, uint32_t* __restrict__ node_counter,
-                           uint32_t* __restrict__ prim_counter, int n, int leaf_max, int width,
-                           const uint2* __restrict__ child,
-                           const uint2* __restrict__ range, const uint32_t* __restrict__ vals,
-                           const float4* __restrict__ blo, const float4* __restrict__ bhi, const float* __restrict__ nlo,
-                           const float* __restrict__ nhi, WideNode* __restrict__ nodes,
-                           uint32_t* __restrict__ prim_slots, SahParams sp) {
-    uint32_t ti = blockIdx.x * blockDim.x + threadIdx.x;
-    if (ti >= *ntin) return;
-    Task task = tin[ti];
-    uint32_t ref[8], cnt[8], first[8];
-    float lo[8][3], hi[8][3];
-    int ne = 0;
-    auto load = [&](int e, uint32_t r) {
-        ref[e] = r;
-        if (r & kLeafFlag) {
-            cnt[e] = 1;
-            first[e] = r & ~kLeafFlag;
-            uint32_t p = vals[first[e]];
-            float4 a = blo[p], b = bhi[p];
-            lo[e][0] = a.x;
-            lo[e][1] = a.y;
-            lo[e][2] = a.z;
-            hi[e][0] = b.x;
-            hi[e][1] = b.y;
-            hi[e][2] = b.z;
-        } else {
-            uint2 rg = range[r];
-            cnt[e] = rg.y - rg.x + 1;
-            first[e] = rg.x;
-            for (int k = 0; k < 3; ++k) {
-                lo[e][k] = nlo[r * 3 + k];
-                hi[e][k] = nhi[r * 3 + k];
+// Top-down collapse, one tree level per launch. Eight lanes make one wide node: lane e of the group
+// holds child e, so the opening, the slot order and the quantization run one child per lane in
+// registers. (One thread per node kept the eight boxes in scratch memory and walked them in
+// series: 2666 us for the 10 levels of 3.2M curves, 73 us per level even for a few nodes; now 1205
+// and about 18. Bound by the chain of dependent loads while a node is opened.)
+// The nodes of a level are consecutive, bounds[level] .. bounds[level + 1], and tasks[w] is the
+// binary node that wide node w covers; a block allocates the children and leaf records of its 32
+// nodes with one atomic on the packed counter (nodes in the low, records in the high half). The
+// last block to finish records where the next level ends.
+constexpr uint32_t kCollapseNodes = kBlock / 8;  // wide nodes per block and pass
+constexpr uint32_t kMaxWideLevels = 128;         // a binary tree over 64-bit keys and 32-bit ties is at most 96 deep
+
+struct CollapseState {
+    unsigned long long alloc;  // wide nodes | leaf records << 32
+    uint32_t bounds[kMaxWideLevels + 2];
+    uint32_t done[kMaxWideLevels];  // blocks finished per level
+};
+
+__device__ __forceinline__ float group_min8(float v) {
+    for (int k = 1; k < 8; k <<= 1) v = fminf(v, __shfl_xor(v, k));
+    return v;
+}
+__device__ __forceinline__ float group_max8(float v) {
+    for (int k = 1; k < 8; k <<= 1) v = fmaxf(v, __shfl_xor(v, k));
+    return v;
+}
+__device__ __forceinline__ uint32_t group_or8(uint32_t v) {
+    for (int k = 1; k < 8; k <<= 1) v |= __shfl_xor(v, k);
+    return v;
+}
+
+__global__ __launch_bounds__(kBlock) void k_collapse(uint32_t level, CollapseState* __restrict__ state,
+                                                     uint32_t* __restrict__ tasks, uint32_t n, int leaf_max, int width,
+                                                     const BinNode* __restrict__ bin, const Box* __restrict__ leaf_box,
+                                                     const uint32_t* __restrict__ vals, WideNode* __restrict__ nodes,
+                                                     uint32_t* __restrict__ prim_slots, SahParams sp) {
+    __shared__ uint32_t s_node[kCollapseNodes * sizeof(WideNode) / 4];
+    __shared__ uint32_t s_nint[kCollapseNodes], s_nprim[kCollapseNodes];  // then their offsets
+    const uint32_t begin = state->bounds[level], end = min(state->bounds[level + 1], n);
+    const uint32_t sub = threadIdx.x & 7u, grp = threadIdx.x >> 3;
+    const int lane0 = int(threadIdx.x & 56u);  // first lane of the group
+    for (uint32_t base = begin + blockIdx.x * kCollapseNodes; base < end; base += gridDim.x * kCollapseNodes) {
+        const uint32_t w = base + grp;
+        const bool live = w < end;
+        // child `sub`: reference, box, range and (internal) its own children
+        uint32_t ref = 0, cnt = 0, first = 0, c0 = 0, c1 = 0;
+        Box box{{INFINITY, INFINITY, INFINITY}, {-INFINITY, -INFINITY, -INFINITY}};
+        bool is_int = false;
+        uint32_t ne = 0;
+        auto load = [&](uint32_t r) {
+            ref = r;
+            if (r & kLeafFlag) {
+                cnt = 1;
+                first = r & ~kLeafFlag;
+                box = leaf_box[first];
+            } else {
+                const BinNode b = bin[r];
+                cnt = b.count;
+                first = b.first;
+                box = b.box;
+                c0 = b.child[0];
+                c1 = b.child[1];
             }
-        }
-    };
-    bool is_int[8];
-    if (task.bref & kLeafFlag) {
-        load(0, task.bref);
-        ne = 1;
-    } else if (sp.cost) {
-        // the slots recorded by the cost pass: D(root, width) split, each side expanded along
-        // its choices (a binary leaf, or one slot, ends the expansion)
-        uint2 stk[16];
-        int sn = 0;
-        const uint2 c = child[task.bref];
-        const int k = int(sp.cost[task.bref].kint);
-        stk[sn++] = make_uint2(c.y, uint32_t(width - k));
-        stk[sn++] = make_uint2(c.x, uint32_t(k));
-        while (sn > 0 && ne < 8) {
-            const uint2 t = stk[--sn];
-            const uint32_t m = t.x;
-            const int j = int(t.y);
-            if ((m & kLeafFlag) || j <= 1) {
-                load(ne, m);
-                is_int[ne] = !(m & kLeafFlag) && sp.cost[m].dec[0] == 0;
-                ++ne;
-                continue;
-            }
-            const int d = sp.cost[m].dec[j - 1];
-            if (d == 0) {
-                stk[sn++] = make_uint2(m, uint32_t(j - 1));
-            } else if (sn + 2 <= 16) {
-                const uint2 cm = child[m];
-                stk[sn++] = make_uint2(cm.y, uint32_t(j - d));
-                stk[sn++] = make_uint2(cm.x, uint32_t(d));
-            }
-        }
-    } else {
-        uint2 c = child[task.bref];
-        load(0, c.x);
-        load(1, c.y);
-        ne = 2;
-    }
-    while (!sp.cost && ne < width) {
-        int best = -1;
-        float ba = -1.0f;
-        for (int e = 0; e < ne; ++e) {
-            if ((ref[e] & kLeafFlag) || cnt[e] <= uint32_t(leaf_max)) continue;
-            float a = area(lo[e], hi[e]);
-            if (a > ba) {
-                ba = a;
-                best = e;
-            }
-        }
-        if (best < 0) break;
-        uint2 c = child[ref[best]];
-        load(best, c.x);
-        load(ne, c.y);
-        ++ne;
-    }
-    // node box and centroid
-    float nb_lo[3] = {INFINITY, INFINITY, INFINITY}, nb_hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (int e = 0; e < ne; ++e)
-        for (int k = 0; k < 3; ++k) {
-            nb_lo[k] = fminf(nb_lo[k], lo[e][k]);
-            nb_hi[k] = fmaxf(nb_hi[k], hi[e][k]);
-        }
-    // octant slot assignment: slot s should hold the child met first along direction
-    // d_s = ((s&1)?-1:1, (s&2)?-1:1, (s&4)?-1:1), i.e. the lowest dot(centroid offset, d_s)
-    float off[8][3];
-    for (int e = 0; e < ne; ++e)
-        for (int k = 0; k < 3; ++k)
-            off[e][k] = (0.5f * lo[e][k] + 0.5f * hi[e][k]) - (0.5f * nb_lo[k] + 0.5f * nb_hi[k]);
-    int slot_of[8];
-    uint32_t used_slots = 0, used_e = 0;
-    for (int round = 0; round < ne; ++round) {
-        float bc = INFINITY;
-        int be = -1, bs = -1;
-        for (int e = 0; e < ne; ++e) {
-            if (used_e & (1u << e)) continue;
-            for (int s = 0; s < 8; ++s) {
-                if (used_slots & (1u << s)) continue;
-                float c = ((s & 1) ? -off[e][0] : off[e][0]) + ((s & 2) ? -off[e][1] : off[e][1]) +
-                          ((s & 4) ? -off[e][2] : off[e][2]);
-                if (c < bc) {
-                    bc = c;
-                    be = e;
-                    bs = s;
+        };
+        const uint32_t bref = live ? tasks[w] : kLeafFlag;
+        const bool single = (bref & kLeafFlag) != 0;  // a tree of one primitive
+        if (live && single) {
+            if (sub == 0) load(bref);
+            ne = 1;
+        } else if (live && sp.cost) {
+            // the slots recorded by the cost pass: D(root, width) split, each side expanded along
+            // its choices (a binary leaf, or one slot, ends the expansion)
+            uint2 stk[16];
+            int sn = 0;
+            const BinNode& b = bin[bref];
+            const int k = int(sp.cost[bref].kint);
+            stk[sn++] = make_uint2(b.child[1], uint32_t(width - k));
+            stk[sn++] = make_uint2(b.child[0], uint32_t(k));
+            while (sn > 0 && ne < 8) {
+                const uint2 t = stk[--sn];
+                const uint32_t m = t.x;
+                const int j = int(t.y);
+                if ((m & kLeafFlag) || j <= 1) {
+                    if (sub == ne) {
+                        load(m);
+                        is_int = !(m & kLeafFlag) && sp.cost[m].dec[0] == 0;
+                    }
+                    ++ne;
+                    continue;
+                }
+                const int d = sp.cost[m].dec[j - 1];
+                if (d == 0) {
+                    stk[sn++] = make_uint2(m, uint32_t(j - 1));
+                } else if (sn + 2 <= 16) {
+                    stk[sn++] = make_uint2(bin[m].child[1], uint32_t(j - d));
+                    stk[sn++] = make_uint2(bin[m].child[0], uint32_t(d));
                 }
             }
+        } else if (live) {
+            if (sub < 2) load(bin[bref].child[sub]);
+            ne = 2;
         }
-        if (be < 0) {  // NaN costs: take the first free pair
-            for (int e = 0; e < ne && be < 0; ++e)
-                if (!(used_e & (1u << e))) be = e;
-            for (int s = 0; s < 8 && bs < 0; ++s)
-                if (!(used_slots & (1u << s))) bs = s;
+        if (!sp.cost) {
+            // greedy: open the child of the largest area (the first of equals) until `width`
+            bool more = live && !single && ne < uint32_t(width);
+            while (__ballot(more)) {
+                float a = -1.0f;
+                if (more && sub < ne && !(ref & kLeafFlag) && cnt > uint32_t(leaf_max)) {
+                    const float q = box_area(box.lo, box.hi);
+                    if (q > a) a = q;  // not a NaN
+                }
+                uint32_t best = sub;
+                for (int k = 1; k < 8; k <<= 1) {
+                    const float oa = __shfl_xor(a, k);
+                    const uint32_t ob = __shfl_xor(best, k);
+                    if (oa > a || (oa == a && ob < best)) {
+                        a = oa;
+                        best = ob;
+                    }
+                }
+                const uint32_t r0 = __shfl(c0, lane0 + int(best)), r1 = __shfl(c1, lane0 + int(best));
+                more = more && a >= 0.0f;
+                if (more) {
+                    if (sub == best) load(r0);
+                    if (sub == ne) load(r1);
+                    more = ++ne < uint32_t(width);
+                }
+            }
+            is_int = live && !single && sub < ne && !(ref & kLeafFlag) && cnt > uint32_t(leaf_max);
         }
-        slot_of[be] = bs;
-        used_e |= 1u << be;
-        used_slots |= 1u << bs;
-    }
-    // quantization frame
-    uint32_t ebyte[3];
-    float scale[3];
-    for (int k = 0; k < 3; ++k) {
-        uint32_t eb = fexp_for(nb_hi[k] - nb_lo[k]);
-        for (;;) {
-            float s = __uint_as_float(eb << 23);
-            if (nb_lo[k] + 255.0f * s >= nb_hi[k] || eb >= 254) break;
-            ++eb;
-        }
-        ebyte[k] = eb;
-        scale[k] = __uint_as_float(eb << 23);
-    }
-    // allocation of children
-    int n_int = 0;
-    uint32_t n_prims = 0;
-    uint32_t slot_entry[8];
-    for (int s = 0; s < 8; ++s) slot_entry[s] = 0xFFu;
-    for (int e = 0; e < ne; ++e) slot_entry[slot_of[e]] = uint32_t(e);
-    for (int e = 0; e < ne; ++e) {
-        if (!sp.cost || (task.bref & kLeafFlag)) is_int[e] = !(ref[e] & kLeafFlag) && cnt[e] > uint32_t(leaf_max);
-        if (is_int[e])
-            ++n_int;
-        else
-            n_prims += cnt[e];
-    }
-    uint32_t cbase = n_int ? atomicAdd(node_counter, uint32_t(n_int)) : 0u;
-    uint32_t pbase = n_prims ? atomicAdd(prim_counter, n_prims) : 0u;
-    // capacity guards (a consistent tree never trips them; the host checks the counters)
-    if (cbase + uint32_t(n_int) > uint32_t(n) || pbase + n_prims > uint32_t(n)) return;
-    WideNode W;
-    W.px = nb_lo[0];
-    W.py = nb_lo[1];
-    W.pz = nb_lo[2];
-    uint32_t imask = 0;
-    uint8_t meta[8], ql[3][8], qh[3][8];
-    uint32_t rank = 0, poff = 0;
-    for (int s = 0; s < 8; ++s) {
-        meta[s] = 0;
+        const bool mine = sub < ne;
+        // node box, and the child's centre relative to the node's
+        Box nb;
+        float off[3];
         for (int k = 0; k < 3; ++k) {
-            ql[k][s] = 0;
-            qh[k][s] = 0;
+            nb.lo[k] = group_min8(box.lo[k]);
+            nb.hi[k] = group_max8(box.hi[k]);
+            off[k] = (0.5f * box.lo[k] + 0.5f * box.hi[k]) - (0.5f * nb.lo[k] + 0.5f * nb.hi[k]);
         }
-        uint32_t e = slot_entry[s];
-        if (e == 0xFFu) continue;
+        // octant slot assignment: slot s should hold the child met first along direction
+        // d_s = ((s&1)?-1:1, (s&2)?-1:1, (s&4)?-1:1), i.e. the lowest dot(centroid offset, d_s);
+        // per round the lowest cost of all free children and slots is placed (ties: the first
+        // child, its first slot; NaN costs take the first free pair)
+        uint32_t slot = 8, used = 0;
+        for (int round = 0; round < 8; ++round) {
+            float bc = INFINITY;
+            uint32_t bs = __ffs(~used) - 1u;
+            if (mine && slot == 8u)
+                for (uint32_t s = 0; s < 8; ++s) {
+                    const float c = ((s & 1) ? -off[0] : off[0]) + ((s & 2) ? -off[1] : off[1]) +
+                                    ((s & 4) ? -off[2] : off[2]);
+                    if (!((used >> s) & 1u) && c < bc) {
+                        bc = c;
+                        bs = s;
+                    }
+                }
+            uint32_t be = (mine && slot == 8u ? sub : sub + 8u) | (bs << 8);  // placed children lose every tie
+            for (int k = 1; k < 8; k <<= 1) {
+                const float oc = __shfl_xor(bc, k);
+                const uint32_t oe = __shfl_xor(be, k);
+                if (oc < bc || (oc == bc && (oe & 255u) < (be & 255u))) {
+                    bc = oc;
+                    be = oe;
+                }
+            }
+            if ((be & 255u) < 8u) {
+                if (sub == (be & 255u)) slot = be >> 8;
+                used |= 1u << (be >> 8);
+            }
+        }
+        // quantization frame
+        uint32_t ebyte[3];
+        float scale[3];
         for (int k = 0; k < 3; ++k) {
-            float org = nb_lo[k];
-            int q0 = int(floorf((lo[e][k] - org) / scale[k]));
-            q0 = max(0, min(255, q0));
-            while (q0 > 0 && org + float(q0) * scale[k] > lo[e][k]) --q0;
-            int q1 = int(ceilf((hi[e][k] - org) / scale[k]));
-            q1 = max(0, min(255, q1));
-            while (q1 < 255 && org + float(q1) * scale[k] < hi[e][k]) ++q1;
-            ql[k][s] = uint8_t(q0);
-            qh[k][s] = uint8_t(q1);
+            uint32_t eb = fexp_for(nb.hi[k] - nb.lo[k]);
+            for (;;) {
+                float s = __uint_as_float(eb << 23);
+                if (!(nb.lo[k] + 255.0f * s < nb.hi[k]) || eb >= 254) break;
+                ++eb;
+            }
+            ebyte[k] = eb;
+            scale[k] = __uint_as_float(eb << 23);
         }
-        if (is_int[e]) {
-            imask |= 1u << s;
-            meta[s] = 0x80;
-            uint32_t wi = cbase + rank;
-            ++rank;
-            uint32_t to = atomicAdd(ntout, 1u);
-            if (to <= uint32_t(n)) tout[to] = Task{ref[e], wi};
-        } else {
-            meta[s] = uint8_t((cnt[e] << 5) | poff);
-            for (uint32_t j = 0; j < cnt[e]; ++j) prim_slots[pbase + poff + j] = vals[first[e] + j];
-            poff += cnt[e];
+        // children in slot order: internal children ranked, leaf records by their counts (1..3)
+        const uint32_t imask = group_or8(mine && is_int ? 1u << slot : 0u);
+        const uint32_t counts = group_or8(mine && !is_int ? cnt << (2u * slot) : 0u);
+        const uint32_t below = (1u << slot) - 1u;
+        uint32_t poff = 0, n_prims = 0;
+        for (uint32_t s = 0; s < 8; ++s) {
+            const uint32_t c = (counts >> (2u * s)) & 3u;
+            n_prims += c;
+            poff += s < slot ? c : 0u;
         }
+        if (sub == 0) {
+            s_nint[grp] = live ? __popc(imask) : 0u;
+            s_nprim[grp] = live ? n_prims : 0u;
+        }
+        for (uint32_t i = threadIdx.x; i < kCollapseNodes * sizeof(WideNode) / 4; i += kBlock) s_node[i] = 0u;
+        __syncthreads();
+        if (threadIdx.x < kCollapseNodes) {
+            const uint32_t a = s_nint[threadIdx.x], b = s_nprim[threadIdx.x];
+            uint32_t sa = a, sb = b;
+            for (uint32_t k = 1; k < kCollapseNodes; k <<= 1) {
+                const uint32_t xa = __shfl_up(sa, k), xb = __shfl_up(sb, k);
+                if (threadIdx.x >= k) {
+                    sa += xa;
+                    sb += xb;
+                }
+            }
+            unsigned long long at = 0;
+            if (threadIdx.x == kCollapseNodes - 1)
+                at = atomicAdd(&state->alloc, (static_cast<unsigned long long>(sb) << 32) | sa);
+            at = __shfl(at, int(kCollapseNodes - 1));
+            s_nint[threadIdx.x] = uint32_t(at) + sa - a;
+            s_nprim[threadIdx.x] = uint32_t(at >> 32) + sb - b;
+        }
+        __syncthreads();
+        const uint32_t cbase = s_nint[grp], pbase = s_nprim[grp];
+        // capacity guards (a consistent tree never trips them; the host checks the counters)
+        const bool fits = cbase + __popc(imask) <= n && pbase + n_prims <= n;
+        if (live && mine && fits) {
+            uint8_t* q = reinterpret_cast<uint8_t*>(s_node + grp * (sizeof(WideNode) / 4)) + slot;
+            for (int k = 0; k < 3; ++k) {
+                const float org = nb.lo[k];
+                int q0 = int(floorf((box.lo[k] - org) / scale[k]));
+                q0 = max(0, min(255, q0));
+                while (q0 > 0 && org + float(q0) * scale[k] > box.lo[k]) --q0;
+                int q1 = int(ceilf((box.hi[k] - org) / scale[k]));
+                q1 = max(0, min(255, q1));
+                while (q1 < 255 && org + float(q1) * scale[k] < box.hi[k]) ++q1;
+                q[offsetof(WideNode, qlo_x) + 8 * k] = uint8_t(q0);
+                q[offsetof(WideNode, qhi_x) + 8 * k] = uint8_t(q1);
+            }
+            if (is_int) {
+                q[offsetof(WideNode, meta)] = 0x80u;
+                tasks[cbase + __popc(imask & below)] = ref;
+            } else {
+                q[offsetof(WideNode, meta)] = uint8_t((cnt << 5) | poff);
+                for (uint32_t j = 0; j < cnt; ++j) prim_slots[pbase + poff + j] = vals[first + j];
+            }
+            if (sub == 0) {
+                uint32_t* h = s_node + grp * (sizeof(WideNode) / 4);
+                h[0] = __float_as_uint(nb.lo[0]);
+                h[1] = __float_as_uint(nb.lo[1]);
+                h[2] = __float_as_uint(nb.lo[2]);
+                h[3] = ebyte[0] | (ebyte[1] << 8) | (ebyte[2] << 16) | (imask << 24);
+                h[4] = cbase;
+                h[5] = pbase;
+            }
+        }
+        __syncthreads();
+        const uint32_t words = min(kCollapseNodes, end - base) * uint32_t(sizeof(WideNode) / 4);
+        uint32_t* dst = reinterpret_cast<uint32_t*>(nodes + base);
+        for (uint32_t i = threadIdx.x; i < words; i += kBlock) dst[i] = s_node[i];
+        __syncthreads();
     }
-    W.e_imask = ebyte[0] | (ebyte[1] << 8) | (ebyte[2] << 16) | (imask << 24);
-    W.child_base = cbase;
-    W.prim_base = pbase;
-    auto pack = [](const uint8_t* b, uint32_t* o) {
-        o[0] = uint32_t(b[0]) | (uint32_t(b[1]) << 8) | (uint32_t(b[2]) << 16) | (uint32_t(b[3]) << 24);
-        o[1] = uint32_t(b[4]) | (uint32_t(b[5]) << 8) | (uint32_t(b[6]) << 16) | (uint32_t(b[7]) << 24);
-    };
-    pack(meta, W.meta);
-    pack(ql[0], W.qlo_x);
-    pack(ql[1], W.qlo_y);
-    pack(ql[2], W.qlo_z);
-    pack(qh[0], W.qhi_x);
-    pack(qh[1], W.qhi_y);
-    pack(qh[2], W.qhi_z);
-    nodes[task.wnode] = W;
+    if (threadIdx.x == 0) {
+        __threadfence();
+        if (atomicAdd(&state->done[level], 1u) == gridDim.x - 1)
+            state->bounds[level + 2] = uint32_t(atomicAdd(&state->alloc, 0ull));
+    }
 }
 
 __global__ void k_gather(const float4* __restrict__ in, const uint32_t* __restrict__ slots, uint32_t n, int rec,
@@ -756,10 +840,14 @@ __global__ void k_set_u32(uint32_t* p, uint32_t v, uint32_t n) {
     if (i < n) p[i] = v;
 }
 
-__global__ void k_root_task(Task* t, uint32_t* nt, uint32_t* node_counter, uint32_t bref) {
-    t[0] = Task{bref, 0u};
-    *nt = 1u;
-    *node_counter = 1u;
+__global__ void k_collapse_init(CollapseState* state, uint32_t* tasks, uint32_t root) {
+    for (uint32_t i = threadIdx.x; i < kMaxWideLevels; i += blockDim.x) state->done[i] = 0u;
+    if (threadIdx.x == 0) {
+        state->alloc = 1ull;  // the root
+        state->bounds[0] = 0u;
+        state->bounds[1] = 1u;
+        tasks[0] = root;
+    }
 }
 
 template <class T>
@@ -787,20 +875,19 @@ hipError_t build_bvh(int mode, const float4* prims_in, uint32_t n, int radius_mo
     uint32_t* cb = nullptr;
     uint64_t *k0 = nullptr, *k1 = nullptr;
     uint32_t *v0 = nullptr, *v1 = nullptr, *hist = nullptr, *scan_sums = nullptr;
-    uint2 *child = nullptr, *range = nullptr;
-    uint32_t *par_i = nullptr, *par_l = nullptr, *counters = nullptr;
-    float *nlo = nullptr, *nhi = nullptr;
-    Task *ta = nullptr, *tb = nullptr;
+    BoxTree tree{};
+    BinNode* bin = nullptr;
+    uint32_t *tasks = nullptr, *done = nullptr;
+    CollapseState* state = nullptr;
     SahParams sp{};
-    uint32_t* cnt = nullptr;  // [0] ntasks a, [1] ntasks b, [2] nodes, [3] prims
     WideNode* nodes = nullptr;
     uint32_t* slots = nullptr;
     float4* prims_sorted = nullptr;
     float* aux = nullptr;
     hipError_t rc = hipSuccess;
     uint32_t nb = 0;
-    uint32_t host_cnt[4] = {0, 0, 0, 0};
-    uint32_t cur = 0;
+    CollapseState fin{};
+    size_t boxes = 0;
     uint32_t cb_host[6];
     *out = BuiltBvh{};
     if (n == 0) return hipSuccess;
@@ -819,23 +906,21 @@ hipError_t build_bvh(int mode, const float4* prims_in, uint32_t n, int radius_mo
     nb = blocks(n, kRsTile);
     VK_TRY(dalloc(&hist, size_t(nb) * 256));
     VK_TRY(dalloc(&scan_sums, (size_t(nb) * 256 + kScanTile - 1) / kScanTile));
-    VK_TRY(dalloc(&child, n));
-    VK_TRY(dalloc(&range, n));
-    VK_TRY(dalloc(&par_i, n));
-    VK_TRY(dalloc(&par_l, n));
-    VK_TRY(dalloc(&counters, n));
-    VK_TRY(dalloc(&nlo, size_t(n) * 3));
-    VK_TRY(dalloc(&nhi, size_t(n) * 3));
-    VK_TRY(dalloc(&ta, n + 1));
-    VK_TRY(dalloc(&tb, n + 1));
-    VK_TRY(dalloc(&cnt, 4));
+    for (int k = 0; k < kBoxLevels; ++k) {
+        tree.off[k] = boxes;
+        boxes += n >> k;
+    }
+    VK_TRY(dalloc(&tree.box, boxes));
+    VK_TRY(dalloc(&bin, n));
+    VK_TRY(dalloc(&tasks, n));
+    VK_TRY(dalloc(&state, 1));
     VK_TRY(dalloc(&nodes, n));
     VK_TRY(dalloc(&slots, n));
     VK_TRY(dalloc(&prims_sorted, size_t(n) * rec));
     if (mode == kPhantom) VK_TRY(dalloc(&aux, n));
     if (collapse > 0 && n >= 2) {
         VK_TRY(dalloc(&sp.cost, n));
-        sp.range = range;
+        VK_TRY(dalloc(&done, n));
         sp.leaf_max = leaf_max;
         sp.width = width;
         sp.c_node = 1.0f;
@@ -861,42 +946,54 @@ hipError_t build_bvh(int mode, const float4* prims_in, uint32_t n, int radius_mo
         std::swap(v0, v1);
     }
     VK_TRY(hipGetLastError());
-    if (n >= 2) {
-        hipLaunchKernelGGL(k_karras, dim3(blocks(n - 1)), dim3(kBlock), 0, st, k0, int(n), child, range, par_i, par_l);
-        hipLaunchKernelGGL(k_set_u32, dim3(blocks(n)), dim3(kBlock), 0, st, counters, 0u, n);
+    for (int lv = 0; lv == 0 || (n >> lv) > 1; lv += kBoxPass)
+        hipLaunchKernelGGL(k_box_levels, dim3(blocks(n >> lv, 2 * kBlock)), dim3(kBlock), 0, st, tree, n, lv, v0, blo, bhi);
+    if (n >= 2) hipLaunchKernelGGL(k_karras, dim3(blocks(n - 1)), dim3(kBlock), 0, st, k0, int(n), tree, bin);
+    VK_TRY(hipGetLastError());
+    if (sp.cost) {
+        hipLaunchKernelGGL(k_set_u32, dim3(blocks(n)), dim3(kBlock), 0, st, done, 0u, n);
         // rounds in groups of 8; the root is the last node to finish
         uint32_t root_done = 0;
         for (uint32_t round = 1; !root_done; round += 8) {
             if (round > 8192) {
-                err = "BVH refit did not reach the root";
+                err = "BVH cost rounds did not reach the root";
                 rc = hipErrorUnknown;
                 goto fail;
             }
             for (uint32_t r = round; r < round + 8; ++r)
-                hipLaunchKernelGGL(k_refit_round, dim3(blocks(n - 1)), dim3(kBlock), 0, st, int(n - 1), child, v0, blo,
-                                   bhi, nlo, nhi, counters, r, sp);
+                hipLaunchKernelGGL(k_sah_round, dim3(blocks(n - 1)), dim3(kBlock), 0, st, int(n - 1), bin, tree.box, done, r,
+                                   sp);
             VK_TRY(hipGetLastError());
-            VK_TRY(hipMemcpyAsync(&root_done, counters, 4, hipMemcpyDeviceToHost, st));
+            VK_TRY(hipMemcpyAsync(&root_done, done, 4, hipMemcpyDeviceToHost, st));
             VK_TRY(hipStreamSynchronize(st));
         }
     }
-    hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(64), 0, st, cnt, 0u, 4u);
-    hipLaunchKernelGGL(k_root_task, dim3(1), dim3(1), 0, st, ta, cnt + 0, cnt + 2, n >= 2 ? 0u : kLeafFlag);
-    VK_TRY(hipGetLastError());
-    cur = 1;
-    for (int level = 0; level < 4096 && cur > 0; ++level) {
-        uint32_t* nin = cnt + (level & 1);
-        uint32_t* nout = cnt + ((level & 1) ^ 1);
-        hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(64), 0, st, nout, 0u, 1u);
-        hipLaunchKernelGGL(k_collapse, dim3(blocks(cur, 64)), dim3(64), 0, st, (level & 1) ? tb : ta, nin,
-                           (level & 1) ? ta : tb, nout, cnt + 2, cnt + 3, int(n), leaf_max, width, child, range, v0, blo, bhi,
-                           nlo, nhi, nodes, slots, sp);
-        VK_TRY(hipGetLastError());
-        VK_TRY(hipMemcpyAsync(&cur, nout, 4, hipMemcpyDeviceToHost, st));
-        VK_TRY(hipStreamSynchronize(st));
-        out->depth = uint32_t(level + 1);
+    hipLaunchKernelGGL(k_collapse_init, dim3(1), dim3(64), 0, st, state, tasks, n >= 2 ? 0u : kLeafFlag);
+    {
+        // as many levels as an evenly filled tree of this size has and three more, then four at a time; level L has
+        // at most 8^L nodes
+        uint32_t level = 0, until = 3, depth = 0;
+        for (uint64_t m = 1; m < n; m *= 8) ++until;
+        while (depth == 0) {
+            if (until > kMaxWideLevels) {
+                err = "BVH collapse did not reach the leaves";
+                rc = hipErrorUnknown;
+                goto fail;
+            }
+            for (; level < until; ++level) {
+                const uint64_t most = level < 10 ? std::min<uint64_t>(n, 1ull << (3 * level)) : n;
+                hipLaunchKernelGGL(k_collapse, dim3(std::min<uint32_t>(blocks(most, kCollapseNodes), 4096u)), dim3(kBlock), 0,
+                                   st, level, state, tasks, n, leaf_max, width, bin, tree.box, v0, nodes, slots, sp);
+            }
+            VK_TRY(hipGetLastError());
+            VK_TRY(hipMemcpyAsync(&fin, state, sizeof(fin), hipMemcpyDeviceToHost, st));
+            VK_TRY(hipStreamSynchronize(st));
+            for (uint32_t l = 1; l <= level && !depth; ++l)
+                if (fin.bounds[l + 1] == fin.bounds[l]) depth = l;
+            until = level + 4;
+        }
+        out->depth = depth;
     }
-    VK_TRY(hipMemcpyAsync(host_cnt, cnt, 16, hipMemcpyDeviceToHost, st));
     VK_TRY(hipMemcpyAsync(cb_host, cb, 24, hipMemcpyDeviceToHost, st));
     hipLaunchKernelGGL(k_gather, dim3(blocks(uint64_t(n) * rec)), dim3(kBlock), 0, st, prims_in, slots, n, rec,
                        prims_sorted);
@@ -905,8 +1002,8 @@ hipError_t build_bvh(int mode, const float4* prims_in, uint32_t n, int radius_mo
                            aux);
     VK_TRY(hipGetLastError());
     VK_TRY(hipStreamSynchronize(st));
-    if (host_cnt[3] != n || host_cnt[2] > n) {
-        err = "BVH collapse placed " + std::to_string(host_cnt[3]) + " of " + std::to_string(n) + " primitives";
+    if (uint32_t(fin.alloc >> 32) != n || uint32_t(fin.alloc) > n) {
+        err = "BVH collapse placed " + std::to_string(uint32_t(fin.alloc >> 32)) + " of " + std::to_string(n) + " primitives";
         rc = hipErrorUnknown;
         goto fail;
     }
@@ -916,7 +1013,7 @@ hipError_t build_bvh(int mode, const float4* prims_in, uint32_t n, int radius_mo
         out->depth = depth;
     }
     out->nodes = nodes;
-    out->nnodes = host_cnt[2];
+    out->nnodes = uint32_t(fin.alloc);
     out->prim_ids = slots;
     out->prims = prims_sorted;
     out->aux = aux;
@@ -937,16 +1034,11 @@ done:
     hipFree(v1);
     hipFree(hist);
     hipFree(scan_sums);
-    hipFree(child);
-    hipFree(range);
-    hipFree(par_i);
-    hipFree(par_l);
-    hipFree(counters);
-    hipFree(nlo);
-    hipFree(nhi);
-    hipFree(ta);
-    hipFree(tb);
-    hipFree(cnt);
+    hipFree(tree.box);
+    hipFree(bin);
+    hipFree(tasks);
+    hipFree(done);
+    hipFree(state);
     hipFree(nodes);
     hipFree(slots);
     hipFree(prims_sorted);
