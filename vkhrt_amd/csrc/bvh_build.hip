@@ -26,6 +26,7 @@
 
 #include <algorithm>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "build.hpp"
@@ -545,13 +546,15 @@ __device__ __forceinline__ uint32_t fexp_for(float extent) {
 // Top-down collapse, one tree level per launch. Eight lanes make one wide node: lane e of the group
 // holds child e, so the opening, the slot order and the quantization run one child per lane in
 // registers. (One thread per node kept the eight boxes in scratch memory and walked them in
-// series: 2666 us for the 10 levels of 3.2M curves, 73 us per level even for a few nodes; now 1205
-// and about 18. Bound by the chain of dependent loads while a node is opened.)
+// series: 2666 us for the 10 levels of 3.2M curves, 73 us per level even for a few nodes; now 772
+// and about 15. Bound by the chain of dependent loads while a node is opened.)
 // The nodes of a level are consecutive, bounds[level] .. bounds[level + 1], and tasks[w] is the
-// binary node that wide node w covers; a block allocates the children and leaf records of its 32
-// nodes with one atomic on the packed counter (nodes in the low, records in the high half). The
-// last block to finish records where the next level ends.
-constexpr uint32_t kCollapseNodes = kBlock / 8;  // wide nodes per block and pass
+// binary node that wide node w covers; a block allocates the children and leaf records of its 128
+// nodes with one atomic on the packed counter (nodes in the low, records in the high half): atomics
+// on one address take about 18 ns each, one after the other, which with 32 nodes per block was the
+// time of the large levels. The last working block to finish records where the next level ends.
+constexpr uint32_t kCollapseBlock = 1024;
+constexpr uint32_t kCollapseNodes = kCollapseBlock / 8;  // wide nodes per block and pass
 constexpr uint32_t kMaxWideLevels = 128;         // a binary tree over 64-bit keys and 32-bit ties is at most 96 deep
 
 struct CollapseState {
@@ -560,20 +563,34 @@ struct CollapseState {
     uint32_t done[kMaxWideLevels];  // blocks finished per level
 };
 
+// Value of a lane in another part of the caller's eight lanes, step 0: its neighbour, 1: the other
+// pair of the four, 2: the other four (mirrored: which of the four does not matter once steps 0 and
+// 1 have made them equal). Register moves, where a shuffle goes through the LDS.
+template <int STEP, class T>
+__device__ __forceinline__ T group_other(T v) {
+    constexpr int ctrl = STEP == 0 ? 0xB1 : STEP == 1 ? 0x4E : 0x141;  // quad_perm 1,0,3,2; 2,3,0,1; row_half_mirror
+    return __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), ctrl, 0xf, 0xf, true));
+}
+template <class F>
+__device__ __forceinline__ void group_steps(F&& f) {
+    f(std::integral_constant<int, 0>{});
+    f(std::integral_constant<int, 1>{});
+    f(std::integral_constant<int, 2>{});
+}
 __device__ __forceinline__ float group_min8(float v) {
-    for (int k = 1; k < 8; k <<= 1) v = fminf(v, __shfl_xor(v, k));
+    group_steps([&](auto k) { v = fminf(v, group_other<decltype(k)::value>(v)); });
     return v;
 }
 __device__ __forceinline__ float group_max8(float v) {
-    for (int k = 1; k < 8; k <<= 1) v = fmaxf(v, __shfl_xor(v, k));
+    group_steps([&](auto k) { v = fmaxf(v, group_other<decltype(k)::value>(v)); });
     return v;
 }
 __device__ __forceinline__ uint32_t group_or8(uint32_t v) {
-    for (int k = 1; k < 8; k <<= 1) v |= __shfl_xor(v, k);
+    group_steps([&](auto k) { v |= group_other<decltype(k)::value>(v); });
     return v;
 }
 
-__global__ __launch_bounds__(kBlock) void k_collapse(uint32_t level, CollapseState* __restrict__ state,
+__global__ __launch_bounds__(kCollapseBlock) void k_collapse(uint32_t level, CollapseState* __restrict__ state,
                                                      uint32_t* __restrict__ tasks, uint32_t n, int leaf_max, int width,
                                                      const BinNode* __restrict__ bin, const Box* __restrict__ leaf_box,
                                                      const uint32_t* __restrict__ vals, WideNode* __restrict__ nodes,
@@ -654,19 +671,18 @@ __global__ __launch_bounds__(kBlock) void k_collapse(uint32_t level, CollapseSta
                     if (q > a) a = q;  // not a NaN
                 }
                 uint32_t best = sub;
-                for (int k = 1; k < 8; k <<= 1) {
-                    const float oa = __shfl_xor(a, k);
-                    const uint32_t ob = __shfl_xor(best, k);
+                group_steps([&](auto k) {
+                    const float oa = group_other<decltype(k)::value>(a);
+                    const uint32_t ob = group_other<decltype(k)::value>(best);
                     if (oa > a || (oa == a && ob < best)) {
                         a = oa;
                         best = ob;
                     }
-                }
-                const uint32_t r0 = __shfl(c0, lane0 + int(best)), r1 = __shfl(c1, lane0 + int(best));
+                });
+                const uint32_t r1 = __shfl(c1, lane0 + int(best));
                 more = more && a >= 0.0f;
                 if (more) {
-                    if (sub == best) load(r0);
-                    if (sub == ne) load(r1);
+                    if (sub == best || sub == ne) load(sub == best ? c0 : r1);
                     more = ++ne < uint32_t(width);
                 }
             }
@@ -699,14 +715,14 @@ __global__ __launch_bounds__(kBlock) void k_collapse(uint32_t level, CollapseSta
                     }
                 }
             uint32_t be = (mine && slot == 8u ? sub : sub + 8u) | (bs << 8);  // placed children lose every tie
-            for (int k = 1; k < 8; k <<= 1) {
-                const float oc = __shfl_xor(bc, k);
-                const uint32_t oe = __shfl_xor(be, k);
+            group_steps([&](auto k) {
+                const float oc = group_other<decltype(k)::value>(bc);
+                const uint32_t oe = group_other<decltype(k)::value>(be);
                 if (oc < bc || (oc == bc && (oe & 255u) < (be & 255u))) {
                     bc = oc;
                     be = oe;
                 }
-            }
+            });
             if ((be & 255u) < 8u) {
                 if (sub == (be & 255u)) slot = be >> 8;
                 used |= 1u << (be >> 8);
@@ -739,12 +755,14 @@ __global__ __launch_bounds__(kBlock) void k_collapse(uint32_t level, CollapseSta
             s_nint[grp] = live ? __popc(imask) : 0u;
             s_nprim[grp] = live ? n_prims : 0u;
         }
-        for (uint32_t i = threadIdx.x; i < kCollapseNodes * sizeof(WideNode) / 4; i += kBlock) s_node[i] = 0u;
+        for (uint32_t i = threadIdx.x; i < kCollapseNodes * sizeof(WideNode) / 4; i += kCollapseBlock) s_node[i] = 0u;
         __syncthreads();
-        if (threadIdx.x < kCollapseNodes) {
-            const uint32_t a = s_nint[threadIdx.x], b = s_nprim[threadIdx.x];
-            uint32_t sa = a, sb = b;
-            for (uint32_t k = 1; k < kCollapseNodes; k <<= 1) {
+        if (threadIdx.x < 64u) {  // one wave scans two nodes per lane
+            static_assert(kCollapseNodes == 128, "two nodes per lane");
+            const uint32_t i = 2u * threadIdx.x;
+            const uint32_t a0 = s_nint[i], a1 = s_nint[i + 1], b0 = s_nprim[i], b1 = s_nprim[i + 1];
+            uint32_t sa = a0 + a1, sb = b0 + b1;
+            for (uint32_t k = 1; k < 64u; k <<= 1) {
                 const uint32_t xa = __shfl_up(sa, k), xb = __shfl_up(sb, k);
                 if (threadIdx.x >= k) {
                     sa += xa;
@@ -752,11 +770,12 @@ __global__ __launch_bounds__(kBlock) void k_collapse(uint32_t level, CollapseSta
                 }
             }
             unsigned long long at = 0;
-            if (threadIdx.x == kCollapseNodes - 1)
-                at = atomicAdd(&state->alloc, (static_cast<unsigned long long>(sb) << 32) | sa);
-            at = __shfl(at, int(kCollapseNodes - 1));
-            s_nint[threadIdx.x] = uint32_t(at) + sa - a;
-            s_nprim[threadIdx.x] = uint32_t(at >> 32) + sb - b;
+            if (threadIdx.x == 63u) at = atomicAdd(&state->alloc, (static_cast<unsigned long long>(sb) << 32) | sa);
+            at = __shfl(at, 63);
+            s_nint[i] = uint32_t(at) + sa - a0 - a1;
+            s_nint[i + 1] = uint32_t(at) + sa - a1;
+            s_nprim[i] = uint32_t(at >> 32) + sb - b0 - b1;
+            s_nprim[i + 1] = uint32_t(at >> 32) + sb - b1;
         }
         __syncthreads();
         const uint32_t cbase = s_nint[grp], pbase = s_nprim[grp];
@@ -795,12 +814,13 @@ __global__ __launch_bounds__(kBlock) void k_collapse(uint32_t level, CollapseSta
         __syncthreads();
         const uint32_t words = min(kCollapseNodes, end - base) * uint32_t(sizeof(WideNode) / 4);
         uint32_t* dst = reinterpret_cast<uint32_t*>(nodes + base);
-        for (uint32_t i = threadIdx.x; i < words; i += kBlock) dst[i] = s_node[i];
+        for (uint32_t i = threadIdx.x; i < words; i += kCollapseBlock) dst[i] = s_node[i];
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
+    const uint32_t working = max(1u, min(gridDim.x, (end - begin + kCollapseNodes - 1) / kCollapseNodes));
+    if (threadIdx.x == 0 && blockIdx.x < working) {
         __threadfence();
-        if (atomicAdd(&state->done[level], 1u) == gridDim.x - 1)
+        if (atomicAdd(&state->done[level], 1u) == working - 1)
             state->bounds[level + 2] = uint32_t(atomicAdd(&state->alloc, 0ull));
     }
 }
@@ -982,8 +1002,8 @@ hipError_t build_bvh(int mode, const float4* prims_in, uint32_t n, int radius_mo
             }
             for (; level < until; ++level) {
                 const uint64_t most = level < 10 ? std::min<uint64_t>(n, 1ull << (3 * level)) : n;
-                hipLaunchKernelGGL(k_collapse, dim3(std::min<uint32_t>(blocks(most, kCollapseNodes), 4096u)), dim3(kBlock), 0,
-                                   st, level, state, tasks, n, leaf_max, width, bin, tree.box, v0, nodes, slots, sp);
+                hipLaunchKernelGGL(k_collapse, dim3(std::min<uint32_t>(blocks(most, kCollapseNodes), 2048u)), dim3(kCollapseBlock),
+                                   0, st, level, state, tasks, n, leaf_max, width, bin, tree.box, v0, nodes, slots, sp);
             }
             VK_TRY(hipGetLastError());
             VK_TRY(hipMemcpyAsync(&fin, state, sizeof(fin), hipMemcpyDeviceToHost, st));
