@@ -128,7 +128,6 @@ struct vkhrt_shadow_mlp {
 struct vkhrt_blas {
     vkhrt_context* ctx = nullptr;
     float4* normals = nullptr;  // triangle meshes: 3 vertex normals per triangle
-    uint32_t* slot_of = nullptr;  // phantom: leaf slot per original primitive id
     uint32_t mode = 0;
     uint32_t radius_mode = 0;
     float radius = 0.02f;
@@ -960,14 +959,6 @@ int vkhrt_blas_build(vkhrt_context* c, const vkhrt_blas_desc* d, void* stream, v
             goto out;
         }
         root_bounds(root, b->lo, b->hi);
-        if (d->mode == VKHRT_GEOMETRY_PHANTOM_CURVES) {  // for the double-word re-run of final hits
-            e = hipMalloc(&b->slot_of, size_t(d->count) * sizeof(uint32_t));
-            if (e == hipSuccess) e = vk::gen_slot_of(b->bvh.prim_ids, d->count, b->slot_of, st);
-            if (e != hipSuccess) {
-                rc = hip_fail(c, e, "slot map");
-                goto out;
-            }
-        }
     } else {
         for (int k = 0; k < 3; ++k) {
             b->lo[k] = INFINITY;
@@ -1042,7 +1033,7 @@ void vkhrt_blas_destroy(vkhrt_blas* b) {
     hipFree(b->voxels);
     hipFree(b->vbricks);
     hipFree(b->vblocks);
-    hipFree(b->slot_of);
+    hipFree(b->bvh.slot_of);
     delete b;
 }
 
@@ -1069,7 +1060,7 @@ int vkhrt_tlas_build(vkhrt_context* c, const vkhrt_blas* const* blases, uint32_t
         I.blas.radius_mode = b->radius_mode;
         I.blas.radius = b->radius;
         I.blas.normals = b->normals;
-        I.blas.slot_of = b->slot_of;
+        I.blas.slot_of = b->bvh.slot_of;
         I.blas.voxels = b->voxels;
         I.blas.vbricks = b->vbricks;
         I.blas.vblocks = b->vblocks;

@@ -15,6 +15,7 @@ struct BuiltBvh {
     uint32_t* prim_ids = nullptr;
     float4* prims = nullptr;  // primitive records in leaf order
     float* aux = nullptr;     // phantom: early-out cylinder radius per leaf slot
+    uint32_t* slot_of = nullptr;  // phantom: leaf slot per original primitive id (the re-run of final hits)
     uint32_t depth = 0;       // wide levels
 };
 
