@@ -1,0 +1,122 @@
+"""BLAS builds at the edges of their kernels, through the C-ABI: record counts around a wave's and a
+tile's share of the sort (4 and 16 keys per thread) and the aligned runs of the boxes, equal sort
+keys, and blocks that one build leaves to the next (sizes growing and shrinking, two threads, a BLAS
+that outlives its context)."""
+import threading
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def G():
+    import gpu_util
+    return gpu_util
+
+
+def capsules(n, seed, same=False):
+    """n short LSS records scattered in a box, or all at one place but for their length."""
+    rng = np.random.default_rng(seed)
+    a = np.zeros((n, 8), np.float32)
+    a[:, :3] = rng.uniform(-50.0, 50.0, (1 if same else n, 3))
+    a[:, 4:7] = a[:, :3] + (np.array([1.0, 0.5, 0.25], np.float32) if same else rng.uniform(-1.0, 1.0, (n, 3)))
+    a[:, 3] = a[:, 7] = rng.uniform(0.02, 0.1, n)
+    return a
+
+
+def rays_at(caps, idx, seed):
+    """Rays into the middle of the capsules `idx` from 0.3 units away."""
+    rng = np.random.default_rng(seed)
+    d = rng.standard_normal((len(idx), 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    r = np.zeros((len(idx), 8), np.float32)
+    r[:, :3] = 0.5 * (caps[idx, :3] + caps[idx, 4:7]) - 0.3 * d
+    r[:, 3] = 0.0
+    r[:, 4:7] = d
+    r[:, 7] = 1000.0
+    return r
+
+
+def check(ctx, G, oracle, caps, blas, label):
+    import vkhrt_amd as V
+    n = len(caps)
+    idx = np.unique(np.concatenate([np.arange(min(n, 300)), np.arange(max(0, n - 300), n),
+                                    np.linspace(0, n - 1, 400).astype(int)]))
+    rays = rays_at(caps, idx, 5)
+    tlas = V.TopLevelAccelerationStructure(ctx, [blas])
+    S = oracle.Scene()
+    S.add(oracle.MODE_LSS, caps)
+    ref = S.trace(rays)
+    assert (ref["prim"] != 0xFFFFFFFF).mean() > 0.9
+    G.compare_hits(G.trace(ctx, tlas, rays), ref, label)
+    assert blas.info()["leaf_records"] == n
+    tlas.close()
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 9, 63, 64, 65, 127, 128, 129, 1023, 1025, 4097, 16383, 520193, 520192, 524289])
+def test_counts(gpu_ctx, G, oracle, n):
+    import vkhrt_amd as V
+    caps = capsules(n, n)
+    blas = G.build_blas(gpu_ctx, V.GEOMETRY_LSS, caps)
+    check(gpu_ctx, G, oracle, caps, blas, f"{n} records")
+    blas.close()
+
+
+@pytest.mark.parametrize("leaf", [1, 3])
+def test_equal_keys(gpu_ctx, G, oracle, leaf):
+    """Records with one sort key: the tree splits them by index."""
+    import vkhrt_amd as V
+    caps = capsules(3000, 7, same=True)
+    blas = G.build_blas(gpu_ctx, V.GEOMETRY_LSS, caps, leaf_size=leaf)
+    check(gpu_ctx, G, oracle, caps, blas, f"equal keys, leaves of {leaf}")
+    blas.close()
+
+
+def test_blocks_pass_from_build_to_build(G, oracle):
+    import vkhrt_amd as V
+    ctx = V.Context(0)
+    keep = []
+    for k, n in enumerate([5000, 5200, 70000, 300, 5100, 66000, 5000]):
+        caps = capsules(n, 100 + k)
+        blas = G.build_blas(ctx, V.GEOMETRY_LSS, caps)
+        keep.append((caps, blas))
+        if len(keep) == 3:  # two builds old: its memory goes to later ones
+            keep.pop(0)[1].close()
+        for c, b in keep:
+            check(ctx, G, oracle, c, b, f"build {k}")
+    ctx.close()
+    for _, b in keep:
+        b.close()
+
+
+def test_builds_in_two_threads(G, oracle):
+    import torch
+    import vkhrt_amd as V
+    ctx = V.Context(0)
+    sets = [[capsules(4000 + 500 * i, 10 * t + i) for i in range(4)] for t in range(2)]
+    dev = [[G.dev(c) for c in s] for s in sets]
+    streams = [torch.cuda.Stream() for _ in sets]
+    torch.cuda.synchronize()
+    built = [[], []]
+
+    def work(t):
+        for c, d in zip(sets[t], dev[t]):
+            old = V.BottomLevelAccelerationStructure(ctx, V.GEOMETRY_LSS, d.data_ptr(), c.shape[0],
+                                                     stream=streams[t].cuda_stream)
+            old.close()
+            built[t].append(V.BottomLevelAccelerationStructure(ctx, V.GEOMETRY_LSS, d.data_ptr(), c.shape[0],
+                                                               stream=streams[t].cuda_stream))
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for t in range(2):
+        assert len(built[t]) == 4
+        for c, b in zip(sets[t], built[t]):
+            check(ctx, G, oracle, c, b, f"thread {t}")
+            b.close()
+    ctx.close()

@@ -8,6 +8,7 @@
 #include <cstring>
 #include <atomic>
 #include <map>
+#include <memory>
 #include <numeric>
 #include <new>
 #include <string>
@@ -34,6 +35,7 @@ struct vkhrt_context {
     int device = 0;
     hipStream_t stream = nullptr;
     std::string err;
+    std::shared_ptr<vk::MemPool> pool;  // memory of BLAS builds
     int stack_kind = 1;
     int leaf_size = 1;
     int bvh_width = 8;
@@ -135,6 +137,7 @@ struct vkhrt_blas {
     bool has_xf = false;
     float xf[12];
     vk::BuiltBvh bvh;
+    std::shared_ptr<vk::MemPool> pool;  // where bvh's memory goes back to
     uint32_t records = 0;
     float lo[3], hi[3];  // object-space bounds
     vkhrt_blas_info info{};
@@ -529,6 +532,12 @@ int vkhrt_context_create(int device, vkhrt_context** out) {
     vkhrt_context* c = new (std::nothrow) vkhrt_context();
     if (!c) return VKHRT_ERROR_OUT_OF_MEMORY;
     c->device = device;
+    try {
+        c->pool = std::make_shared<vk::MemPool>(device);
+    } catch (const std::bad_alloc&) {
+        delete c;
+        return VKHRT_ERROR_OUT_OF_MEMORY;
+    }
     hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipMalloc(&c->status, 16);
     if (e == hipSuccess) e = hipMalloc(&c->counters, vk::kRenderCounterWords * sizeof(uint32_t));
@@ -556,6 +565,7 @@ void vkhrt_context_destroy(vkhrt_context* c) {
         hipEventDestroy(p.a);
         hipEventDestroy(p.b);
     }
+    if (c->pool) c->pool->close();
     hipFree(c->status);
     hipFree(c->work_counts);
     hipFree(c->counters);
@@ -887,6 +897,7 @@ int vkhrt_blas_build(vkhrt_context* c, const vkhrt_blas_desc* d, void* stream, v
     vkhrt_blas* b = new (std::nothrow) vkhrt_blas();
     if (!b) return fail(c, VKHRT_ERROR_OUT_OF_MEMORY, "blas");
     b->ctx = c;
+    b->pool = c->pool;
     b->mode = d->mode;
     b->radius_mode = per_point ? 1u : 0u;
     b->radius = d->radius;
@@ -944,21 +955,14 @@ int vkhrt_blas_build(vkhrt_context* c, const vkhrt_blas_desc* d, void* stream, v
         {
             Timer tm(c, st, "blas_build");
             e = vk::build_bvh(int(d->mode), records, d->count, int(b->radius_mode), d->radius,
-                              d->leaf_size ? int(d->leaf_size) : c->leaf_size, c->bvh_width, c->bvh_collapse, st,
-                              &b->bvh, err);
+                              d->leaf_size ? int(d->leaf_size) : c->leaf_size, c->bvh_width, c->bvh_collapse,
+                              *c->pool, st, &b->bvh, err);
         }
         if (e != hipSuccess) {
             rc = fail(c, e == hipErrorOutOfMemory ? VKHRT_ERROR_OUT_OF_MEMORY : VKHRT_ERROR_DEVICE, "bvh build: " + err);
             goto out;
         }
-        vk::WideNode root;
-        e = hipMemcpyAsync(&root, b->bvh.nodes, sizeof(root), hipMemcpyDeviceToHost, st);
-        if (e == hipSuccess) e = hipStreamSynchronize(st);
-        if (e != hipSuccess) {
-            rc = hip_fail(c, e, "root readback");
-            goto out;
-        }
-        root_bounds(root, b->lo, b->hi);
+        root_bounds(b->bvh.root, b->lo, b->hi);
     } else {
         for (int k = 0; k < 3; ++k) {
             b->lo[k] = INFINITY;
@@ -1025,15 +1029,12 @@ int vkhrt_blas_info_get(const vkhrt_blas* b, vkhrt_blas_info* out) {
 
 void vkhrt_blas_destroy(vkhrt_blas* b) {
     if (!b) return;
-    hipFree(b->bvh.nodes);
-    hipFree(b->bvh.prim_ids);
-    hipFree(b->bvh.prims);
-    hipFree(b->bvh.aux);
+    for (const vk::MemPool::Block& m : b->bvh.mem)
+        if (m.p) b->pool->release(m, false);
     hipFree(b->normals);
     hipFree(b->voxels);
     hipFree(b->vbricks);
     hipFree(b->vblocks);
-    hipFree(b->bvh.slot_of);
     delete b;
 }
 

@@ -6,6 +6,7 @@
 #include <string>
 
 #include "internal.hpp"
+#include "mem_pool.hpp"
 
 namespace vk {
 
@@ -17,13 +18,15 @@ struct BuiltBvh {
     float* aux = nullptr;     // phantom: early-out cylinder radius per leaf slot
     uint32_t* slot_of = nullptr;  // phantom: leaf slot per original primitive id (the re-run of final hits)
     uint32_t depth = 0;       // wide levels
+    WideNode root{};          // host copy of nodes[0]
+    MemPool::Block mem[2];    // the blocks that hold the arrays, for MemPool::release
 };
 
-// Builds the 8-wide BVH over `n` primitive records (device pointer) on stream `st`.
-// `width` (2..8) caps the children per wide node. `collapse` 0: greedy largest-area opening;
-// c >= 1: SAH-optimal collapse with node cost 1 and primitive cost c / 4.
+// Builds the 8-wide BVH over `n` primitive records (device pointer) on stream `st`, in memory of
+// `pool`. `width` (2..8) caps the children per wide node. `collapse` 0: greedy largest-area opening;
+// c >= 1: SAH-optimal collapse with node cost 1 and primitive cost c / 4. Returns with the stream idle.
 hipError_t build_bvh(int mode, const float4* prims_in, uint32_t n, int radius_mode, float radius, int leaf_max,
-                     int width, int collapse, hipStream_t st, BuiltBvh* out, std::string& err);
+                     int width, int collapse, MemPool& pool, hipStream_t st, BuiltBvh* out, std::string& err);
 
 struct TraceParams {
     const InstanceDev* inst;

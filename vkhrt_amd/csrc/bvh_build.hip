@@ -1,7 +1,7 @@
 // GPU builder for the bottom-level structure (replaces the driver-internal build behind
 // vkCmdBuildAccelerationStructuresKHR, bottom_level_acceleration_structure.cpp:34-78).
 //
-// Pipeline (all on one stream, temporaries freed at the end):
+// Pipeline (all on one stream, in one scratch block):
 //   1. primitive boxes (GenerateAABBs semantics, geometry_processor.cpp:422-436, plus a
 //      small conservative pad) and centroid bounds (wave reduction + ordered-int atomics)
 //   2. 63-bit Morton codes of box centroids
@@ -904,10 +904,17 @@ __global__ void k_collapse_init(CollapseState* state, uint32_t* tasks, uint32_t 
     }
 }
 
-template <class T>
-hipError_t dalloc(T** p, size_t count) {
-    return hipMalloc(reinterpret_cast<void**>(p), std::max<size_t>(1, count) * sizeof(T));
-}
+// Hands out 256-byte aligned parts of one block; with a null base it only adds up their sizes.
+struct Carver {
+    char* base;
+    size_t at = 0;
+    template <class T>
+    void part(T** p, size_t count) {
+        at = (at + 255) & ~size_t(255);
+        *p = base ? reinterpret_cast<T*>(base + at) : nullptr;
+        at += std::max<size_t>(1, count) * sizeof(T);
+    }
+};
 
 inline uint32_t blocks(uint64_t n, int b = kBlock) { return uint32_t((n + b - 1) / b); }
 
@@ -923,67 +930,83 @@ inline uint32_t blocks(uint64_t n, int b = kBlock) { return uint32_t((n + b - 1)
     } while (0)
 
 hipError_t build_bvh(int mode, const float4* prims_in, uint32_t n, int radius_mode, float radius, int leaf_max,
-                     int width, int collapse, hipStream_t st, BuiltBvh* out, std::string& err) {
+                     int width, int collapse, MemPool& pool, hipStream_t st, BuiltBvh* out, std::string& err) {
     const int rec = mode == kLss ? 2 : mode == kTriangles ? 3 : 4;
     float4* box = nullptr;
-    uint32_t* cb = nullptr;
+    uint32_t *cb = nullptr, *v0 = nullptr, *v1 = nullptr, *hist = nullptr, *totals = nullptr, *tasks = nullptr, *done = nullptr;
     uint64_t *k0 = nullptr, *k1 = nullptr;
-    uint32_t *v0 = nullptr, *v1 = nullptr, *hist = nullptr, *totals = nullptr;
     BoxTree tree{};
     BinNode* bin = nullptr;
-    uint32_t *tasks = nullptr, *done = nullptr;
-    CollapseState* state = nullptr;
     SahParams sp{};
+    struct Head {  // read back together: the collapse's state and the root node
+        CollapseState state;
+        alignas(16) WideNode root;
+    };
+    Head* head = nullptr;
     WideNode* nodes = nullptr;
-    uint32_t* slots = nullptr;
-    float4* prims_sorted = nullptr;
-    float* aux = nullptr;
-    uint32_t* slot_of = nullptr;
+    MemPool::Block scratch, records, node_block;
+    BuiltBvh built;
+    Head fin{};
     hipError_t rc = hipSuccess;
     uint32_t tiles = 0;
     bool small = false;
-    CollapseState fin{};
     size_t boxes = 0;
-    uint32_t cb_host[6];
     *out = BuiltBvh{};
     if (n == 0) return hipSuccess;
     if (leaf_max < 1) leaf_max = 1;
     if (leaf_max > 3) leaf_max = 3;
     if (width < 2) width = 2;
     if (width > 8) width = 8;
-
-    VK_TRY(dalloc(&box, size_t(n) * 2));
-    VK_TRY(dalloc(&cb, 6));
-    VK_TRY(dalloc(&k0, n));
-    VK_TRY(dalloc(&k1, n));
-    VK_TRY(dalloc(&v0, n));
-    VK_TRY(dalloc(&v1, n));
     // tiles of 16 keys per thread; of 4 where those would leave more than half of the 256 CUs idle (16k keys:
     // a scatter of 4 tiles took 15 us, of 16 tiles 6)
     small = blocks(n, kBlock * 16) < 128u;
     tiles = blocks(n, kBlock * (small ? 4 : 16));
-    VK_TRY(dalloc(&hist, size_t(tiles) * kRsDigits));
-    VK_TRY(dalloc(&totals, kRsDigits));
     for (int k = 0; k < kBoxLevels; ++k) {
         tree.off[k] = boxes;
         boxes += n >> k;
     }
-    VK_TRY(dalloc(&tree.box, boxes));
-    VK_TRY(dalloc(&bin, n));
-    VK_TRY(dalloc(&tasks, n));
-    VK_TRY(dalloc(&state, 1));
-    VK_TRY(dalloc(&nodes, n));
-    VK_TRY(dalloc(&slots, n));
-    VK_TRY(dalloc(&prims_sorted, size_t(n) * rec));
-    if (mode == kPhantom) VK_TRY(dalloc(&aux, n));
-    if (mode == kPhantom) VK_TRY(dalloc(&slot_of, n));
-    if (collapse > 0 && n >= 2) {
-        VK_TRY(dalloc(&sp.cost, n));
-        VK_TRY(dalloc(&done, n));
-        sp.leaf_max = leaf_max;
-        sp.width = width;
-        sp.c_node = 1.0f;
-        sp.c_prim = 0.25f * float(collapse);
+
+    // One scratch block. The wide nodes (at most n) take the place of the primitive boxes and of the
+    // keys' first buffer, which are done with when the collapse starts.
+    for (int pass = 0; pass < 2; ++pass) {
+        Carver c{static_cast<char*>(scratch.p)};
+        c.part(&head, 1);
+        c.at = offsetof(Head, root);  // head comes first in the block; the nodes follow its state, from `root` on
+        nodes = scratch.p ? &head->root : nullptr;
+        {
+            Carver early{c.base, c.at};
+            early.part(&box, size_t(n) * 2);
+            early.part(&k0, n);
+            early.part(&v0, n);
+            c.at = std::max(early.at, c.at + size_t(n) * sizeof(WideNode));
+        }
+        c.part(&k1, n);
+        c.part(&v1, n);
+        c.part(&cb, 6);
+        c.part(&hist, size_t(tiles) * kRsDigits);
+        c.part(&totals, kRsDigits);
+        c.part(&tree.box, boxes);
+        c.part(&bin, n);
+        c.part(&tasks, n);
+        if (collapse > 0 && n >= 2) {
+            c.part(&sp.cost, n);
+            c.part(&done, n);
+        }
+        if (pass == 0) VK_TRY(pool.acquire(c.at, &scratch));
+    }
+    sp.leaf_max = leaf_max;
+    sp.width = width;
+    sp.c_node = 1.0f;
+    sp.c_prim = 0.25f * float(collapse);
+    for (int pass = 0; pass < 2; ++pass) {
+        Carver c{static_cast<char*>(records.p)};
+        c.part(&built.prims, size_t(n) * rec);
+        c.part(&built.prim_ids, n);
+        if (mode == kPhantom) {
+            c.part(&built.aux, n);
+            c.part(&built.slot_of, n);
+        }
+        if (pass == 0) VK_TRY(pool.acquire(c.at, &records));
     }
 
     hipLaunchKernelGGL(k_init_bounds, dim3(1), dim3(64), 0, st, cb);
@@ -991,6 +1014,7 @@ hipError_t build_bvh(int mode, const float4* prims_in, uint32_t n, int radius_mo
                        radius_mode, radius, box, cb);
     hipLaunchKernelGGL(k_morton, dim3(blocks(n)), dim3(kBlock), 0, st, box, n, cb, k0, v0);
     VK_TRY(hipGetLastError());
+    static_assert(kRsPasses % 2 == 1, "the sorted keys end in the second buffer");
     for (int pass = 0; pass < kRsPasses; ++pass) {
         const int shift = pass * kRsBits;
         if (small)
@@ -1030,13 +1054,13 @@ hipError_t build_bvh(int mode, const float4* prims_in, uint32_t n, int radius_mo
             VK_TRY(hipStreamSynchronize(st));
         }
     }
-    hipLaunchKernelGGL(k_collapse_init, dim3(1), dim3(64), 0, st, state, tasks, n >= 2 ? 0u : kLeafFlag);
+    hipLaunchKernelGGL(k_collapse_init, dim3(1), dim3(64), 0, st, &head->state, tasks, n >= 2 ? 0u : kLeafFlag);
     {
         // as many levels as an evenly filled tree of this size has and three more, then four at a time; level L has
         // at most 8^L nodes
-        uint32_t level = 0, until = 3, depth = 0;
+        uint32_t level = 0, until = 3;
         for (uint64_t m = 1; m < n; m *= 8) ++until;
-        while (depth == 0) {
+        while (built.depth == 0) {
             if (until > kMaxWideLevels) {
                 err = "BVH collapse did not reach the leaves";
                 rc = hipErrorUnknown;
@@ -1045,70 +1069,50 @@ hipError_t build_bvh(int mode, const float4* prims_in, uint32_t n, int radius_mo
             for (; level < until; ++level) {
                 const uint64_t most = level < 10 ? std::min<uint64_t>(n, 1ull << (3 * level)) : n;
                 hipLaunchKernelGGL(k_collapse, dim3(std::min<uint32_t>(blocks(most, kCollapseNodes), 2048u)), dim3(kCollapseBlock),
-                                   0, st, level, state, tasks, n, leaf_max, width, bin, tree.box, v0, nodes, slots, sp);
+                                   0, st, level, &head->state, tasks, n, leaf_max, width, bin, tree.box, v0, nodes,
+                                   built.prim_ids, sp);
             }
             VK_TRY(hipGetLastError());
-            VK_TRY(hipMemcpyAsync(&fin, state, sizeof(fin), hipMemcpyDeviceToHost, st));
+            VK_TRY(hipMemcpyAsync(&fin, head, sizeof(fin), hipMemcpyDeviceToHost, st));
             VK_TRY(hipStreamSynchronize(st));
-            for (uint32_t l = 1; l <= level && !depth; ++l)
-                if (fin.bounds[l + 1] == fin.bounds[l]) depth = l;
+            for (uint32_t l = 1; l <= level && !built.depth; ++l)
+                if (fin.state.bounds[l + 1] == fin.state.bounds[l]) built.depth = l;
             until = level + 4;
         }
-        out->depth = depth;
     }
-    VK_TRY(hipMemcpyAsync(cb_host, cb, 24, hipMemcpyDeviceToHost, st));
-    if (mode == kPhantom)
-        hipLaunchKernelGGL(k_leaf_curves, dim3(blocks(uint64_t(n) * 4)), dim3(kBlock), 0, st, prims_in, slots, n, radius_mode,
-                           radius, prims_sorted, aux, slot_of);
-    else
-        hipLaunchKernelGGL(k_gather, dim3(blocks(uint64_t(n) * rec)), dim3(kBlock), 0, st, prims_in, slots, n, rec,
-                           prims_sorted);
-    VK_TRY(hipGetLastError());
-    VK_TRY(hipStreamSynchronize(st));
-    if (uint32_t(fin.alloc >> 32) != n || uint32_t(fin.alloc) > n) {
-        err = "BVH collapse placed " + std::to_string(uint32_t(fin.alloc >> 32)) + " of " + std::to_string(n) + " primitives";
+    built.nnodes = uint32_t(fin.state.alloc);
+    built.root = fin.root;
+    if (uint32_t(fin.state.alloc >> 32) != n || built.nnodes > n) {
+        err = "BVH collapse placed " + std::to_string(uint32_t(fin.state.alloc >> 32)) + " of " + std::to_string(n) +
+              " primitives";
         rc = hipErrorUnknown;
         goto fail;
     }
     {
-        uint32_t depth = out->depth;
-        *out = BuiltBvh{};
-        out->depth = depth;
+        // a sixteenth more, so that the next frame of a moving groom fits the block too
+        const size_t bytes = size_t(built.nnodes) * sizeof(WideNode);
+        VK_TRY(pool.acquire(bytes + bytes / 16, &node_block));
+        built.nodes = static_cast<WideNode*>(node_block.p);
+        VK_TRY(hipMemcpyAsync(built.nodes, nodes, bytes, hipMemcpyDeviceToDevice, st));
     }
-    out->nodes = nodes;
-    out->nnodes = uint32_t(fin.alloc);
-    out->prim_ids = slots;
-    out->prims = prims_sorted;
-    out->aux = aux;
-    out->slot_of = slot_of;
-    aux = nullptr;
-    slot_of = nullptr;
-    nodes = nullptr;
-    slots = nullptr;
-    prims_sorted = nullptr;
-    goto done;
+    if (mode == kPhantom)
+        hipLaunchKernelGGL(k_leaf_curves, dim3(blocks(uint64_t(n) * 4)), dim3(kBlock), 0, st, prims_in, built.prim_ids, n,
+                           radius_mode, radius, built.prims, built.aux, built.slot_of);
+    else
+        hipLaunchKernelGGL(k_gather, dim3(blocks(uint64_t(n) * rec)), dim3(kBlock), 0, st, prims_in, built.prim_ids, n, rec,
+                           built.prims);
+    VK_TRY(hipGetLastError());
+    VK_TRY(hipStreamSynchronize(st));
+    pool.release(scratch, true);
+    built.mem[0] = records;
+    built.mem[1] = node_block;
+    *out = built;
+    return hipSuccess;
 fail:
     if (rc == hipSuccess) rc = hipErrorUnknown;
-done:
-    hipFree(box);
-    hipFree(cb);
-    hipFree(k0);
-    hipFree(k1);
-    hipFree(v0);
-    hipFree(v1);
-    hipFree(hist);
-    hipFree(totals);
-    hipFree(tree.box);
-    hipFree(bin);
-    hipFree(tasks);
-    hipFree(done);
-    hipFree(state);
-    hipFree(nodes);
-    hipFree(slots);
-    hipFree(prims_sorted);
-    hipFree(aux);
-    hipFree(slot_of);
-    hipFree(sp.cost);
+    pool.release(scratch, false);
+    pool.release(records, false);
+    pool.release(node_block, false);
     return rc;
 }
 
