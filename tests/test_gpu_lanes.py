@@ -100,3 +100,27 @@ def test_negative_tmin(gpu_ctx, G, oracle, curves, mode):
     if mode != "phantom":  # a phantom hit lies in front of the origin
         assert (ref["t"][ref["prim"] != 0xFFFFFFFF] < 0).sum() > 100
     G.compare_hits(G.trace(gpu_ctx, tlas, rays), ref, f"{mode}, negative tmin")
+
+
+@pytest.mark.parametrize("count", [65535, 65536, 65537])
+def test_shared_out_and_claimed_rays_agree(gpu_ctx, G, curves, count):
+    """As many rays as a grid of one block per CU has lanes, one fewer and one more: shared out
+    evenly up to there, claimed from counters beyond; the default grid shares out all three."""
+    import scenes
+    import torch
+    import vkhrt_amd as V
+    tlas = V.TopLevelAccelerationStructure(gpu_ctx, [G.build_blas(gpu_ctx, V.GEOMETRY_PHANTOM_CURVES, curves, per_point=True)])
+    assert torch.cuda.get_device_properties(0).multi_processor_count == 256
+    rays = scenes.targeted_rays(curves, count, seed=37, dist=(1.0, 60.0))
+    for flags in (V.TRACE_FP64_POLISH, V.TRACE_TERMINATE_ON_FIRST_HIT):
+        ref = G.trace(gpu_ctx, tlas, rays, flags=flags)
+        gpu_ctx.set_option(V.OPTION_BLOCKS_PER_CU, 1)
+        try:
+            got = G.trace(gpu_ctx, tlas, rays, flags=flags)
+        finally:
+            gpu_ctx.set_option(V.OPTION_BLOCKS_PER_CU, 0)
+        if flags == V.TRACE_FP64_POLISH:
+            assert got.tobytes() == ref.tobytes()
+        else:
+            assert np.array_equal(got["prim"] == 0xFFFFFFFF, ref["prim"] == 0xFFFFFFFF)
+    tlas.close()

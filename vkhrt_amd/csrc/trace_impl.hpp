@@ -923,11 +923,28 @@ struct WorkClaim {
     uint32_t total, shift;
     uint32_t cx, left;  // counter in use; XCD counters not yet found dry
     bool exhausted;     // no item left anywhere
+    bool shared;        // the items are shared out evenly instead
+    uint32_t next, end;  // this wave's share
 
     __device__ __forceinline__ WorkClaim(uint32_t* c, uint32_t* x, uint32_t chunk, uint32_t n, uint32_t* d)
         : counter(c), xcd(chunk ? x : nullptr), dry(d), total(n), shift(chunk ? uint32_t(__ffs(chunk) - 1) : 0u),
           cx(__builtin_amdgcn_s_getreg((3 << 11) | 20) & 7u),  // hwreg(HW_REG_XCC_ID, 0, 4)
-          left(8u), exhausted(false) {}
+          left(8u), exhausted(false), shared(fits_lanes(n, gridDim.x)), next(0u), end(0u) {
+        if (!shared) return;
+        const uint32_t waves = gridDim.x * (kTraceBlock / 64), per = (n + waves - 1) / waves;
+        // blocks go round the XCDs: each XCD's blocks get neighbouring shares
+        const uint32_t row = gridDim.x / 8u;
+        const uint32_t b = blockIdx.x < row * 8u ? (blockIdx.x & 7u) * row + (blockIdx.x >> 3) : blockIdx.x;
+        const uint64_t w = b * (kTraceBlock / 64) + (threadIdx.x >> 6);
+        next = uint32_t(min(w * per, uint64_t(n)));
+        end = min(next + per, n);
+    }
+
+    // Whether a launch of `blocks` blocks needs no counters for `n` items (also asked by the host,
+    // which then clears none).
+    static __host__ __device__ __forceinline__ bool fits_lanes(uint32_t n, uint32_t blocks) {
+        return n <= uint64_t(blocks) * kTraceBlock;
+    }
 
     // The idle lanes of the wave (mask `idle`, the same in every lane) claim one item each;
     // returns the calling lane's item for `rank` = its rank among the idle lanes, or a value
@@ -937,6 +954,10 @@ struct WorkClaim {
         const uint32_t leader = __ffsll((unsigned long long)idle) - 1;
         const uint32_t lane = threadIdx.x & 63u;
         uint32_t base = 0;
+        if (shared) {
+            exhausted = true;
+            return next + rank < end ? next + rank : 0xFFFFFFFFu;
+        }
         if (!xcd) {
             if (lane == leader) base = atomicAdd(counter, n);
             base = __shfl(base, int(leader));
@@ -2580,29 +2601,27 @@ hipError_t launch_trace_pass(const TraceParams& tp, const float* rays, uint32_t 
     uint2* stats = nullptr;
     if constexpr (G::kCompact) {
         if (tp.work) {
-            hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, st, tp.work, 1u);
-            if (tp.xcd_chunk && tp.xcd_work)
-                hipLaunchKernelGGL(k_zero, dim3(8 * kXcdStride / 64), dim3(64), 0, st, tp.xcd_work, 8u * kXcdStride);
+            auto launch = [&](auto kernel) {
+                const dim3 lanes = persistent_grid(kernel, tp.blocks_per_cu);
+                if (!WorkClaim::fits_lanes(n, lanes.x)) {
+                    hipLaunchKernelGGL(k_zero, dim3(1), dim3(64), 0, st, tp.work, 1u);
+                    if (tp.xcd_chunk && tp.xcd_work)
+                        hipLaunchKernelGGL(k_zero, dim3(8 * kXcdStride / 64), dim3(64), 0, st, tp.xcd_work, 8u * kXcdStride);
+                }
+                hipLaunchKernelGGL(kernel, lanes, block, 0, st, tp, rays, n, hits, tp.work);
+            };
             // one-instance TLASes take kernels that read the BLAS fields once
             // (a TLAS of several modes has several instances)
             const bool one = !G::kMixed && instance_mode(tp.ninst) == kInstOne;
             constexpr int kOne = G::kMixed ? kInstMany : kInstOne;
             if (any && one)
-                hipLaunchKernelGGL((k_trace_rays_persistent<G, true, STACK, kOne>),
-                                   persistent_grid(k_trace_rays_persistent<G, true, STACK, kOne>, tp.blocks_per_cu), block, 0,
-                                   st, tp, rays, n, hits, tp.work);
+                launch(k_trace_rays_persistent<G, true, STACK, kOne>);
             else if (any)
-                hipLaunchKernelGGL((k_trace_rays_persistent<G, true, STACK, kInstMany>),
-                                   persistent_grid(k_trace_rays_persistent<G, true, STACK, kInstMany>, tp.blocks_per_cu), block, 0,
-                                   st, tp, rays, n, hits, tp.work);
+                launch(k_trace_rays_persistent<G, true, STACK, kInstMany>);
             else if (one)
-                hipLaunchKernelGGL((k_trace_rays_persistent<G, false, STACK, kOne>),
-                                   persistent_grid(k_trace_rays_persistent<G, false, STACK, kOne>, tp.blocks_per_cu), block,
-                                   0, st, tp, rays, n, hits, tp.work);
+                launch(k_trace_rays_persistent<G, false, STACK, kOne>);
             else
-                hipLaunchKernelGGL((k_trace_rays_persistent<G, false, STACK, kInstMany>),
-                                   persistent_grid(k_trace_rays_persistent<G, false, STACK, kInstMany>, tp.blocks_per_cu), block,
-                                   0, st, tp, rays, n, hits, tp.work);
+                launch(k_trace_rays_persistent<G, false, STACK, kInstMany>);
             return hipGetLastError();
         }
     }
