@@ -284,7 +284,10 @@ __device__ __forceinline__ bool prhi(const RayFrame& F, const float4* cv, float 
 // FP64 evaluation from the start, without the early-out test, for a ray / curve pair the FP32
 // pass already chose. On convergence with s > 0 it returns t, u and the unit normal (ray-
 // centric vector rotated back), rounded once, in `out` (marked polished: the normal is final).
-__device__ __forceinline__ bool prhi_ff(f3 of, f3 df, const float4* cv, int radius_mode, float const_r,
+// PAIR: the call runs one side of the iteration, 0 the one Prhi starts from, 1 the other, whose
+// result counts when side 0 has none; else both, one after the other.
+template <bool PAIR>
+__device__ __forceinline__ bool prhi_ff(f3 of, f3 df, const float4* cv, int radius_mode, float const_r, int only,
                                         PhantomHit& out) {
     const ff3 o = dw::toff(of), d = dw::toff(df);
     ff3 e1, e2, e3 = nrm3(d);
@@ -302,7 +305,8 @@ __device__ __forceinline__ bool prhi_ff(f3 of, f3 df, const float4* cv, int radi
     const ff3 cd = nrm3(sub(q[3], q[0]));
     const ff dz = cd.x * ff(0) + cd.y * ff(0) + cd.z * ff(1);
     ff tStart = dz > ff(0) ? ff(0) : ff(1);
-    for (int side = 0; side < 2; ++side) {
+    if (PAIR && only) tStart = ff(1) - tStart;
+    for (int side = 0; side < (PAIR ? 1 : 2); ++side) {
         ff t = tStart, told = ff(0), dt1 = ff(0), dt2 = ff(0), s_rel = ff(0), cx = ff(0), cy = ff(0), cz = ff(0),
            last = ff(0);
         const int st = prhi_iterate(q[0], q[1], q[2], q[3], rr, radius_mode, ff(const_r), t, told, dt1, dt2, 0, 8, s_rel,

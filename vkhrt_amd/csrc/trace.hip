@@ -355,8 +355,13 @@ hipError_t launch_shadow_rays(const float* rays, const HitRec* hits, uint32_t n,
 hipError_t launch_accurate_hits(const TraceParams& tp, const float* rays, uint32_t n, HitRec* hits, hipStream_t st) {
     using namespace trace_detail;
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_accurate_hits<SrcRays>, dim3((n + kTraceBlock - 1) / kTraceBlock), dim3(kTraceBlock), 0, st, tp,
-                       SrcRays{reinterpret_cast<const float4*>(rays)}, hits, n);
+    const SrcRays src{reinterpret_cast<const float4*>(rays)};
+    if (n <= kAccuratePairs)
+        hipLaunchKernelGGL(k_accurate_pairs<SrcRays>, dim3((2 * n + kTraceBlock - 1) / kTraceBlock), dim3(kTraceBlock), 0, st,
+                           tp, src, hits, n);
+    else
+        hipLaunchKernelGGL(k_accurate_hits<SrcRays>, dim3((n + kTraceBlock - 1) / kTraceBlock), dim3(kTraceBlock), 0, st, tp,
+                           src, hits, n);
     return hipGetLastError();
 }
 

@@ -1640,7 +1640,8 @@ struct SrcCamera {
 // Double-word re-run of each final phantom hit (VKHRT_*_ACCURATE_NORMALS): the ray from `src`,
 // in the instance's object space, against the hit's curve record; t, u and the normal are
 // replaced when the re-run converges. Misses, other modes and FP64-polished roots are kept.
-template <class Src>
+// PAIR: lanes 2k and 2k + 1 call it for the same ray and run one side each.
+template <bool PAIR = false, class Src>
 __device__ __forceinline__ bool accurate_refine(const TraceParams& tp, const Src& src, uint32_t i, HitRec& h) {
     if (h.prim_id == 0xFFFFFFFFu || h.v != 0.0f || h.inst_id >= tp.ninst) return false;
     const InstanceDev& I = tp.inst[h.inst_id];
@@ -1655,7 +1656,9 @@ __device__ __forceinline__ bool accurate_refine(const TraceParams& tp, const Src
     const uint32_t slot = I.blas.slot_of[h.prim_id];
     if (slot >= I.blas.nprims) return false;
     PhantomHit ph;
-    if (!prhi_ff(o, d, I.blas.prims + size_t(slot) * 4, int(I.blas.radius_mode), I.blas.radius, ph)) return false;
+    if (!prhi_ff<PAIR>(o, d, I.blas.prims + size_t(slot) * 4, int(I.blas.radius_mode), I.blas.radius,
+                       int(threadIdx.x & 1u), ph))
+        return false;
     f3 nn{ph.ncx, ph.ncy, ph.nsz};
     if (!I.identity) {
         const float* x = I.xf;
@@ -1681,6 +1684,26 @@ __global__ __launch_bounds__(kTraceBlock) void k_accurate_hits(TraceParams tp, S
                                                                uint32_t n) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) accurate_one(tp, src, i, hits);
+}
+// The same with two lanes per ray, for so few rays that the longest re-run is the time: in nearly
+// every wavefront some ray needs the second side, and the others wait for it. (Whole traces of
+// 12000, 30000 and 65000 rays: 255, 244 and 294 us -> 226, 215 and 272; up to 4096 rays no change.
+// Where the lanes are all busy the doubled preparation costs more than it saves: a frame's 180000
+// hits 96 -> 114 us.)
+constexpr uint32_t kAccuratePairs = 65536;  // rays up to which a trace takes two lanes each: half of the chip's lanes
+                                            // at the two waves per SIMD of this kernel
+template <class Src>
+__global__ __launch_bounds__(kTraceBlock) void k_accurate_pairs(TraceParams tp, Src src, HitRec* __restrict__ hits,
+                                                                uint32_t n) {
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, i = t >> 1;
+    HitRec h{};
+    bool ok = false;
+    if (i < n) {
+        h = hits[i];
+        ok = accurate_refine<true>(tp, src, i, h);
+    }
+    const bool first = (wave_ballot(ok) >> (threadIdx.x & 62u)) & 1u;  // side 0 has a result
+    if (ok && (!(threadIdx.x & 1u) || !first)) hits[i] = h;
 }
 
 // Shadow queue entries are ids pixel * samples + light sample.
