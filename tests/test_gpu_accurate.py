@@ -93,3 +93,22 @@ def test_accurate_render_matches_oracle(gpu_ctx, oracle):
         assert e.value.code == -4
     finally:
         gpu_ctx.set_option(V.OPTION_PERSISTENT, 1)
+
+
+def test_two_lanes_per_ray_match_one(gpu_ctx):
+    """A trace of 65537 rays re-runs each hit in one lane, of up to 65536 rays in two: the same
+    records, whole and in parts (an odd one, one of a single ray)."""
+    import gpu_util as G
+    import scenes
+    import vkhrt_amd as V
+    curves = scenes.c0_curves()[:20000]
+    blases = [G.build_blas(gpu_ctx, V.GEOMETRY_PHANTOM_CURVES, curves, per_point=True, transform=x)
+              for x in (None, XF.reshape(12))]
+    tlas = V.TopLevelAccelerationStructure(gpu_ctx, blases)
+    rays = scenes.targeted_rays(curves, 65537, seed=17, dist=(5.0, 300.0))
+    for flags in (V.TRACE_ACCURATE_NORMALS, V.TRACE_ACCURATE_NORMALS | V.TRACE_FP64_POLISH):
+        whole = G.trace(gpu_ctx, tlas, rays, flags)
+        assert (whole["prim"] != 0xFFFFFFFF).sum() > 10000
+        for cuts in ([0, 65536, 65537], [0, 31, 4096, 65537]):
+            parts = np.concatenate([G.trace(gpu_ctx, tlas, rays[a:b], flags) for a, b in zip(cuts, cuts[1:])])
+            assert parts.tobytes() == whole.tobytes(), (flags, cuts)
