@@ -97,6 +97,40 @@ def test_gradient_matches_oracle(gpu_ctx, O):
     assert np.array_equal(np.array(mlp.get_params(), np.float32), P)
 
 
+@pytest.mark.parametrize("n", [1, 15, 64, 65, 16385, 20000])
+def test_gradient_at_chunk_edges(gpu_ctx, O, n):
+    """One sample, part of a wave's 16, a chunk of 64 and one more, one chunk more than 256 blocks
+    take in their first pass: the gradient matches the oracle's in every parameter block, biases and
+    output layer among them, and a second evaluation gives the same bits."""
+    import vkhrt_amd as V
+    mlp = V.ShadowMLP(gpu_ctx, SCENE_MIN, SCENE_MAX, seed=4)
+    P = O.mlp_init(21)
+    P[O.MLP_OFF["b1"]:O.MLP_OFF["b1"] + 64] = 0.05
+    mlp.set_params(P)
+    smp = _samples(n, 24)
+    tgt = (np.random.default_rng(25).random(n) < 0.4).astype(np.float32)
+    ds, dt = _dev(smp), _dev(tgt)
+    runs = []
+    for _ in range(2):
+        grad = torch.zeros(V.SHADOW_MLP_PARAMS, dtype=torch.float32, device="cuda")
+        loss = mlp.gradient(ds.data_ptr(), dt.data_ptr(), n, grad.data_ptr())
+        torch.cuda.synchronize()
+        runs.append(grad.cpu().numpy())
+    assert runs[0].tobytes() == runs[1].tobytes()
+    center, inv_half = _box(O)
+    gref, lref = O.mlp_grad(P, center, inv_half, smp, tgt)
+    assert abs(loss - lref) < 1e-5 * max(1.0, abs(lref)), (loss, lref)
+    # a bf16 rounding that falls the other way moves one of 64 inputs by 2^-8: 5e-4 of a layer's
+    # output for a single sample; a few samples of 64 flip (4e-4 of the gradient measured), and over
+    # thousands the flips average out
+    tol = 2e-3 if n <= 65 else 2e-4
+    for name, size in [("W1", 6144), ("b1", 64), ("W2", 4096), ("b2", 64), ("W3", 4096), ("b3", 64), ("W4", 4096),
+                       ("b4", 64), ("w5", 64), ("b5", 1)]:
+        a, b = (x[O.MLP_OFF[name]:O.MLP_OFF[name] + size] for x in (runs[0], gref))
+        rel = np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-30)
+        assert rel < tol, (name, rel)
+
+
 def test_training_learns_a_half_space(gpu_ctx, O):
     """Visibility = [y_normalized > 0.2]: Adam on the device drives the loss down and the
     classifier right on held-out samples."""
