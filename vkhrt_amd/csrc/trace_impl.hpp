@@ -917,6 +917,7 @@ __device__ __forceinline__ T wave_uniform(const T& v) {
 // one line are serialized, and a grid of 4096 waves probing 7 empty counters each would cost
 // more than the whole tail. All members are wave-uniform.
 struct WorkClaim {
+    static constexpr uint32_t kLeastGrab = 16;
     uint32_t* counter;
     uint32_t* xcd;  // null: one counter
     uint32_t* dry;  // LDS, bit c: counter c is empty (chunked only)
@@ -925,11 +926,12 @@ struct WorkClaim {
     bool exhausted;     // no item left anywhere
     bool shared;        // the items are shared out evenly instead
     uint32_t next, end;  // this wave's share
+    uint32_t grab;       // items the wave takes at a time
 
     __device__ __forceinline__ WorkClaim(uint32_t* c, uint32_t* x, uint32_t chunk, uint32_t n, uint32_t* d)
         : counter(c), xcd(chunk ? x : nullptr), dry(d), total(n), shift(chunk ? uint32_t(__ffs(chunk) - 1) : 0u),
           cx(__builtin_amdgcn_s_getreg((3 << 11) | 20) & 7u),  // hwreg(HW_REG_XCC_ID, 0, 4)
-          left(8u), exhausted(false), shared(fits_lanes(n, gridDim.x)), next(0u), end(0u) {
+          left(8u), exhausted(false), shared(fits_lanes(n, gridDim.x)), next(0u), end(0u), grab(64u) {
         if (!shared) return;
         const uint32_t waves = gridDim.x * (kTraceBlock / 64), per = (n + waves - 1) / waves;
         // blocks go round the XCDs: each XCD's blocks get neighbouring shares
@@ -946,11 +948,11 @@ struct WorkClaim {
         return n <= uint64_t(blocks) * kTraceBlock;
     }
 
-    // The idle lanes of the wave (mask `idle`, the same in every lane) claim one item each;
-    // returns the calling lane's item for `rank` = its rank among the idle lanes, or a value
+    // The idle lanes of the wave (mask `idle`, the same in every lane) claim one item each, the first
+    // `grab` of them; returns the calling lane's item for `rank` = its rank among the idle lanes, or a value
     // >= total when none was left for it.
     __device__ __forceinline__ uint32_t claim(uint64_t idle, uint32_t rank) {
-        const uint32_t n = __popcll(idle);
+        const uint32_t n = min(uint32_t(__popcll(idle)), grab);
         const uint32_t leader = __ffsll((unsigned long long)idle) - 1;
         const uint32_t lane = threadIdx.x & 63u;
         uint32_t base = 0;
@@ -961,8 +963,11 @@ struct WorkClaim {
         if (!xcd) {
             if (lane == leader) base = atomicAdd(counter, n);
             base = __shfl(base, int(leader));
-            if (base + n >= total) exhausted = true;
-            return base + rank;
+            if (base + n >= total)
+                exhausted = true;
+            else
+                grab = min(64u, max(kLeastGrab, (total - base - n) / (gridDim.x * 8u)));
+            return rank < n ? base + rank : 0xFFFFFFFFu;
         }
         // skip the counters the block already found empty
         const uint32_t known = __shfl(*reinterpret_cast<volatile uint32_t*>(dry), 0);
@@ -983,8 +988,12 @@ struct WorkClaim {
         base = __shfl(base, int(leader));
         const uint64_t i = uint64_t(base) + rank;
         uint32_t r = 0xFFFFFFFFu;
-        if (i < lim) r = uint32_t(((((i >> shift) << 3) + cx) << shift) + (i & (chunk - 1)));
-        if (uint64_t(base) + n >= lim) {
+        if (i < lim && rank < n) r = uint32_t(((((i >> shift) << 3) + cx) << shift) + (i & (chunk - 1)));
+        if (uint64_t(base) + n < lim) {
+            // an eighth of the waves, half of gridDim.x, draws on this counter
+            static_assert(kTraceBlock == 256, "four waves a block");
+            grab = min(64u, max(kLeastGrab, uint32_t(lim - base - n) / gridDim.x));
+        } else {
             if (lane == leader) atomicOr(dry, 1u << cx);
             cx = (cx + 1u) & 7u;
             if (--left == 0u) exhausted = true;
@@ -1271,7 +1280,7 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
         // (b) refill idle lanes from the work counters
         if (!work.exhausted) {
             const uint64_t idle = wave_ballot(state == kIdle);
-            if (idle && (__popcll(idle) >= tp.refill_min || idle == wave_ballot(true))) {
+            if (idle && (__popcll(idle) >= min(tp.refill_min, work.grab) || idle == wave_ballot(true))) {
                 const uint32_t r = work.claim(idle, __popcll(idle & lt));
                 if (state == kIdle) {
                     if (r < work.total) {
