@@ -35,7 +35,8 @@ public:
                     best = i;
             if (best >= 0) {
                 *out = kept_[best];
-                kept_[best] = kept_[--count_];
+                --count_;
+                for (int i = best; i < count_; ++i) kept_[i] = kept_[i + 1];
                 return hipSuccess;
             }
         }
@@ -51,14 +52,10 @@ public:
     }
 
     // Takes a block back. Without `idle` the GPU may still be using it; like hipFree this then
-    // waits for the device.
+    // waits for the device. The blocks kept longest make room for it.
     void release(Block b, bool idle) {
         if (!b.p) return;
-        bool keep;
-        {
-            std::lock_guard<std::mutex> g(m_);
-            keep = fits(b);
-        }
+        bool keep = b.bytes >= kMinBytes && b.bytes <= kMaxBytes;
         if (keep && !idle) {
             int cur = device_;
             (void)hipGetDevice(&cur);
@@ -66,11 +63,24 @@ public:
             keep = hipDeviceSynchronize() == hipSuccess;
             if (cur != device_) (void)hipSetDevice(cur);
         }
+        Block old[kMaxBlocks];
+        int n = 0;
         if (keep) {
             std::lock_guard<std::mutex> g(m_);
-            keep = fits(b);
-            if (keep) kept_[count_++] = b;
+            keep = !closed_;
+            if (keep) {
+                size_t held = b.bytes;
+                for (int i = 0; i < count_; ++i) held += kept_[i].bytes;
+                for (; n < count_ && (count_ - n == kMaxBlocks || held > kMaxBytes); ++n) {
+                    old[n] = kept_[n];
+                    held -= kept_[n].bytes;
+                }
+                count_ -= n;
+                for (int i = 0; i < count_; ++i) kept_[i] = kept_[i + n];
+                kept_[count_++] = b;
+            }
         }
+        for (int i = 0; i < n; ++i) (void)hipFree(old[i].p);
         if (!keep) (void)hipFree(b.p);
     }
 
@@ -95,14 +105,9 @@ public:
     }
 
 private:
-    static constexpr size_t kMaxBytes = size_t(1) << 30, kSlack = 4096;
+    // smaller blocks are not kept: hipMalloc and hipFree of up to 1 MiB take 0.4 us each
+    static constexpr size_t kMinBytes = size_t(1) << 20, kMaxBytes = size_t(1) << 30, kSlack = 4096;
     static constexpr int kMaxBlocks = 8;
-
-    bool fits(const Block& b) const {
-        size_t held = b.bytes;
-        for (int i = 0; i < count_; ++i) held += kept_[i].bytes;
-        return !closed_ && count_ < kMaxBlocks && held <= kMaxBytes;
-    }
 
     std::mutex m_;
     Block kept_[kMaxBlocks];
