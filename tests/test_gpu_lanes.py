@@ -124,3 +124,43 @@ def test_shared_out_and_claimed_rays_agree(gpu_ctx, G, curves, count):
         else:
             assert np.array_equal(got["prim"] == 0xFFFFFFFF, ref["prim"] == 0xFFFFFFFF)
     tlas.close()
+
+
+def _mesh(G, ctx, S, verts, idx):
+    """A triangle soup as a BLAS and in the oracle scene."""
+    import torch
+    import vkhrt_amd as V
+    v = np.zeros((len(verts), 8), np.float32)
+    v[:, :3] = verts
+    v[:, 5] = 1.0
+    idx = np.ascontiguousarray(idx, np.uint32)
+    S.add_mesh(v, idx)
+    dv, di = G.dev(v), G.dev(idx)
+    b = V.BottomLevelAccelerationStructure(ctx, V.GEOMETRY_TRIANGLES, dv.data_ptr(), idx.shape[0],
+                                           indices_ptr=di.data_ptr(), vertex_count=v.shape[0], stream=G.stream_ptr())
+    torch.cuda.synchronize()
+    return b
+
+
+@pytest.mark.parametrize("half", [1e3, 1e12, 1e14, 1e15])
+def test_axis_parallel_rays_in_wide_scenes(gpu_ctx, G, oracle, half):
+    """A ray parallel to an axis takes 1e20 for the reciprocal of its zero direction components; the
+    planes of a node 2e15 units wide are then 1e33 or more apart in t, and none of them may overflow
+    on the way. Triangles of a 10000th of the scene, each with an axis-parallel ray at its middle (the
+    triangle test forms size^2 x distance, which stays below 1e37 so)."""
+    import vkhrt_amd as V
+    rng = np.random.default_rng(41)
+    n = 500
+    mid = rng.uniform(-half, half, (n, 1, 3))
+    tri = mid + rng.normal(size=(n, 3, 3)) * (half / 10000.0)
+    S = oracle.Scene()
+    tlas = V.TopLevelAccelerationStructure(gpu_ctx, [_mesh(G, gpu_ctx, S, tri.reshape(-1, 3), np.arange(3 * n).reshape(n, 3))])
+    axis, sign = rng.integers(0, 3, n), rng.choice([-1.0, 1.0], n)
+    rays = np.zeros((n, 8), np.float32)
+    rays[:, :3] = tri.mean(1)
+    rays[np.arange(n), axis] -= sign * half / 20.0
+    rays[np.arange(n), 4 + axis] = sign
+    rays[:, 7] = 3e38
+    ref = S.trace(rays)
+    assert (ref["prim"] != 0xFFFFFFFF).mean() > 0.9
+    G.compare_hits(G.trace(gpu_ctx, tlas, rays), ref, f"scene of +-{half:g}")

@@ -161,12 +161,16 @@ __device__ __forceinline__ void node_visit(const WideNode* nodes, uint32_t node,
     // widened by 8 ulp), so it uses fused multiply-adds. A byte placed in the low half of a 16-bit
     // float is the subnormal q * 2^-24 exactly, and v_fma_mix_f32 reads a 16-bit float operand
     // beside two 32-bit ones: one byte permute prepares two planes, where a conversion each took
-    // two instructions. The factor 2^24 goes into the scale. (About 230 -> 180 VALU instructions per
-    // node test; 1080p frames of 100k strands: LSS 760 -> 730 us, phantom 1316 -> 1300 us.)
+    // two instructions. So the test runs on t / 2^24: the other operands are scaled down to
+    // match, since the scale times 2^24 would overflow for a ray parallel to an axis (inv = 1e20)
+    // in nodes wider than 5e13. (The scaled t lose bits where t < 2e-31: an error of at most 2.4e-38
+    // |d| in distance, far inside the boxes' padding.) About 230 -> 180 VALU instructions per node
+    // test.
     // Each slot contributes one bit of a slot-order hit mask; the metadata is decoded afterwards
     // for the leaf slots hit only. Empty slots are not excluded: they are no internal child and
     // their metadata byte names no record.
-    const float sx24 = sx * 16777216.0f, sy24 = sy * 16777216.0f, sz24 = sz * 16777216.0f;
+    constexpr float kDown = 1.0f / 16777216.0f;
+    const float ox24 = ox * kDown, oy24 = oy * kDown, oz24 = oz * kDown, tmin24 = tmin * kDown, tcur24 = tcur * kDown;
     uint32_t lm = 0;
 #pragma unroll
     for (int h = 0; h < 4; ++h) {
@@ -175,11 +179,11 @@ __device__ __forceinline__ void node_visit(const WideNode* nodes, uint32_t node,
         const h2 az = qpair(nzl, nzh, h), bz = qpair(fzl, fzh, h);
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
-            const float t0x = fmaf(float(ax[k]), sx24, ox), t1x = fmaf(float(bx[k]), sx24, ox);
-            const float t0y = fmaf(float(ay[k]), sy24, oy), t1y = fmaf(float(by[k]), sy24, oy);
-            const float t0z = fmaf(float(az[k]), sz24, oz), t1z = fmaf(float(bz[k]), sz24, oz);
-            const float tn = fmaxf(fmaxf(t0x, t0y), fmaxf(t0z, tmin));
-            const float tf = fminf(fminf(t1x, t1y), fminf(t1z, tcur)) * 1.00000095f;
+            const float t0x = fmaf(float(ax[k]), sx, ox24), t1x = fmaf(float(bx[k]), sx, ox24);
+            const float t0y = fmaf(float(ay[k]), sy, oy24), t1y = fmaf(float(by[k]), sy, oy24);
+            const float t0z = fmaf(float(az[k]), sz, oz24), t1z = fmaf(float(bz[k]), sz, oz24);
+            const float tn = fmaxf(fmaxf(t0x, t0y), fmaxf(t0z, tmin24));
+            const float tf = fminf(fminf(t1x, t1y), fminf(t1z, tcur24)) * 1.00000095f;
             lm |= tn <= tf ? 1u << (2 * h + k) : 0u;
         }
     }
