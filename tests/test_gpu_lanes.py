@@ -164,3 +164,27 @@ def test_axis_parallel_rays_in_wide_scenes(gpu_ctx, G, oracle, half):
     ref = S.trace(rays)
     assert (ref["prim"] != 0xFFFFFFFF).mean() > 0.9
     G.compare_hits(G.trace(gpu_ctx, tlas, rays), ref, f"scene of +-{half:g}")
+
+
+def test_zero_distances_of_either_sign_are_equal(gpu_ctx, G, oracle):
+    """A ray that starts in the plane of two triangles of opposite winding hits one at t = +0 and the
+    other at t = -0 (the numerator cancels to +0, the determinants have opposite signs; all numbers
+    here are exact): equal distances, so the lower triangle wins, whichever of them it is."""
+    import vkhrt_amd as V
+    a, b = [[-1, -1, 0], [2, -1, 0], [-1, 2, 0]], [[-1, -1, 0], [-1, 2, 0], [2, -1, 0]]
+    rays = np.zeros((4, 8), np.float32)
+    rays[:, :2] = [[0.25, 0.125], [0.25, -0.5], [-0.5, 0.25], [0.0625, 0.125]]
+    rays[:, 4:7] = [[1.0, 0.5, 0.25], [1.0, 0.5, -0.25], [-1.0, 0.25, 0.5], [0.25, 1.0, -0.5]]
+    rays[:, 7] = 10.0
+    for tris in ([a, b], [b, a]):
+        S = oracle.Scene()
+        verts, idx = np.array(tris, np.float32).reshape(-1, 3), np.arange(6).reshape(2, 3)
+        one = _mesh(G, gpu_ctx, S, verts, idx)
+        ref = S.trace(rays)
+        assert (ref["t"] == 0.0).all() and (ref["prim"] == 0).all()
+        G.compare_hits(G.trace(gpu_ctx, V.TopLevelAccelerationStructure(gpu_ctx, [one]), rays), ref, "one mesh")
+        S = oracle.Scene()
+        parts = [_mesh(G, gpu_ctx, S, np.array(t, np.float32), np.arange(3).reshape(1, 3)) for t in tris]
+        ref = S.trace(rays)
+        assert (ref["t"] == 0.0).all() and (ref["inst"] == 0).all()
+        G.compare_hits(G.trace(gpu_ctx, V.TopLevelAccelerationStructure(gpu_ctx, parts), rays), ref, "two instances")

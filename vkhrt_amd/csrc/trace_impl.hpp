@@ -1033,9 +1033,11 @@ constexpr uint32_t kEarlierLow = 0u;
 constexpr uint32_t kCompactIterationCap = 1u << 24;
 constexpr uint32_t kWalkerOne = 1u << 16;  // s_cnt: queued pairs in the low half, helper lanes in the high half
 
-// float <-> unsigned with the float order (t may be negative for rays with a negative tmin)
+// float <-> unsigned with the float order (t may be negative for rays with a negative tmin); -0
+// takes the place of +0, since equal distances resolve by primitive (a triangle's t at the ray's
+// origin may be either)
 __device__ __forceinline__ uint32_t t_ord(float f) {
-    const uint32_t b = __float_as_uint(f);
+    const uint32_t b = __float_as_uint(f + 0.0f);
     return b ^ ((b & 0x80000000u) ? 0xFFFFFFFFu : 0x80000000u);
 }
 __device__ __forceinline__ float ord_t(uint32_t u) {
@@ -1123,8 +1125,12 @@ struct CWalker {
 
 // One leaf record of a mode other than phantom against a ray: the hit within [tmin, tmax] with
 // its primitive id and payload (LSS: u and the normal; DOTS, triangles: two barycentrics, the
-// record's slot and the triangle of a DOTS piece). A piece's nearest triangle wins, the lower
-// one on equal t.
+// record's slot, and the triangle of a DOTS piece with kZeroNegative where t is -0, which the key
+// does not tell from +0). A piece's nearest triangle wins, the lower one on equal t.
+constexpr uint32_t kZeroNegative = 0x80000000u;
+__device__ __forceinline__ uint32_t zero_sign(float t) {
+    return __float_as_uint(t) == kZeroNegative ? kZeroNegative : 0u;
+}
 __device__ __forceinline__ bool leaf_intersect(int mode, const BlasDev& B, uint32_t slot, f3 o, f3 d, float tmin,
                                                float tmax, float& t, uint32_t& pid, float4& pay) {
     bool hit = false;
@@ -1146,7 +1152,7 @@ __device__ __forceinline__ bool leaf_intersect(int mode, const BlasDev& B, uint3
                           b2)) {
             hit = true;
             pid = gmem(B.prim_ids)[slot];
-            pay = make_float4(b1, b2, __uint_as_float(slot), 0.0f);
+            pay = make_float4(b1, b2, __uint_as_float(slot), __uint_as_float(zero_sign(t)));
         }
     } else {
         const auto* pr = gmem(B.prims + size_t(slot) * 4);
@@ -1163,7 +1169,7 @@ __device__ __forceinline__ bool leaf_intersect(int mode, const BlasDev& B, uint3
                 hit = true;
                 bt = tt;
                 btri = uint32_t(tri);
-                pay = make_float4(b1, b2, __uint_as_float(slot), __uint_as_float(btri));
+                pay = make_float4(b1, b2, __uint_as_float(slot), __uint_as_float(btri | zero_sign(tt)));
             }
         }
         if (hit) {
@@ -1331,9 +1337,12 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
                     best.c = pay.w;
                     if constexpr (G::kMixed || G::kMode == kDots || G::kMode == kTriangles) {
                         best.slot = __float_as_uint(pay.z);  // read for DOTS and triangle hits only
-                        best.extra = __float_as_uint(pay.w);
-                        if constexpr (G::kMixed)
-                            if (const uint32_t mode = blas(best.inst).mode; mode != kDots) best.extra = 0u;
+                        const int mode = G::kMixed ? int(blas(best.inst).mode) : G::kMode;
+                        if (mode == kDots || mode == kTriangles) {
+                            const uint32_t w = __float_as_uint(pay.w);
+                            best.extra = w & ~kZeroNegative;
+                            best.t = __uint_as_float(__float_as_uint(best.t) | (w & kZeroNegative));
+                        }
                     }
                 }
                 snk(idx, ow, dw, best);
