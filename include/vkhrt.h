@@ -153,7 +153,10 @@ typedef struct vkhrt_hit {
 } vkhrt_hit;
 
 /* vkhrt_trace_rays flags */
-#define VKHRT_TRACE_TERMINATE_ON_FIRST_HIT (1u << 0) /* shadow / any-hit rays */
+#define VKHRT_TRACE_TERMINATE_ON_FIRST_HIT (1u << 0) /* shadow / any-hit rays; the record is the first hit
+                                                        of the ray's walk through the tree, or some hit
+                                                        where all instances are phantom curves of one
+                                                        radius model */
 #define VKHRT_TRACE_FP64_POLISH (1u << 3)            /* FP64 Newton polish of grazing phantom roots */
 #define VKHRT_TRACE_ACCURATE_NORMALS (1u << 5)       /* phantom hits: t, u and normal of the final hit
                                                         re-evaluated in double-word FP32 (the FP64

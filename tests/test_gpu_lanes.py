@@ -188,3 +188,29 @@ def test_zero_distances_of_either_sign_are_equal(gpu_ctx, G, oracle):
         ref = S.trace(rays)
         assert (ref["t"] == 0.0).all() and (ref["inst"] == 0).all()
         G.compare_hits(G.trace(gpu_ctx, V.TopLevelAccelerationStructure(gpu_ctx, parts), rays), ref, "two instances")
+
+
+@pytest.mark.parametrize("modes", [("lss",), ("dots",), ("mesh",), ("lss", "lss"), ("phantom", "mesh"),
+                                   ("phantom", "lss", "dots")])
+def test_any_hit_record_is_the_rays_own(gpu_ctx, G, oracle, curves, modes):
+    """The record that an any-hit trace of these modes returns is the first hit of the ray's own walk:
+    the same whole and in parts, in any order, and with one thread per ray."""
+    import scenes
+    import vkhrt_amd as V
+    tlas = V.TopLevelAccelerationStructure(gpu_ctx, [_add(oracle.Scene(), oracle, G, gpu_ctx, m, curves) for m in modes])
+    rays = scenes.targeted_rays(curves, 300001, seed=43, dist=(1.0, 60.0))
+    for flags in (V.TRACE_TERMINATE_ON_FIRST_HIT, V.TRACE_TERMINATE_ON_FIRST_HIT | V.TRACE_FP64_POLISH):
+        gpu_ctx.set_option(V.OPTION_PERSISTENT, 0)
+        try:
+            ref = G.trace(gpu_ctx, tlas, rays, flags=flags)
+        finally:
+            gpu_ctx.set_option(V.OPTION_PERSISTENT, 1)
+        assert (ref["prim"] != 0xFFFFFFFF).mean() > 0.25
+        whole = G.trace(gpu_ctx, tlas, rays, flags=flags)
+        assert whole.tobytes() == ref.tobytes(), (whole["prim"] != ref["prim"]).sum()
+        order = np.random.default_rng(44).permutation(len(rays))
+        mixed = np.empty_like(ref)
+        mixed[order] = G.trace(gpu_ctx, tlas, rays[order], flags=flags)
+        assert mixed.tobytes() == ref.tobytes()
+        cut = 4099
+        assert G.trace(gpu_ctx, tlas, rays[:cut], flags=flags).tobytes() == ref[:cut].tobytes()

@@ -1215,9 +1215,12 @@ int trace_launch(vkhrt_context* c, const vkhrt_tlas* t, const vkhrt_ray* rays, u
         tp.cand_keys = s.cand_keys;
         if (!tp.work) tp.work = s.work;  // the deferred pipeline runs on persistent kernels
     }
+    // With any hit and polish, a TLAS of several modes keeps one thread per ray: the candidates are
+    // those met before the ray's first hit, where the lanes may queue later ones too.
+    const bool lanes = tp.work != nullptr && !(polish && (flags & VKHRT_TRACE_TERMINATE_ON_FIRST_HIT));
     Timer tm(c, st, timed ? "trace_rays" : nullptr);
     hipError_t e = vk::launch_trace_rays(tp, reinterpret_cast<const float*>(rays), count,
-                                         reinterpret_cast<vk::HitRec*>(hits), nullptr, trace_variant(t, polish, tp.work != nullptr),
+                                         reinterpret_cast<vk::HitRec*>(hits), nullptr, trace_variant(t, polish, lanes),
                                          stack_kind_for(c, t), st);
     if (e == hipSuccess && accurate)
         e = vk::launch_accurate_hits(tp, reinterpret_cast<const float*>(rays), count, reinterpret_cast<vk::HitRec*>(hits),

@@ -1126,11 +1126,13 @@ struct CWalker {
 // One leaf record of a mode other than phantom against a ray: the hit within [tmin, tmax] with
 // its primitive id and payload (LSS: u and the normal; DOTS, triangles: two barycentrics, the
 // record's slot, and the triangle of a DOTS piece with kZeroNegative where t is -0, which the key
-// does not tell from +0). A piece's nearest triangle wins, the lower one on equal t.
+// does not tell from +0). A piece's nearest triangle wins, the lower one on equal t; with FIRST
+// its first triangle hit.
 constexpr uint32_t kZeroNegative = 0x80000000u;
 __device__ __forceinline__ uint32_t zero_sign(float t) {
     return __float_as_uint(t) == kZeroNegative ? kZeroNegative : 0u;
 }
+template <bool FIRST>
 __device__ __forceinline__ bool leaf_intersect(int mode, const BlasDev& B, uint32_t slot, f3 o, f3 d, float tmin,
                                                float tmax, float& t, uint32_t& pid, float4& pay) {
     bool hit = false;
@@ -1165,6 +1167,7 @@ __device__ __forceinline__ bool leaf_intersect(int mode, const BlasDev& B, uint3
             f3 v0, v1, v2;
             dots_tri(P, tri >> 1, tri & 1, v0, v1, v2);
             float tt, b1, b2;
+            if (FIRST && hit) continue;
             if (tri_intersect(TR, o, v0, v1, v2, tmin, bt, tt, b1, b2) && (!hit || tt < bt)) {
                 hit = true;
                 bt = tt;
@@ -1180,7 +1183,15 @@ __device__ __forceinline__ bool leaf_intersect(int mode, const BlasDev& B, uint3
     return hit;
 }
 
-template <class G, bool ANY, int STACK, int IM, class Src, class Snk>
+// ORDERED (any hit): the ray's result is the first hit of its own walk, whichever rays share the
+// wave. A walker numbers the records that it queues; a hit's key has that number in the place of
+// t, and only records after the least hit are dropped. A walker that hands over its bottom group,
+// which comes last in what it has left, hands the last quarter of its remaining numbers with it,
+// so the numbers of a ray's walkers follow the order of its walk; it keeps the group when the
+// quarter would not cover every record of the instance. (12.8M records allow some 15 hand-overs in
+// a row. Any-hit traces of 4096, 262144 and 2M rays against 128k capsules: 119, 257 and 1023 us,
+// 108, 242 and 1005 with whichever hit comes first, 276, 399 and 2163 with one thread per ray.)
+template <class G, bool ANY, bool ORDERED, int STACK, int IM, class Src, class Snk>
 __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkClaim& work, uint2* lds, Src&& src,
                                                    Snk&& snk) {
     // One instance: its BLAS fields are read once here, into scalar registers, instead of per
@@ -1204,6 +1215,7 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
             return tp.inst[i].blas;
     };
     static_assert(!G::kMixed || G::kCompact, "compacted lanes serve BVH instances");
+    static_assert(ANY || !ORDERED, "closest hits are ordered by t");
     constexpr bool kHasPhantom = G::kMixed || G::kMode == kPhantom;
     constexpr uint32_t kWaves = kTraceBlock / 64;
     __shared__ uint32_t s_leaf[kWaves * kLeafQueue];     // leaf queue: slots
@@ -1214,6 +1226,9 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
     __shared__ uint32_t s_cnt[kTraceBlock];            // pairs of the lane's ray still queued (low half),
                                                        // other lanes walking its subtrees (high half)
     __shared__ uint8_t s_xfer[kTraceBlock];            // donor lane by rank (subtree hand-over)
+    __shared__ uint32_t s_leaf_no[ORDERED ? kWaves * kLeafQueue : 1];  // numbers of the queued records
+    __shared__ uint32_t s_queue_no[ORDERED && kHasPhantom ? kWaves * kCompactQueue : 1];
+    __shared__ float s_t[ORDERED ? kTraceBlock : 1];   // t of the lane's hit
     // kTrav: walking its own ray; kHelp: walking a subtree of the ray of lane `home`; kWait: own
     // walk done, waiting for queued pairs and helpers of its ray
     enum { kIdle = 0, kInst = 1, kTrav = 2, kWait = 3, kHelp = 4 };
@@ -1223,6 +1238,8 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
     uint32_t* leaf = s_leaf + (threadIdx.x >> 6) * kLeafQueue;
     uint8_t* leaf_lane = s_leaf_lane + (threadIdx.x >> 6) * kLeafQueue;
     uint32_t* queue = s_queue + (kHasPhantom ? (threadIdx.x >> 6) * kCompactQueue : 0u);
+    uint32_t* leaf_no = s_leaf_no + (ORDERED ? (threadIdx.x >> 6) * kLeafQueue : 0u);
+    uint32_t* queue_no = s_queue_no + (ORDERED && kHasPhantom ? (threadIdx.x >> 6) * kCompactQueue : 0u);
     CWalker<STACK> W;
     W.o = W.d = f3{0.0f, 0.0f, 0.0f};
     W.pmask = 0;
@@ -1234,6 +1251,11 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
     int state = kIdle;
     bool ray_done = false;
     uint32_t ln = 0, qn = 0;  // wave-uniform lengths of the leaf queue and the Prhi queue
+    uint32_t no = 0, no_end = 0;  // ORDERED: the walker's next number and the end of its numbers
+    // whether an any-hit ray with key `kk` has no use for the record numbered `n` or what follows it
+    auto over = [](unsigned long long kk, uint32_t n) {
+        return uint32_t(kk) != kNoHitLow && (!ORDERED || uint32_t(kk >> 32) < n);
+    };
 #ifdef VKHRT_WORK_COUNTERS
     unsigned long long wc[14] = {};  // WorkCounter sums of this wave (wave-uniform)
     unsigned long long t_it = clock64(), t_mid = t_it;
@@ -1258,6 +1280,10 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
         __builtin_amdgcn_wave_barrier();
         if (state != kIdle) {
             const unsigned long long kk = s_key[wbase + home];
+            if constexpr (ORDERED) {
+                if (state == kTrav && over(kk, no)) state = kWait;
+                return;
+            }
             tcur = ord_t(uint32_t(kk >> 32));
             if (ANY && state != kHelp && uint32_t(kk) != kNoHitLow && !ray_done) {
                 ray_done = true;
@@ -1275,6 +1301,7 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
         }
         // (a) a waiting lane whose pairs are all merged moves to its next instance or finishes
         if (state == kWait && s_cnt[threadIdx.x] == 0u) {
+            if constexpr (ORDERED) ray_done = ray_done || uint32_t(s_key[threadIdx.x]) != kNoHitLow;
             if constexpr (IM != kInstOne) {
                 const unsigned long long kk = s_key[threadIdx.x];
                 const uint32_t lo = uint32_t(kk);
@@ -1296,7 +1323,7 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
                     if (r < work.total) {
                         src(r, idx, ow, dw, tmin, tmax);
                         tcur = tmax;
-                        s_key[threadIdx.x] = lane_key(tmax, kNoHitLow);
+                        s_key[threadIdx.x] = ORDERED ? ~0ull : lane_key(tmax, kNoHitLow);
                         s_cnt[threadIdx.x] = 0u;
                         home = lane;
                         inst = 0;
@@ -1328,7 +1355,7 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
                     best.u = best.a = best.b = best.c = 0.0f;
                 } else {
                     const float4 pay = s_pay[threadIdx.x];
-                    best.t = ord_t(uint32_t(kk >> 32));
+                    best.t = ORDERED ? s_t[threadIdx.x] : ord_t(uint32_t(kk >> 32));
                     best.inst = IM == kInstOne ? 0u : binst;
                     best.pid = IM == kInstOne ? lo - 1u : bpid;
                     best.u = pay.x;
@@ -1358,6 +1385,8 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
                     dd = xform_dir(I.inv, dw);
                 }
                 W.begin(oo, dd);
+                no = 0u;
+                no_end = 0xFFFFFFFFu;
                 state = kTrav;
             }
         }
@@ -1368,7 +1397,9 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
         // group of a walking lane and continue that ray from there, so the last long rays of
         // the frame are walked by many lanes instead of one
         if (work.exhausted) {
-            const bool give = (state == kTrav || state == kHelp) && W.sp > W.sb;
+            bool give = (state == kTrav || state == kHelp) && W.sp > W.sb;
+            const uint32_t part = (no_end - no) >> 2;  // of its numbers
+            if constexpr (ORDERED) give = give && part > blas(inst).nprims;
             const uint64_t dm = wave_ballot(give);
             const uint64_t im = wave_ballot(state == kIdle);
             if (dm && im) {
@@ -1385,19 +1416,35 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
                 const uint32_t goct = __shfl(W.oct, from), gsb = uint32_t(__shfl(W.sb, from));
                 const uint32_t ghome = __shfl(home, from), ginst = __shfl(inst, from);
                 const float gtmin = __shfl(tmin, from);
+                uint32_t gno = 0, gend = 0;
+                float gtmax = 0.0f;
+                if constexpr (ORDERED) {
+                    gend = __shfl(no_end, from);
+                    gno = gend - uint32_t(__shfl(part, from));
+                    gtmax = __shfl(tcur, from);
+                }
                 if (take) {
                     const uint2 grp = lds[(from - int(lane)) + int(gsb) * kTraceBlock];
                     W.adopt(go, gd, gi, goct, grp);
                     home = ghome;
                     inst = ginst;
                     tmin = gtmin;
-                    tcur = ord_t(uint32_t(s_key[wbase + home] >> 32));
+                    if constexpr (ORDERED) {
+                        tcur = gtmax;
+                        no = gno;
+                        no_end = gend;
+                    } else {
+                        tcur = ord_t(uint32_t(s_key[wbase + home] >> 32));
+                    }
                     atomicAdd(&s_cnt[wbase + home], kWalkerOne);
                     state = kHelp;
                 }
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 __builtin_amdgcn_wave_barrier();
-                if (give && kd < n) ++W.sb;  // the group now belongs to the helper
+                if (give && kd < n) {  // the group now belongs to the helper
+                    ++W.sb;
+                    if constexpr (ORDERED) no_end -= part;
+                }
                 VK_WC(kWcHandovers, n);
             }
         }
@@ -1424,11 +1471,12 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
                 const float ptmin = __shfl(tmin, owner), ptmax = __shfl(tmax, owner);
                 const uint32_t pinst = __shfl(inst, owner), pidx = __shfl(idx, owner);
                 const uint32_t os = wbase + uint32_t(owner);
+                const uint32_t pno = ORDERED && lane < m ? queue_no[qn - m + lane] : 0u;
                 unsigned long long k = ~0ull;
                 PhantomHit ph;
                 bool hit = false;
                 if (lane < m) {
-                    const bool skip = ANY && uint32_t(s_key[os]) != kNoHitLow;  // already occluded
+                    const bool skip = ANY && over(s_key[os], pno);  // already occluded
                     if (!skip) {
                         const BlasDev& B = blas(pinst);
                         RayFrame F;
@@ -1450,7 +1498,8 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
                         }
                         hit = hit && ph.t >= ptmin && ph.t <= ptmax;
                         if (hit) {
-                            k = lane_key(ph.t, gmem(B.prim_ids)[slot] + 1u);
+                            const uint32_t low = gmem(B.prim_ids)[slot] + 1u;
+                            k = ORDERED ? (static_cast<unsigned long long>(pno) << 32) | low : lane_key(ph.t, low);
                             atomicMin(&s_key[os], k);
                         }
                     }
@@ -1459,7 +1508,10 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 __builtin_amdgcn_wave_barrier();
                 // the unique winner for this owner writes the payload
-                if (hit && s_key[os] == k) s_pay[os] = make_float4(ph.u, ph.ncx, ph.ncy, ph.nsz);
+                if (hit && s_key[os] == k) {
+                    s_pay[os] = make_float4(ph.u, ph.ncx, ph.ncy, ph.nsz);
+                    if constexpr (ORDERED) s_t[os] = ph.t;
+                }
                 qn -= m;
                 merged();
                 VK_WC_END(kWcCyclesRounds);
@@ -1479,11 +1531,13 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
             bool cand = false, hit = false;
             unsigned long long k = ~0ull;
             float4 pay = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            float ptmin = 0.0f;
+            float ptmin = 0.0f, t = 0.0f;
             if constexpr (G::kMixed || G::kMode != kPhantom) ptmin = __shfl(tmin, owner);
+            const float ptmax = ORDERED ? __shfl(tmax, owner) : 0.0f;
+            const uint32_t pno = ORDERED && lane < m ? leaf_no[ln - m + lane] : 0u;
             if (lane < m) {
                 const unsigned long long kk = s_key[os];
-                const bool skip = ANY && uint32_t(kk) != kNoHitLow;  // already occluded
+                const bool skip = ANY && over(kk, pno);  // already occluded
                 if (!skip) {
                     const BlasDev& B = blas(pinst);
                     const int mode = G::kMixed ? int(B.mode) : G::kMode;
@@ -1492,11 +1546,11 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
                         const float4 a = pr[0], b = pr[3];
                         cand = ray_cylinder(po, pd, f3{a.x, a.y, a.z}, f3{b.x, b.y, b.z}, gmem(B.aux)[slot]);
                     } else if (G::kMixed || G::kMode != kPhantom) {
-                        float t = 0.0f;
                         uint32_t pid = 0;
-                        hit = leaf_intersect(mode, B, slot, po, pd, ptmin, ord_t(uint32_t(kk >> 32)), t, pid, pay);
+                        hit = leaf_intersect<ORDERED>(mode, B, slot, po, pd, ptmin, ORDERED ? ptmax : ord_t(uint32_t(kk >> 32)),
+                                                      t, pid, pay);
                         if (hit) {
-                            k = lane_key(t, pid + 1u);
+                            k = ORDERED ? (static_cast<unsigned long long>(pno) << 32) | (pid + 1u) : lane_key(t, pid + 1u);
                             atomicMin(&s_key[os], k);
                         }
                     }
@@ -1505,7 +1559,11 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
             }
             if constexpr (kHasPhantom) {
                 const uint64_t cm = wave_ballot(cand);
-                if (cand) queue[qn + __popcll(cm & lt)] = (uint32_t(owner) << kCompactSlotBits) | slot;
+                if (cand) {
+                    const uint32_t at = qn + __popcll(cm & lt);
+                    queue[at] = (uint32_t(owner) << kCompactSlotBits) | slot;
+                    if constexpr (ORDERED) queue_no[at] = pno;
+                }
                 qn += __popcll(cm);
                 VK_WC(kWcPairs, __popcll(cm));
             }
@@ -1513,7 +1571,10 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
             if constexpr (G::kMixed || G::kMode != kPhantom) {
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 __builtin_amdgcn_wave_barrier();
-                if (hit && s_key[os] == k) s_pay[os] = pay;
+                if (hit && s_key[os] == k) {
+                    s_pay[os] = pay;
+                    if constexpr (ORDERED) s_t[os] = t;
+                }
                 merged();
             } else {
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -1535,7 +1596,7 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
                 VK_WC(kWcStepLanes, __popcll(wave_ballot(wk)));
             }
 #endif
-            if (state == kHelp && ANY && uint32_t(s_key[wbase + home]) != kNoHitLow) {
+            if (state == kHelp && ANY && over(s_key[wbase + home], no)) {
                 atomicSub(&s_cnt[wbase + home], kWalkerOne);  // the ray is occluded already
                 W.pmask = 0;
                 state = kIdle;
@@ -1554,6 +1615,7 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
                     const uint32_t at = ln + __popcll(am & lt);
                     leaf[at] = W.pbase + uint32_t(__ffs(W.pmask) - 1);
                     leaf_lane[at] = uint8_t(home);
+                    if constexpr (ORDERED) leaf_no[at] = no++;
                     W.pmask &= W.pmask - 1u;
                     ++added;
                 }
@@ -1598,7 +1660,7 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
 constexpr int lanes_waves(int stack) { return stack <= 12 ? 4 : 1; }
 
 // Persistent loop for one geometry variant.
-template <class G, bool ANY, int STACK, int IM = kInstMany, class Src, class Snk>
+template <class G, bool ANY, int STACK, int IM = kInstMany, bool ORDERED = false, class Src, class Snk>
 __device__ __forceinline__ void persistent_lanes(const TraceParams& tp, uint32_t total, uint32_t* counter, uint2* lds,
                                                  Src&& src, Snk&& snk, uint32_t* xcd = nullptr) {
     // an empty queue (uniform over the grid) ends the launch without touching the counter
@@ -1610,7 +1672,7 @@ __device__ __forceinline__ void persistent_lanes(const TraceParams& tp, uint32_t
         __syncthreads();
     }
     WorkClaim work(counter, xcd, chunk, total, &s_dry);
-    persistent_compact<G, ANY, STACK, IM>(tp, work, lds, src, snk);
+    persistent_compact<G, ANY, ORDERED, STACK, IM>(tp, work, lds, src, snk);
 }
 
 template <class G, bool ANY, int STACK, int IM>
@@ -1618,7 +1680,8 @@ __global__ __launch_bounds__(kTraceBlock, lanes_waves(STACK)) void k_trace_rays_
                                                                        uint32_t n, HitRec* __restrict__ hits,
                                                                        uint32_t* __restrict__ counter) {
     __shared__ uint2 stk[STACK * kTraceBlock];
-    persistent_lanes<G, ANY, STACK, IM>(
+    // An any-hit record is the ray's own first hit, but for phantom curves alone, where it may be any.
+    persistent_lanes<G, ANY, STACK, IM, ANY && (G::kMixed || G::kMode != kPhantom)>(
         tp, n, counter, stk + threadIdx.x,
         [&](uint32_t i, uint32_t& id, f3& o, f3& d, float& tmin, float& tmax) {
             id = i;
