@@ -266,3 +266,26 @@ def test_cpp_mirror_without_device():
     cam = np.array([float.fromhex(x) for x in lines[0].split()], np.float32)
     vi, pi = O.camera((0, 60, 300), (0, 40, 0), tan_half_fovy=np.float32(0.57735026), aspect=16.0 / 9.0)
     assert np.array_equal(cam[:16], vi) and np.array_equal(cam[16:], pi)
+
+
+def test_build_memory_pool():
+    """vkhrt_amd/csrc/mem_pool.hpp over a stand-in for the HIP allocator (tests/cpp/mem_pool_test):
+    reuse, eviction, memory running out while a pool keeps blocks, blocks passed between threads."""
+    import subprocess
+    exe = os.path.join(ROOT, "tests", "cpp", "mem_pool_test")
+    subprocess.run(["make", "-s", "-C", os.path.join(ROOT, "tests", "cpp"), exe], check=True)
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout.strip() == "mem_pool ok", r.stderr
+
+
+def test_device_memory_gives_the_kept_blocks_back():
+    """Every allocation of device memory frees what the build pools keep before it fails: only
+    mem_pool.hpp names the allocator itself."""
+    import glob
+    for path in glob.glob(os.path.join(ROOT, "vkhrt_amd", "csrc", "*")):
+        if not path.endswith((".cpp", ".hpp", ".hip")) or path.endswith("mem_pool.hpp"):
+            continue
+        src = open(path).read()
+        direct = [m for m in re.finditer(r"\bhipMalloc(Async|Managed)?\(", src)
+                  if "retry_trimmed" not in src[max(0, m.start() - 80):m.start()]]
+        assert not direct, (path, [src.count("\n", 0, m.start()) + 1 for m in direct])

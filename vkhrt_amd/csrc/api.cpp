@@ -364,12 +364,12 @@ int ensure_render_scratch(vkhrt_context* c, size_t npix, size_t nwork) {
     c->vis = nullptr;
     c->cap_pixels = 0;
     c->cap_work = 0;
-    hipError_t e = hipMalloc(&c->hitbuf, npix * sizeof(float4));
-    if (e == hipSuccess) e = hipMalloc(&c->queue, npix * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc(&c->hitrec, npix * sizeof(vk::HitRec));
-    if (e == hipSuccess) e = hipMalloc(&c->vis, npix * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(&c->live, npix * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc(&c->live_mask, (nwork + 63) / 64 * sizeof(uint64_t));
+    hipError_t e = vk::device_malloc(&c->hitbuf, npix * sizeof(float4));
+    if (e == hipSuccess) e = vk::device_malloc(&c->queue, npix * sizeof(uint32_t));
+    if (e == hipSuccess) e = vk::device_malloc(&c->hitrec, npix * sizeof(vk::HitRec));
+    if (e == hipSuccess) e = vk::device_malloc(&c->vis, npix * sizeof(float));
+    if (e == hipSuccess) e = vk::device_malloc(&c->live, npix * sizeof(uint32_t));
+    if (e == hipSuccess) e = vk::device_malloc(&c->live_mask, (nwork + 63) / 64 * sizeof(uint64_t));
     if (e != hipSuccess) return hip_fail(c, e, "render scratch");
     c->cap_pixels = npix;
     c->cap_work = nwork;
@@ -384,7 +384,7 @@ int ensure_polish_scratch(vkhrt_context* c, size_t nrays) {
         hipFree(c->keys);
         c->keys = nullptr;
         c->keys_cap = 0;
-        e = hipMalloc(&c->keys, nrays * sizeof(unsigned long long));
+        e = vk::device_malloc(&c->keys, nrays * sizeof(unsigned long long));
         if (e != hipSuccess) return hip_fail(c, e, "polish keys");
         c->keys_cap = nrays;
     }
@@ -397,9 +397,9 @@ int ensure_polish_scratch(vkhrt_context* c, size_t nrays) {
         c->cand_hits = nullptr;
         c->cand_keys = nullptr;
         c->defer_cap = 0;
-        e = hipMalloc(&c->defer, cap * sizeof(uint4));
-        if (e == hipSuccess) e = hipMalloc(&c->cand_hits, cap * sizeof(vk::HitRec));
-        if (e == hipSuccess) e = hipMalloc(&c->cand_keys, cap * sizeof(unsigned long long));
+        e = vk::device_malloc(&c->defer, cap * sizeof(uint4));
+        if (e == hipSuccess) e = vk::device_malloc(&c->cand_hits, cap * sizeof(vk::HitRec));
+        if (e == hipSuccess) e = vk::device_malloc(&c->cand_keys, cap * sizeof(unsigned long long));
         if (e != hipSuccess) return hip_fail(c, e, "polish queue");
         c->defer_cap = uint32_t(cap);
     }
@@ -415,9 +415,9 @@ int ensure_neural_scratch(vkhrt_context* c, size_t npix) {
     c->fallback = nullptr;
     c->dirs = nullptr;
     c->cap_neural = 0;
-    hipError_t e = hipMalloc(&c->origins, npix * sizeof(float4));
-    if (e == hipSuccess) e = hipMalloc(&c->fallback, npix * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc(&c->dirs, npix * sizeof(float4));
+    hipError_t e = vk::device_malloc(&c->origins, npix * sizeof(float4));
+    if (e == hipSuccess) e = vk::device_malloc(&c->fallback, npix * sizeof(uint32_t));
+    if (e == hipSuccess) e = vk::device_malloc(&c->dirs, npix * sizeof(float4));
     if (e != hipSuccess) return hip_fail(c, e, "neural shadow scratch");
     c->cap_neural = npix;
     return VKHRT_SUCCESS;
@@ -445,22 +445,22 @@ int ensure_batch_scratch(vkhrt_context* c, size_t paths) {
     free_batch_scratch(c);
     ++c->batch_gen;
     const size_t cand = std::max<size_t>(paths, 65536);
-    hipError_t e = hipMalloc(&c->b_ray, paths * 2 * sizeof(float4));
-    if (e == hipSuccess) e = hipMalloc(&c->b_thr, paths * sizeof(float4));
-    if (e == hipSuccess) e = hipMalloc(&c->b_rad, paths * sizeof(float4));
-    if (e == hipSuccess) e = hipMalloc(&c->b_nee, paths * sizeof(float4));
-    if (e == hipSuccess) e = hipMalloc(&c->b_hits, paths * sizeof(vk::HitRec));
-    if (e == hipSuccess) e = hipMalloc(&c->b_q0, paths * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc(&c->b_q1, paths * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc(&c->b_order, paths * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc(&c->b_squeue, paths * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc(&c->b_qsort, paths * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc(&c->b_bins, 2 * vk::kRayBins * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc(&c->b_counters, vk::kBatchCounterWords * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMalloc(&c->b_keys, paths * sizeof(unsigned long long));
-    if (e == hipSuccess) e = hipMalloc(&c->b_defer, cand * sizeof(uint4));
-    if (e == hipSuccess) e = hipMalloc(&c->b_cand_hits, cand * sizeof(vk::HitRec));
-    if (e == hipSuccess) e = hipMalloc(&c->b_cand_keys, cand * sizeof(unsigned long long));
+    hipError_t e = vk::device_malloc(&c->b_ray, paths * 2 * sizeof(float4));
+    if (e == hipSuccess) e = vk::device_malloc(&c->b_thr, paths * sizeof(float4));
+    if (e == hipSuccess) e = vk::device_malloc(&c->b_rad, paths * sizeof(float4));
+    if (e == hipSuccess) e = vk::device_malloc(&c->b_nee, paths * sizeof(float4));
+    if (e == hipSuccess) e = vk::device_malloc(&c->b_hits, paths * sizeof(vk::HitRec));
+    if (e == hipSuccess) e = vk::device_malloc(&c->b_q0, paths * sizeof(uint32_t));
+    if (e == hipSuccess) e = vk::device_malloc(&c->b_q1, paths * sizeof(uint32_t));
+    if (e == hipSuccess) e = vk::device_malloc(&c->b_order, paths * sizeof(uint32_t));
+    if (e == hipSuccess) e = vk::device_malloc(&c->b_squeue, paths * sizeof(uint32_t));
+    if (e == hipSuccess) e = vk::device_malloc(&c->b_qsort, paths * sizeof(uint32_t));
+    if (e == hipSuccess) e = vk::device_malloc(&c->b_bins, 2 * vk::kRayBins * sizeof(uint32_t));
+    if (e == hipSuccess) e = vk::device_malloc(&c->b_counters, vk::kBatchCounterWords * sizeof(uint32_t));
+    if (e == hipSuccess) e = vk::device_malloc(&c->b_keys, paths * sizeof(unsigned long long));
+    if (e == hipSuccess) e = vk::device_malloc(&c->b_defer, cand * sizeof(uint4));
+    if (e == hipSuccess) e = vk::device_malloc(&c->b_cand_hits, cand * sizeof(vk::HitRec));
+    if (e == hipSuccess) e = vk::device_malloc(&c->b_cand_keys, cand * sizeof(unsigned long long));
     if (e != hipSuccess) {
         free_batch_scratch(c);
         return hip_fail(c, e, "batch scratch");
@@ -472,7 +472,7 @@ int ensure_batch_scratch(vkhrt_context* c, size_t paths) {
 // Device view table (+ frame values) and its pinned staging buffer.
 int ensure_batch_tables(vkhrt_context* c, uint32_t nviews) {
     if (!c->b_frame) {
-        hipError_t e = hipMalloc(&c->b_frame, sizeof(vk::BatchFrame));
+        hipError_t e = vk::device_malloc(&c->b_frame, sizeof(vk::BatchFrame));
         if (e == hipSuccess && !c->b_upload) e = hipEventCreateWithFlags(&c->b_upload, hipEventDisableTiming);
         if (e != hipSuccess) return hip_fail(c, e, "batch frame");
     }
@@ -481,7 +481,7 @@ int ensure_batch_tables(vkhrt_context* c, uint32_t nviews) {
         c->b_views = nullptr;
         c->b_views_cap = 0;
         ++c->batch_gen;
-        hipError_t e = hipMalloc(&c->b_views, size_t(nviews) * sizeof(vk::BatchView));
+        hipError_t e = vk::device_malloc(&c->b_views, size_t(nviews) * sizeof(vk::BatchView));
         if (e != hipSuccess) return hip_fail(c, e, "batch views");
         c->b_views_cap = nviews;
     }
@@ -539,11 +539,11 @@ int vkhrt_context_create(int device, vkhrt_context** out) {
         return VKHRT_ERROR_OUT_OF_MEMORY;
     }
     hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipMalloc(&c->status, 16);
-    if (e == hipSuccess) e = hipMalloc(&c->counters, vk::kRenderCounterWords * sizeof(uint32_t));
+    if (e == hipSuccess) e = vk::device_malloc(&c->status, 16);
+    if (e == hipSuccess) e = vk::device_malloc(&c->counters, vk::kRenderCounterWords * sizeof(uint32_t));
     if (e == hipSuccess) e = hipMemset(c->status, 0, 16);
 #ifdef VKHRT_WORK_COUNTERS
-    if (e == hipSuccess) e = hipMalloc(&c->work_counts, vk::kWorkCounters * sizeof(unsigned long long));
+    if (e == hipSuccess) e = vk::device_malloc(&c->work_counts, vk::kWorkCounters * sizeof(unsigned long long));
     if (e == hipSuccess) e = hipMemset(c->work_counts, 0, vk::kWorkCounters * sizeof(unsigned long long));
 #endif
     if (e != hipSuccess) {
@@ -703,11 +703,11 @@ int build_voxels(vkhrt_context* c, const vkhrt_blas_desc* d, hipStream_t st, vkh
     uint32_t* blocks = nullptr;
     uint32_t* scratch = nullptr;  // [0] overflow, [1] filled count, [2..7] bounds keys
     int rc = VKHRT_SUCCESS;
-    hipError_t e = hipMalloc(&scratch, 8 * sizeof(uint32_t));
+    hipError_t e = vk::device_malloc(&scratch, 8 * sizeof(uint32_t));
     if (e == hipSuccess) e = hipMemsetAsync(scratch, 0, 8 * sizeof(uint32_t), st);
     if (e == hipSuccess && d->count) {
         if (d->flags & VKHRT_BLAS_HOST_POINTERS) {
-            e = hipMalloc(&lines, line_bytes);
+            e = vk::device_malloc(&lines, line_bytes);
             if (e == hipSuccess) e = hipMemcpyAsync(lines, d->primitives, line_bytes, hipMemcpyHostToDevice, st);
             own = true;
         } else {
@@ -743,7 +743,7 @@ int build_voxels(vkhrt_context* c, const vkhrt_blas_desc* d, hipStream_t st, vkh
     if (g.count) {
         uint32_t overflow = 0;
         const size_t words = (size_t(g.count) + 31) / 32;
-        e = hipMalloc(&bits, words * sizeof(uint32_t));
+        e = vk::device_malloc(&bits, words * sizeof(uint32_t));
         if (e == hipSuccess) e = hipMemsetAsync(bits, 0, words * sizeof(uint32_t), st);
         if (e == hipSuccess)
             e = vk::voxelize_lines(lines, d->count, g, d->radius, (d->flags & VKHRT_BLAS_VOXEL_REFERENCE_SWEEP) != 0,
@@ -763,7 +763,7 @@ int build_voxels(vkhrt_context* c, const vkhrt_blas_desc* d, hipStream_t st, vkh
             const int32_t cres[3] = {(res[0] + 1) / 2, (res[1] + 1) / 2, (res[2] + 1) / 2};
             const size_t cwords = (size_t(cres[0]) * size_t(cres[1]) * size_t(cres[2]) + 31) / 32;
             uint32_t* coarse = nullptr;
-            e = hipMalloc(&coarse, cwords * sizeof(uint32_t));
+            e = vk::device_malloc(&coarse, cwords * sizeof(uint32_t));
             if (e == hipSuccess) e = vk::voxel_downsample(bits, res, coarse, cres, st);
             if (e == hipSuccess) e = hipStreamSynchronize(st);
             if (e != hipSuccess) {
@@ -797,9 +797,9 @@ int build_voxels(vkhrt_context* c, const vkhrt_blas_desc* d, hipStream_t st, vkh
         const size_t bwords = (size_t(bres[0]) * size_t(bres[1]) * size_t(bres[2]) + 31) / 32;
         const size_t kwords = (size_t(kres[0]) * size_t(kres[1]) * size_t(kres[2]) + 31) / 32;
         uint32_t* half = nullptr;
-        e = hipMalloc(&half, hwords * sizeof(uint32_t));
-        if (e == hipSuccess) e = hipMalloc(&bricks, bwords * sizeof(uint32_t));
-        if (e == hipSuccess) e = hipMalloc(&blocks, kwords * sizeof(uint32_t));
+        e = vk::device_malloc(&half, hwords * sizeof(uint32_t));
+        if (e == hipSuccess) e = vk::device_malloc(&bricks, bwords * sizeof(uint32_t));
+        if (e == hipSuccess) e = vk::device_malloc(&blocks, kwords * sizeof(uint32_t));
         if (e == hipSuccess) e = vk::voxel_downsample(bits, res, half, hres, st);
         if (e == hipSuccess) e = vk::voxel_downsample(half, hres, bricks, bres, st);
         if (e == hipSuccess) e = vk::voxel_downsample(bricks, bres, half, h2res, st);
@@ -910,9 +910,9 @@ int vkhrt_blas_build(vkhrt_context* c, const vkhrt_blas_desc* d, void* stream, v
     int rc = VKHRT_SUCCESS;
     if (d->count) {
         if (d->flags & VKHRT_BLAS_HOST_POINTERS) {
-            e = hipMalloc(&input, in_bytes);
+            e = vk::device_malloc(&input, in_bytes);
             if (e == hipSuccess) e = hipMemcpyAsync(input, d->primitives, in_bytes, hipMemcpyHostToDevice, st);
-            if (e == hipSuccess && mesh) e = hipMalloc(&indices, idx_bytes);
+            if (e == hipSuccess && mesh) e = vk::device_malloc(&indices, idx_bytes);
             if (e == hipSuccess && mesh) e = hipMemcpyAsync(indices, d->indices, idx_bytes, hipMemcpyHostToDevice, st);
             own_input = true;
         } else {
@@ -926,13 +926,13 @@ int vkhrt_blas_build(vkhrt_context* c, const vkhrt_blas_desc* d, void* stream, v
         if (d->mode == VKHRT_GEOMETRY_PHANTOM_CURVES) {
             records = input;
         } else if (d->mode == VKHRT_GEOMETRY_LSS) {
-            e = hipMalloc(&records, size_t(d->count) * 2 * sizeof(float4));
+            e = vk::device_malloc(&records, size_t(d->count) * 2 * sizeof(float4));
             if (e == hipSuccess) e = vk::lss_chain(input, d->count, records, st);
         } else if (mesh) {
             uint32_t nbad = 0;
-            e = hipMalloc(&records, size_t(d->count) * 3 * sizeof(float4));
-            if (e == hipSuccess) e = hipMalloc(&b->normals, size_t(d->count) * 3 * sizeof(float4));
-            if (e == hipSuccess) e = hipMalloc(&bad, sizeof(uint32_t));
+            e = vk::device_malloc(&records, size_t(d->count) * 3 * sizeof(float4));
+            if (e == hipSuccess) e = vk::device_malloc(&b->normals, size_t(d->count) * 3 * sizeof(float4));
+            if (e == hipSuccess) e = vk::device_malloc(&bad, sizeof(uint32_t));
             if (e == hipSuccess) e = hipMemsetAsync(bad, 0, sizeof(uint32_t), st);
             if (e == hipSuccess)
                 e = vk::gen_tri_records(reinterpret_cast<const float*>(input), d->vertex_count, indices, d->count,
@@ -945,7 +945,7 @@ int vkhrt_blas_build(vkhrt_context* c, const vkhrt_blas_desc* d, void* stream, v
                 goto out;
             }
         } else {
-            e = hipMalloc(&records, size_t(d->count) * 4 * sizeof(float4));
+            e = vk::device_malloc(&records, size_t(d->count) * 4 * sizeof(float4));
             if (e == hipSuccess) e = vk::gen_dots(input, d->count, per_point ? -1.0f : d->radius, records, st);
         }
         if (e != hipSuccess) {
@@ -1144,7 +1144,7 @@ int vkhrt_tlas_build(vkhrt_context* c, const vkhrt_blas* const* blases, uint32_t
     }
     if (count) {
         hipStream_t st = pick(c, stream);
-        hipError_t e = hipMalloc(&t->dev, sizeof(vk::InstanceDev) * count);
+        hipError_t e = vk::device_malloc(&t->dev, sizeof(vk::InstanceDev) * count);
         if (e == hipSuccess)
             e = hipMemcpyAsync(t->dev, inst.data(), sizeof(vk::InstanceDev) * count, hipMemcpyHostToDevice, st);
         if (e == hipSuccess) e = hipStreamSynchronize(st);
@@ -1978,7 +1978,7 @@ int vkhrt_generate_mesh_lines(vkhrt_context* c, const float* v, uint32_t nv, con
     hipStream_t st = pick(c, stream);
     uint32_t* bad = nullptr;
     uint32_t nbad = 0;
-    hipError_t e = hipMalloc(&bad, sizeof(uint32_t));
+    hipError_t e = vk::device_malloc(&bad, sizeof(uint32_t));
     if (e == hipSuccess) e = hipMemsetAsync(bad, 0, sizeof(uint32_t), st);
     if (e == hipSuccess) e = vk::gen_mesh_lines(v, nv, idx, n, radius, reinterpret_cast<float4*>(lines), bad, st);
     if (e == hipSuccess) e = hipMemcpyAsync(&nbad, bad, sizeof(uint32_t), hipMemcpyDeviceToHost, st);
@@ -2031,14 +2031,14 @@ int vkhrt_asset_build(vkhrt_context* c, const vkhrt_asset* a, const vkhrt_asset_
             g.done = true;
             g.count = hair ? ni / 2 : ni / 3;
             if (g.count) {
-                hipError_t e = hipMalloc(&g.verts, M.vertices.size() * sizeof(float));
+                hipError_t e = vk::device_malloc(&g.verts, M.vertices.size() * sizeof(float));
                 if (e == hipSuccess)
                     e = hipMemcpyAsync(g.verts, M.vertices.data(), M.vertices.size() * sizeof(float),
                                        hipMemcpyHostToDevice, st);
-                if (e == hipSuccess) e = hipMalloc(&g.idx, size_t(ni) * sizeof(uint32_t));
+                if (e == hipSuccess) e = vk::device_malloc(&g.idx, size_t(ni) * sizeof(uint32_t));
                 if (e == hipSuccess)
                     e = hipMemcpyAsync(g.idx, M.indices.data(), size_t(ni) * sizeof(uint32_t), hipMemcpyHostToDevice, st);
-                if (e == hipSuccess && hair) e = hipMalloc(&g.lines, size_t(g.count) * 8 * sizeof(float));
+                if (e == hipSuccess && hair) e = vk::device_malloc(&g.lines, size_t(g.count) * 8 * sizeof(float));
                 if (e != hipSuccess) {
                     rc = hip_fail(c, e, "asset upload");
                     break;
@@ -2052,7 +2052,7 @@ int vkhrt_asset_build(vkhrt_context* c, const vkhrt_asset* a, const vkhrt_asset_
                         g.recs = g.lines;
                     } else if (rc == VKHRT_SUCCESS) {
                         const bool curves = d->hair_mode == VKHRT_GEOMETRY_PHANTOM_CURVES;
-                        e = hipMalloc(&g.recs, size_t(g.count) * (curves ? 16 : 8) * sizeof(float));
+                        e = vk::device_malloc(&g.recs, size_t(g.count) * (curves ? 16 : 8) * sizeof(float));
                         if (e != hipSuccess) rc = hip_fail(c, e, "asset records");
                         else if (curves) rc = vkhrt_generate_curves(c, g.lines, g.count, d->tension, g.recs, stream);
                         else rc = vkhrt_generate_lss(c, g.lines, g.count, d->radius, g.recs, stream);
@@ -2121,11 +2121,11 @@ int vkhrt_shadow_mlp_create(vkhrt_context* c, const vkhrt_shadow_mlp_desc* d, vk
     std::memcpy(m->dev.center, center, sizeof(center));
     std::memcpy(m->dev.inv_half, inv_half, sizeof(inv_half));
     const size_t P = vk::kMlpParamCount;
-    e = hipMalloc(&m->dev.master, P * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(&m->dev.adam_m, P * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(&m->dev.adam_v, P * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(&m->dev.packed, 120 * 256 * sizeof(uint16_t));
-    if (e == hipSuccess) e = hipMalloc(&m->loss, sizeof(float));
+    e = vk::device_malloc(&m->dev.master, P * sizeof(float));
+    if (e == hipSuccess) e = vk::device_malloc(&m->dev.adam_m, P * sizeof(float));
+    if (e == hipSuccess) e = vk::device_malloc(&m->dev.adam_v, P * sizeof(float));
+    if (e == hipSuccess) e = vk::device_malloc(&m->dev.packed, 120 * 256 * sizeof(uint16_t));
+    if (e == hipSuccess) e = vk::device_malloc(&m->loss, sizeof(float));
     if (e != hipSuccess) {
         vkhrt_shadow_mlp_destroy(m);
         return hip_fail(c, e, "MLP buffers");
@@ -2191,7 +2191,8 @@ int vkhrt_shadow_mlp_collect(vkhrt_context* c, const vkhrt_tlas* t, const vkhrt_
     if (count == 0) return VKHRT_SUCCESS;
     hipStream_t st = pick(c, stream);
     vk::HitRec* hits = nullptr;
-    hipError_t e = hipMallocAsync(reinterpret_cast<void**>(&hits), size_t(count) * sizeof(vk::HitRec), st);
+    hipError_t e = vk::MemPool::retry_trimmed(
+        [&] { return hipMallocAsync(reinterpret_cast<void**>(&hits), size_t(count) * sizeof(vk::HitRec), st); });
     if (e != hipSuccess) return hip_fail(c, e, "collect scratch");
     int rc = vkhrt_trace_rays(c, t, rays, count, reinterpret_cast<vkhrt_hit*>(hits), VKHRT_TRACE_TERMINATE_ON_FIRST_HIT,
                               stream);
@@ -2216,7 +2217,7 @@ int mlp_run(vkhrt_context* c, vkhrt_shadow_mlp* m, const float* samples, const f
         hipFree(m->partial);
         m->partial = nullptr;
         m->partial_blocks = 0;
-        hipError_t e = hipMalloc(&m->partial, size_t(blocks) * vk::kMlpParamCount * sizeof(float));
+        hipError_t e = vk::device_malloc(&m->partial, size_t(blocks) * vk::kMlpParamCount * sizeof(float));
         if (e != hipSuccess) return hip_fail(c, e, "MLP partials");
         m->partial_blocks = blocks;
     }

@@ -13,8 +13,20 @@ namespace vk {
 // and streams: a block is handed to one owner at a time and comes back idle.
 class MemPool {
 public:
-    explicit MemPool(int device) : device_(device) {}
-    ~MemPool() { close(); }
+    explicit MemPool(int device) : device_(device) {
+        std::lock_guard<std::mutex> g(pools().m);
+        next_ = pools().first;
+        pools().first = this;
+    }
+    ~MemPool() {
+        {
+            std::lock_guard<std::mutex> g(pools().m);
+            MemPool** p = &pools().first;
+            while (*p != this) p = &(*p)->next_;
+            *p = next_;
+        }
+        close();
+    }
     MemPool(const MemPool&) = delete;
     MemPool& operator=(const MemPool&) = delete;
 
@@ -24,7 +36,7 @@ public:
     };
 
     // A block of at least `bytes` bytes on the pool's device (the current one); of the kept blocks
-    // the smallest that fits and is at most a quarter larger. When memory runs out the kept blocks are freed first.
+    // the smallest that fits and is at most a quarter larger.
     hipError_t acquire(size_t bytes, Block* out) {
         {
             std::lock_guard<std::mutex> g(m_);
@@ -41,14 +53,27 @@ public:
             }
         }
         out->bytes = bytes;
-        hipError_t e = hipMalloc(&out->p, bytes);
-        if (e == hipErrorOutOfMemory) {
-            (void)hipGetLastError();
-            trim();
-            e = hipMalloc(&out->p, bytes);
-        }
+        const hipError_t e = retry_trimmed([&] { return hipMalloc(&out->p, bytes); });
         if (e != hipSuccess) *out = Block{};
         return e;
+    }
+
+    // `alloc()`, an allocation on the current device, and when memory runs out once more after the
+    // blocks that the pools of all contexts keep on the device are freed: what is kept for the next
+    // build must not fail a call that would have had the memory without the pools.
+    template <class F>
+    static hipError_t retry_trimmed(F&& alloc) {
+        hipError_t e = alloc();
+        if (e != hipErrorOutOfMemory) return e;
+        (void)hipGetLastError();
+        int device = 0;
+        (void)hipGetDevice(&device);
+        {
+            std::lock_guard<std::mutex> g(pools().m);
+            for (MemPool* p = pools().first; p; p = p->next_)
+                if (p->device_ == device) p->trim();
+        }
+        return alloc();
     }
 
     // Takes a block back. Without `idle` the GPU may still be using it; like hipFree this then
@@ -109,11 +134,27 @@ private:
     static constexpr size_t kMinBytes = size_t(1) << 20, kMaxBytes = size_t(1) << 30, kSlack = 4096;
     static constexpr int kMaxBlocks = 8;
 
+    struct Pools {
+        std::mutex m;
+        MemPool* first = nullptr;
+    };
+    static Pools& pools() {  // the process's pools
+        static Pools p;
+        return p;
+    }
+
+    MemPool* next_ = nullptr;
     std::mutex m_;
     Block kept_[kMaxBlocks];
     int count_ = 0;
     bool closed_ = false;
     const int device_;
 };
+
+// hipMalloc for all device memory of the library that is not a pool's.
+template <class T>
+hipError_t device_malloc(T** p, size_t bytes) {
+    return MemPool::retry_trimmed([&] { return hipMalloc(reinterpret_cast<void**>(p), bytes); });
+}
 
 }  // namespace vk
