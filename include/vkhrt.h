@@ -124,7 +124,8 @@ typedef struct vkhrt_blas_info {
     uint32_t leaf_records;    /* curves / capsules / DOTS pieces / filled voxels */
     uint32_t node_count;      /* 8-wide nodes */
     uint32_t depth;           /* 8-wide levels */
-    uint64_t device_bytes;
+    uint64_t device_bytes;    /* device memory that the BLAS holds (blocks reused from an earlier
+                                 build are up to a quarter larger than needed) */
     double build_ms;
 } vkhrt_blas_info;
 

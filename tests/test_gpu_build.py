@@ -91,6 +91,22 @@ def test_blocks_pass_from_build_to_build(G, oracle):
         b.close()
 
 
+def test_device_bytes_counts_the_blocks(G):
+    """What a BLAS holds: its nodes with room for a sixteenth more, records and ids; a smaller one that
+    takes over the blocks of a destroyed one holds as much."""
+    import vkhrt_amd as V
+    ctx = V.Context(0)
+    held = []
+    for n in (200000, 190000):
+        blas = G.build_blas(ctx, V.GEOMETRY_LSS, capsules(n, 9))
+        info = blas.info()
+        held.append(info["device_bytes"])
+        assert held[-1] >= n * 36 + info["node_count"] * 85
+        blas.close()
+    assert held[0] == held[1] < 200000 * (36 + 85)
+    ctx.close()
+
+
 def test_builds_in_two_threads(G, oracle):
     import torch
     import vkhrt_amd as V

@@ -981,9 +981,8 @@ int vkhrt_blas_build(vkhrt_context* c, const vkhrt_blas_desc* d, void* stream, v
     b->info.primitive_count = d->mode == VKHRT_GEOMETRY_DOTS ? d->count * 4u : d->count;
     b->info.node_count = b->bvh.nnodes;
     b->info.depth = b->bvh.depth;
-    b->info.device_bytes = uint64_t(b->bvh.nnodes) * sizeof(vk::WideNode) + uint64_t(d->count) * 4u +
-                           uint64_t(d->count) * (d->mode == VKHRT_GEOMETRY_LSS ? 32u : mesh ? 96u : 64u) +
-                           (d->mode == VKHRT_GEOMETRY_PHANTOM_CURVES ? uint64_t(d->count) * 4u : 0u);
+    for (const vk::MemPool::Block& m : b->bvh.mem) b->info.device_bytes += m.bytes;
+    if (b->normals) b->info.device_bytes += uint64_t(d->count) * 3 * sizeof(float4);
 out:
     if (own_input) {
         hipFree(input);
