@@ -74,11 +74,47 @@ def test_equal_keys(gpu_ctx, G, oracle, leaf):
     blas.close()
 
 
+@pytest.mark.parametrize("collapse,width,leaf", [(2, 8, 1), (4, 8, 3), (1, 5, 2), (2, 4, 3), (4, 7, 1), (0, 4, 1), (0, 5, 3),
+                                                 (0, 7, 2)])
+def test_collapse_rules(G, oracle, collapse, width, leaf):
+    """The SAH-optimal collapse (costs per round, the slots it records) and the greedy one at the
+    widths and leaf sizes that the options allow: every record is in the tree and found."""
+    import vkhrt_amd as V
+    ctx = V.Context(0)
+    ctx.set_option(V.OPTION_BVH_COLLAPSE, collapse)
+    ctx.set_option(V.OPTION_BVH_WIDTH, width)
+    for n in (1, 2, 9, 129, 4097, 3000):
+        caps = capsules(n, n, same=n == 3000)  # 3000: equal sort keys
+        blas = G.build_blas(ctx, V.GEOMETRY_LSS, caps, leaf_size=leaf)
+        info = blas.info()
+        assert info["node_count"] >= -(-n // (width * leaf)) and (n == 1 or info["node_count"] < n)
+        check(ctx, G, oracle, caps, blas, f"{n} records, collapse {collapse}, width {width}, leaves of {leaf}")
+        blas.close()
+    ctx.close()
+
+
+def test_collapse_rules_give_other_trees(G):
+    """The options reach the build: the SAH rule and the width change the tree."""
+    import vkhrt_amd as V
+    ctx = V.Context(0)
+    counts = {}
+    for collapse, width in ((0, 8), (4, 8), (0, 4), (4, 4)):
+        ctx.set_option(V.OPTION_BVH_COLLAPSE, collapse)
+        ctx.set_option(V.OPTION_BVH_WIDTH, width)
+        blas = G.build_blas(ctx, V.GEOMETRY_LSS, capsules(20000, 3), leaf_size=3)
+        counts[collapse, width] = blas.info()["node_count"]
+        blas.close()
+    assert len(set(counts.values())) == 4, counts
+    ctx.close()
+
+
 def test_blocks_pass_from_build_to_build(G, oracle):
+    """Sizes that grow and shrink, all above the least that the pool keeps (1 MiB: 6000 records of
+    scratch, 30000 of records), then more sizes than it holds blocks, so that the oldest go."""
     import vkhrt_amd as V
     ctx = V.Context(0)
     keep = []
-    for k, n in enumerate([5000, 5200, 70000, 300, 5100, 66000, 5000]):
+    for k, n in enumerate([70000, 72000, 150000, 300, 71000, 140000, 70000] + [30000 * 4 ** i // 3 ** i for i in range(6)]):
         caps = capsules(n, 100 + k)
         blas = G.build_blas(ctx, V.GEOMETRY_LSS, caps)
         keep.append((caps, blas))
@@ -111,7 +147,8 @@ def test_builds_in_two_threads(G, oracle):
     import torch
     import vkhrt_amd as V
     ctx = V.Context(0)
-    sets = [[capsules(4000 + 500 * i, 10 * t + i) for i in range(4)] for t in range(2)]
+    # scratch of 12 to 17 MB, records of 2 to 3 MB and nodes of 1 MB or more: all blocks are pooled
+    sets = [[capsules(70000 + 9000 * i, 10 * t + i) for i in range(4)] for t in range(2)]
     dev = [[G.dev(c) for c in s] for s in sets]
     streams = [torch.cuda.Stream() for _ in sets]
     torch.cuda.synchronize()

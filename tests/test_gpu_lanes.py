@@ -102,15 +102,15 @@ def test_negative_tmin(gpu_ctx, G, oracle, curves, mode):
     G.compare_hits(G.trace(gpu_ctx, tlas, rays), ref, f"{mode}, negative tmin")
 
 
-@pytest.mark.parametrize("count", [65535, 65536, 65537])
-def test_shared_out_and_claimed_rays_agree(gpu_ctx, G, curves, count):
+@pytest.mark.parametrize("more", [-1, 0, 1])
+def test_shared_out_and_claimed_rays_agree(gpu_ctx, G, curves, more):
     """As many rays as a grid of one block per CU has lanes, one fewer and one more: shared out
     evenly up to there, claimed from counters beyond; the default grid shares out all three."""
     import scenes
     import torch
     import vkhrt_amd as V
     tlas = V.TopLevelAccelerationStructure(gpu_ctx, [G.build_blas(gpu_ctx, V.GEOMETRY_PHANTOM_CURVES, curves, per_point=True)])
-    assert torch.cuda.get_device_properties(0).multi_processor_count == 256
+    count = torch.cuda.get_device_properties(0).multi_processor_count * 256 + more
     rays = scenes.targeted_rays(curves, count, seed=37, dist=(1.0, 60.0))
     for flags in (V.TRACE_FP64_POLISH, V.TRACE_TERMINATE_ON_FIRST_HIT):
         ref = G.trace(gpu_ctx, tlas, rays, flags=flags)
