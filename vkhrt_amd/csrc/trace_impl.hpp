@@ -67,19 +67,6 @@ __device__ __forceinline__ unsigned long long best_key(const TraceParams& tp, co
     return (static_cast<unsigned long long>(__float_as_uint(b.t)) << 32) |
            (b.inst == 0xFFFFFFFFu ? 0xFFFFFFFFu : tp.inst[b.inst].blas.gbase + b.pid);
 }
-// Instance of a global primitive id: the last instance whose gbase is <= gid.
-__device__ __forceinline__ uint32_t gid_instance(const InstanceDev* inst, uint32_t ninst, uint32_t gid) {
-    uint32_t lo = 0, hi = ninst;  // gbase(lo) <= gid < gbase(hi)
-    while (hi - lo > 1u) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (inst[mid].blas.gbase <= gid)
-            lo = mid;
-        else
-            hi = mid;
-    }
-    return lo;
-}
-
 __device__ __forceinline__ bool better(float t, uint32_t inst, uint32_t pid, const Best& B) {
     if (t < B.t) return true;
     if (t == B.t) return inst < B.inst || (inst == B.inst && pid < B.pid);
@@ -129,9 +116,6 @@ struct TravStats {
 
 enum StepResult { kStepMore = 0, kStepDone = 1, kStepHit = 2, kStepError = 3 };
 
-// Resumable traversal of one BLAS by one lane: begin() sets up the ray, each step() visits
-// one 8-wide node (and tests its leaf primitives) and selects the next node. Used whole by
-// traverse() and one step per iteration by the persistent kernels.
 // Tests the 8 children of one node against [tmin, tcur]: `hits` gets the internal children
 // hit (bit j ^ octant for slot j, so lowest-bit-first is near-to-far), `pmask` the leaf
 // records hit (relative to the node's prim base).
@@ -203,6 +187,8 @@ __device__ __forceinline__ void node_visit(const WideNode* nodes, uint32_t node,
     }
 }
 
+// Traversal of one BLAS by one lane, for traverse() (one thread per ray): begin() sets up the ray,
+// each step() visits one 8-wide node, tests its leaf primitives and selects the next node.
 template <int MODE, int RMODE, bool POLISH, bool ANY, int STACK, bool STATS = false>
 struct Walker {
     f3 o, d, inv;
