@@ -214,3 +214,24 @@ def test_any_hit_record_is_the_rays_own(gpu_ctx, G, oracle, curves, modes):
         assert mixed.tobytes() == ref.tobytes()
         cut = 4099
         assert G.trace(gpu_ctx, tlas, rays[:cut], flags=flags).tobytes() == ref[:cut].tobytes()
+
+
+def test_work_counters_tell_leaf_rounds_from_steps():
+    """The counting build's tool: records are tested in leaf rounds of at most 64, whose cycles are not
+    the steps'. (In a process of its own, which loads the counting library.)"""
+    import json
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-m", "vkhrt_amd.workcount", "--frames", "1", "--strands", "3000", "--width", "320",
+                        "--height", "240"], cwd=root, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
+    out = json.loads(r.stdout.strip().splitlines()[-1])
+    for kind in ("primary", "shadow"):
+        c = out[kind]["per_frame"]
+        assert 0 < c["leaf_rounds"] <= c["leaf_tests"] <= 64 * c["leaf_rounds"]
+        assert c["node_tests"] <= c["step_lanes"] and c["cycles_leaf"] > 0 and c["cycles_steps"] > 0
+        share = out[kind]["cycle_share"]
+        assert abs(sum(share.values()) - 1.0) < 1e-3 and share["leaf_rounds"] > 0
+        assert c["rounds"] + c["leaf_rounds"] <= c["iterations"]

@@ -55,19 +55,22 @@ struct TraceParams {
 // group shadow walker from kWorkWave), wave-level sums over the persistent loop:
 enum WorkCounter {
     kWcIterations = 0,   // loop iterations of all waves
-    kWcRounds = 1,       // intersection rounds (iterations that run Prhi on the queued pairs)
-    kWcSteps = 2,        // traversal-step iterations
+    kWcRounds = 1,       // Prhi rounds (iterations that run the rest of Prhi on the queued pairs)
+    kWcSteps = 2,        // traversal steps (node tests)
     kWcNodeTests = 3,    // lanes that tested a node in a step
-    kWcLeafTests = 4,    // lanes that ran a leaf record's early-out test in a step
+    kWcLeafTests = 4,    // records tested in leaf rounds (phantom: the early-out)
     kWcPairs = 5,        // (ray, record) pairs that passed the early-out (Prhi calls)
-    kWcRoundLanes = 6,   // lanes busy in intersection rounds (sum of the pairs per round)
-    kWcCyclesRounds = 7, // shader clock cycles spent in rounds, summed over waves
+    kWcRoundLanes = 6,   // lanes busy in Prhi rounds (sum of the pairs per round)
+    kWcCyclesRounds = 7, // shader clock cycles spent in Prhi rounds, summed over waves
     kWcCyclesSteps = 8,  // ... in traversal steps
     kWcCyclesOther = 9,  // ... in refill, instance selection, tail hand-over and sinks
     kWcWaves = 10,       // waves that ran the loop
     kWcRays = 11,        // rays finished
     kWcHandovers = 12,   // stacked node groups handed to idle lanes (tail splitting)
-    kWcStepLanes = 13,   // lanes walking (node test or leaf test) summed over step iterations
+    kWcStepLanes = 13,   // lanes walking summed over the steps
+    kWcLeafRounds = 14,  // leaf rounds (iterations that test queued leaf records)
+    kWcCyclesLeaf = 15,  // cycles spent in them
+    kWcCount = 16
 };
 constexpr uint32_t kWorkAnyHit = 16, kWorkWave = 32, kWorkCounters = 48;
 // lane-group shadow walker: kWorkWave + 0 rays, 1 group iterations, 2 node tests, 3 leaf records tested,

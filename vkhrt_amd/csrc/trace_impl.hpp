@@ -1243,7 +1243,7 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
         return uint32_t(kk) != kNoHitLow && (!ORDERED || uint32_t(kk >> 32) < n);
     };
 #ifdef VKHRT_WORK_COUNTERS
-    unsigned long long wc[14] = {};  // WorkCounter sums of this wave (wave-uniform)
+    unsigned long long wc[kWcCount] = {};  // WorkCounter sums of this wave (wave-uniform)
     unsigned long long t_it = clock64(), t_mid = t_it;
     wc[kWcWaves] = 1;
 #define VK_WC(i, v) (wc[i] += (unsigned long long)(v))
@@ -1507,6 +1507,7 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
         // (e) leaf round on up to 64 records, one per lane
         if (ln >= 64u || (stuck && ln != 0u)) {
             const uint32_t m = ln < 64u ? ln : 64u;
+            VK_WC(kWcLeafRounds, 1);
             VK_WC(kWcLeafTests, m);
             const uint32_t slot = lane < m ? leaf[ln - m + lane] : 0u;
             const int owner = lane < m ? int(leaf_lane[ln - m + lane]) : 0;
@@ -1566,7 +1567,7 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
                 __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
                 __builtin_amdgcn_wave_barrier();
             }
-            VK_WC_END(kWcCyclesSteps);
+            VK_WC_END(kWcCyclesLeaf);
             continue;
         }
         // (f) traversal steps, one node test per walking lane each; the leaf records hit are queued.
@@ -1631,7 +1632,7 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
 #ifdef VKHRT_WORK_COUNTERS
     if (lane == 0 && tp.work_counts) {
         const uint32_t base = ANY ? kWorkAnyHit : 0u;
-        for (int i = 0; i < 14; ++i)
+        for (int i = 0; i < kWcCount; ++i)
             if (wc[i]) atomicAdd(&tp.work_counts[base + i], wc[i]);
     }
 #endif

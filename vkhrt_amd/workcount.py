@@ -6,8 +6,8 @@ of the library (libvkhrt_count.so: the same kernels compiled with VKHRT_WORK_COU
 Renders the frame (100,000 seeded strands x 32 tapered segments, 1920x1080, a shadow ray per
 hit, FP64 polish) and prints one JSON object: per frame and per traversal kind (closest hit,
 any hit, and with --area 1 the lane-group walker of the 16M-segment area-light frame's neural
-fallback) the loop iterations, intersection rounds, traversal steps, node and leaf tests, Prhi
-calls, lane use and the shares of shader-clock cycles spent in rounds, steps and bookkeeping.
+fallback) the loop iterations, Prhi rounds, leaf rounds, traversal steps, node and leaf tests, Prhi
+calls, lane use and the shares of shader-clock cycles spent in each kind and in bookkeeping.
 The counters add clock reads and atomics to the kernels, so their frame times are not the
 product's; the counts are those of the product kernels (same code paths).
 """
@@ -21,23 +21,26 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, os.path.dirname(HERE))
 
 NAMES = ["iterations", "rounds", "steps", "node_tests", "leaf_tests", "prhi_calls", "round_lanes", "cycles_rounds",
-         "cycles_steps", "cycles_other", "waves", "rays", "handovers", "step_lanes"]
+         "cycles_steps", "cycles_other", "waves", "rays", "handovers", "step_lanes", "leaf_rounds", "cycles_leaf"]
 WAVE_NAMES = ["rays", "steps", "node_tests", "leaf_tests", "prhi_calls", "record_steps", "cycles"]
 
 
 def summarize(raw, base, frames):
     c = {k: raw[base + i] / frames for i, k in enumerate(NAMES)}
-    cyc = c["cycles_rounds"] + c["cycles_steps"] + c["cycles_other"]
+    cyc = c["cycles_rounds"] + c["cycles_leaf"] + c["cycles_steps"] + c["cycles_other"]
     rays = max(c["rays"], 1.0)
     return {
         "per_frame": {k: round(v, 1) for k, v in c.items()},
         "per_ray": {k: round(c[k] / rays, 3) for k in ("node_tests", "leaf_tests", "prhi_calls", "iterations")},
         "lane_use": {"steps": round(c["step_lanes"] / max(64 * c["steps"], 1), 4),
+                     "leaf_rounds": round(c["leaf_tests"] / max(64 * c["leaf_rounds"], 1), 4),
                      "rounds": round(c["round_lanes"] / max(64 * c["rounds"], 1), 4)},
         "cycle_share": {"rounds": round(c["cycles_rounds"] / max(cyc, 1), 4),
+                        "leaf_rounds": round(c["cycles_leaf"] / max(cyc, 1), 4),
                         "steps": round(c["cycles_steps"] / max(cyc, 1), 4),
                         "other": round(c["cycles_other"] / max(cyc, 1), 4)},
         "iteration_share": {"rounds": round(c["rounds"] / max(c["iterations"], 1), 4),
+                            "leaf_rounds": round(c["leaf_rounds"] / max(c["iterations"], 1), 4),
                             "steps": round(c["steps"] / max(c["iterations"], 1), 4)},
     }
 
