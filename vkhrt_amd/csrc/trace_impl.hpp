@@ -122,15 +122,16 @@ enum StepResult { kStepMore = 0, kStepDone = 1, kStepHit = 2, kStepError = 3 };
 __device__ __forceinline__ void node_visit(const WideNode* nodes, uint32_t node, f3 o, f3 inv, uint32_t oct,
                                            float tmin, float tcur, uint32_t& hits, uint32_t& pmask,
                                            uint32_t& child_base, uint32_t& imask, uint32_t& pbase) {
+    constexpr float kDown = 1.0f / 16777216.0f;  // the slab test's scale of t, see below
     const bool nx = oct & 1u, ny = oct & 2u, nz = oct & 4u;
     const auto* np = gmem(reinterpret_cast<const uint4*>(nodes + node));
     const uint4 n0 = np[0], n1 = np[1], n2 = np[2], n3 = np[3], n4 = np[4];
     const float sx = __uint_as_float((n0.w & 0xffu) << 23) * inv.x;
     const float sy = __uint_as_float(((n0.w >> 8) & 0xffu) << 23) * inv.y;
     const float sz = __uint_as_float(((n0.w >> 16) & 0xffu) << 23) * inv.z;
-    const float ox = (__uint_as_float(n0.x) - o.x) * inv.x;
-    const float oy = (__uint_as_float(n0.y) - o.y) * inv.y;
-    const float oz = (__uint_as_float(n0.z) - o.z) * inv.z;
+    const float ox24 = (__uint_as_float(n0.x) - o.x) * (inv.x * kDown);
+    const float oy24 = (__uint_as_float(n0.y) - o.y) * (inv.y * kDown);
+    const float oz24 = (__uint_as_float(n0.z) - o.z) * (inv.z * kDown);
     imask = n0.w >> 24;
     child_base = n1.x;
     pbase = n1.y;
@@ -147,14 +148,13 @@ __device__ __forceinline__ void node_visit(const WideNode* nodes, uint32_t node,
     // beside two 32-bit ones: one byte permute prepares two planes, where a conversion each took
     // two instructions. So the test runs on t / 2^24: the other operands are scaled down to
     // match, since the scale times 2^24 would overflow for a ray parallel to an axis (inv = 1e20)
-    // in nodes wider than 5e13. (The scaled t lose bits where t < 2e-31: an error of at most 2.4e-38
-    // |d| in distance, far inside the boxes' padding.) About 230 -> 180 VALU instructions per node
+    // in nodes wider than 5e13. (The scaled values lose bits where t < 2e-31 or |d| > 5e30: an error
+    // of 2.4e-38 |d| in distance, far inside the boxes' padding.) About 230 -> 180 VALU instructions per node
     // test.
     // Each slot contributes one bit of a slot-order hit mask; the metadata is decoded afterwards
     // for the leaf slots hit only. Empty slots are not excluded: they are no internal child and
     // their metadata byte names no record.
-    constexpr float kDown = 1.0f / 16777216.0f;
-    const float ox24 = ox * kDown, oy24 = oy * kDown, oz24 = oz * kDown, tmin24 = tmin * kDown, tcur24 = tcur * kDown;
+    const float tmin24 = tmin * kDown, tcur24 = tcur * kDown;
     uint32_t lm = 0;
 #pragma unroll
     for (int h = 0; h < 4; ++h) {
