@@ -561,7 +561,8 @@ __device__ __forceinline__ uint32_t fexp_for(float extent) {
 // holds child e, so the opening, the slot order and the quantization run one child per lane in
 // registers. (One thread per node kept the eight boxes in scratch memory and walked them in
 // series: 2666 us for the 10 levels of 3.2M curves, 73 us per level even for a few nodes; now 772
-// and about 15. Bound by the chain of dependent loads while a node is opened.)
+// and about 15. Bound by the chain of dependent loads while a node is opened, at one block of 16
+// waves per CU: 82 registers, the SAH rule's stack among them.)
 // The nodes of a level are consecutive, bounds[level] .. bounds[level + 1], and tasks[w] is the
 // binary node that wide node w covers; a block allocates the children and leaf records of its 128
 // nodes with one atomic on the packed counter (nodes in the low, records in the high half): atomics

@@ -1003,9 +1003,12 @@ struct WorkClaim {
 // the iteration run for the few lanes that happen to sit at a leaf while the others wait: a leaf
 // hit is yielded by about every fifth node test, so nearly every step of a 64-lane wave had one.
 // 1080p frames of 100k strands, us, before (phantom: early-out tests inside the steps; LSS and
-// DOTS: whole tests inside the steps; several modes: one thread per ray) and now: phantom 1650 ->
-// 1426 (accurate), LSS 1306 -> 758, DOTS 1411 -> 789, hair on a mesh 6457 -> 1650; bound by the
-// VALU work of the node tests.
+// DOTS: whole tests inside the steps; several modes: one thread per ray) and now, with the even
+// shares and smaller claims of WorkClaim: phantom 1544 -> 1332 (accurate), LSS 1315 -> 719, DOTS
+// 1424 -> 756, hair on a mesh 6564 -> 1536. What bounds them: long launches of rays that fill the
+// lanes are VALU work (batched depth 0: 88 % busy, 3.6 of 4 waves per SIMD); a frame is that and a
+// tail of fewer rays than lanes (66 % busy, 2.6 waves, 43 % of the wave cycles waiting), and with
+// 16M curves the waits for nodes that no longer fit the L2 (48 %, 57 % waiting, L2 hits 21 %).
 // Results merge into the owner's LDS slot by a 64-bit atomicMin on (t, primitive) of the current
 // instance: that minimum is unique, so the closest hit and its tie rule do not depend on the
 // processing order. A lane does not move to its next instance, finish or take a new ray while
@@ -1642,8 +1645,11 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
 }
 
 // Waves per SIMD the persistent kernels are held to: the LDS of four 256-thread blocks (36.6-38.7 KB
-// each) fits a CU with stacks of up to 12 entries, so the registers have to stay at 128 there (left
-// alone some variants take 131-150 and run three waves).
+// each) fits a CU with stacks of up to 12 entries, so the registers have to stay at 128 there. Left
+// alone the variants take 131-150 and run three waves; held to 128 the primary kernels with deferred
+// polish spill 3 words per lane (one instance), 6 or 7 (several), which cost less: accurate 1080p
+// frame 1303 us against 1366, 16M curves 2173 against 2242, batch of 16 views 15.4 ms against 17.1.
+// (A 256x256 frame of 16k curves, all of it tail, takes 188 us against 175.)
 constexpr int lanes_waves(int stack) { return stack <= 12 ? 4 : 1; }
 
 // Persistent loop for one geometry variant.
