@@ -646,6 +646,8 @@ def roofline_block(ctx, tlas, cam, W, H, polish, kavg, sp, torch, np, V, accurat
         "unit": "GB/s",
         "frac": round(achieved / HBM_PEAK_GBS, 5),
         "traffic": traffic,
+        "traffic_source": "HBM bytes per launch counted in an earlier run of these kernels "
+                          "(profiles/render_primary_phantom_c1_traffic.md), not in this one" if traffic else None,
         "basis": "per ray 32 B ray + 16 B hit + 64 B x N*_prim (segments whose exact AABB "
                  "overlaps [tmin, t_closest])",
         "algorithmic_bytes": {"render_primary": b_primary, "render_shadow": b_shadow},
