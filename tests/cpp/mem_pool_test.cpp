@@ -14,7 +14,6 @@ namespace {
 std::mutex g_m;
 std::map<void*, std::pair<size_t, int>> g_live;  // size and device
 size_t g_used[2], g_limit[2] = {size_t(1) << 40, size_t(1) << 40};
-int g_syncs;
 thread_local int g_device;
 uintptr_t g_next = 4096;
 
@@ -60,15 +59,6 @@ hipError_t hipGetDevice(int* d) {
     *d = g_device;
     return hipSuccess;
 }
-hipError_t hipSetDevice(int d) {
-    g_device = d;
-    return hipSuccess;
-}
-hipError_t hipDeviceSynchronize(void) {
-    std::lock_guard<std::mutex> g(g_m);
-    ++g_syncs;
-    return hipSuccess;
-}
 hipError_t hipGetLastError(void) { return hipSuccess; }
 }
 
@@ -78,11 +68,20 @@ int main() {
         MemPool::Block a = get(p, 8 * MiB);
         void* first = a.p;
         p.release(a, true);
-        CHECK(g_syncs == 0 && live() == 1);
+        CHECK(live() == 1);
         a = get(p, 7 * MiB);
         CHECK(a.p == first && a.bytes == 8 * MiB);
-        p.release(a, false);  // not idle: waits
-        CHECK(g_syncs == 1 && live() == 1);
+        void* fence = nullptr;
+        CHECK(MemPool::make_fence(&fence) == hipSuccess && live() == 2);
+        p.release(a, MemPool::wait(fence));
+        CHECK(live() == 1);
+        a = get(p, 8 * MiB);
+        CHECK(a.p == first && !MemPool::wait(nullptr));
+        p.release(a, false);  // perhaps in use: not kept
+        CHECK(live() == 0);
+        a = get(p, 8 * MiB);
+        first = a.p;
+        p.release(a, true);
         MemPool::Block b = get(p, 9 * MiB), c = get(p, 4 * MiB);
         CHECK(b.p != first && c.p != first && live() == 3);
         p.release(b, true);

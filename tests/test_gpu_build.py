@@ -143,6 +143,67 @@ def test_device_bytes_counts_the_blocks(G):
     ctx.close()
 
 
+@pytest.mark.parametrize("mode,other", [("relaxed", False), ("relaxed", True), ("thread_local", True)])
+def test_destroyed_during_a_capture(G, mode, other):
+    """A BLAS that is destroyed while a graph is recorded, by this thread or another, leaves the capture
+    whole: every replay gives the eager records, with builds in the freed memory in between."""
+    import torch
+    import vkhrt_amd as V
+    ctx = V.Context(0)
+    caps = capsules(70000, 21)
+    tlas = V.TopLevelAccelerationStructure(ctx, [G.build_blas(ctx, V.GEOMETRY_LSS, caps)])
+    extra = G.build_blas(ctx, V.GEOMETRY_LSS, caps[::-1])
+    rays = G.dev(rays_at(caps, np.arange(5000), 6))
+    hits = torch.zeros(5000 * 8, dtype=torch.float32, device="cuda")
+
+    def trace():
+        ctx.trace_rays(tlas, rays.data_ptr(), 5000, hits.data_ptr(), 0, G.stream_ptr())
+
+    trace()
+    torch.cuda.synchronize()
+    ref = hits.cpu().numpy().tobytes()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, capture_error_mode=mode):
+        trace()
+        if other:
+            t = threading.Thread(target=extra.close)
+            t.start()
+            t.join()
+        else:
+            extra.close()
+    for k in range(3):
+        hits.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert hits.cpu().numpy().tobytes() == ref
+        G.build_blas(ctx, V.GEOMETRY_LSS, capsules(70000, 30 + k)).close()
+    ctx.close()
+
+
+def test_destroying_a_blas_waits_for_the_device(G):
+    """A BLAS's memory goes to the next build only when the GPU is done with it: its destruction waits
+    for work on any stream (here a copy loop of some 20 ms on a stream of its own)."""
+    import time
+    import torch
+    import vkhrt_amd as V
+    ctx = V.Context(0)
+    blas = G.build_blas(ctx, V.GEOMETRY_LSS, capsules(70000, 22))
+    a = torch.zeros(1 << 28, dtype=torch.float32, device="cuda")
+    stream = torch.cuda.Stream()
+    done = torch.cuda.Event()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        for _ in range(40):
+            a.add_(1.0)
+        done.record()
+    assert not done.query()
+    t0 = time.perf_counter()
+    blas.close()
+    waited = time.perf_counter() - t0
+    assert done.query() and waited > 1e-3
+    ctx.close()
+
+
 def test_builds_in_two_threads(G, oracle):
     import torch
     import vkhrt_amd as V

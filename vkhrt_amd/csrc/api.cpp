@@ -1028,8 +1028,10 @@ int vkhrt_blas_info_get(const vkhrt_blas* b, vkhrt_blas_info* out) {
 
 void vkhrt_blas_destroy(vkhrt_blas* b) {
     if (!b) return;
-    for (const vk::MemPool::Block& m : b->bvh.mem)
-        if (m.p) b->pool->release(m, false);
+    if (b->bvh.fence) {
+        const bool idle = vk::MemPool::wait(b->bvh.fence);
+        for (const vk::MemPool::Block& m : b->bvh.mem) b->pool->release(m, idle);
+    }
     hipFree(b->normals);
     hipFree(b->voxels);
     hipFree(b->vbricks);

@@ -19,7 +19,8 @@ struct BuiltBvh {
     uint32_t* slot_of = nullptr;  // phantom: leaf slot per original primitive id (the re-run of final hits)
     uint32_t depth = 0;       // wide levels
     WideNode root{};          // host copy of nodes[0]
-    MemPool::Block mem[2];    // the blocks that hold the arrays, for MemPool::release
+    MemPool::Block mem[2];    // the blocks that hold the arrays, for MemPool::release ...
+    void* fence = nullptr;    // ... and what is freed before them, to wait for the device
 };
 
 // Builds the 8-wide BVH over `n` primitive records (device pointer) on stream `st`, in memory of

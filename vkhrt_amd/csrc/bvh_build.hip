@@ -1009,6 +1009,7 @@ hipError_t build_bvh(int mode, const float4* prims_in, uint32_t n, int radius_mo
         }
         if (pass == 0) VK_TRY(pool.acquire(c.at, &records));
     }
+    VK_TRY(MemPool::make_fence(&built.fence));
 
     hipLaunchKernelGGL(k_init_bounds, dim3(1), dim3(64), 0, st, cb);
     hipLaunchKernelGGL(k_prim_boxes, dim3(std::min<uint32_t>(blocks(n), 2048u)), dim3(kBlock), 0, st, prims_in, n, mode,
@@ -1111,6 +1112,7 @@ hipError_t build_bvh(int mode, const float4* prims_in, uint32_t n, int radius_mo
     return hipSuccess;
 fail:
     if (rc == hipSuccess) rc = hipErrorUnknown;
+    (void)hipFree(built.fence);
     pool.release(scratch, false);
     pool.release(records, false);
     pool.release(node_block, false);

@@ -76,18 +76,21 @@ public:
         return alloc();
     }
 
-    // Takes a block back. Without `idle` the GPU may still be using it; like hipFree this then
-    // waits for the device. The blocks kept longest make room for it.
+    // A fence is a small allocation: an owner of blocks makes one with them and frees it before it
+    // gives them back, since freeing waits for the device. (hipDeviceSynchronize would wait too, but
+    // it ends a stream capture that is under way in the process, where hipFree does not: a program may
+    // destroy what it no longer needs while it, or another of its threads, records a graph.)
+    static hipError_t make_fence(void** f) {
+        return retry_trimmed([&] { return hipMalloc(f, 256); });
+    }
+    // Whether the device was waited for. A null fence: no.
+    static bool wait(void* fence) { return fence && hipFree(fence) == hipSuccess; }
+
+    // Takes a block back; the blocks kept longest make room for it. Without `idle` the GPU may still
+    // be using it: it is freed.
     void release(Block b, bool idle) {
         if (!b.p) return;
-        bool keep = b.bytes >= kMinBytes && b.bytes <= kMaxBytes;
-        if (keep && !idle) {
-            int cur = device_;
-            (void)hipGetDevice(&cur);
-            if (cur != device_) (void)hipSetDevice(device_);
-            keep = hipDeviceSynchronize() == hipSuccess;
-            if (cur != device_) (void)hipSetDevice(cur);
-        }
+        bool keep = idle && b.bytes >= kMinBytes && b.bytes <= kMaxBytes;
         Block old[kMaxBlocks];
         int n = 0;
         if (keep) {

@@ -2847,7 +2847,7 @@ hipError_t launch_render_variant(const RenderParams& rp, hipStream_t st, hipEven
                         scount = rp.counters + 5;
                     }
                     // the neural form's fallback queue is short: a queue of up to rp.wave_limit
-                    // rays is walked one ray per wavefront, a longer one by the persistent lanes
+                    // rays is walked by lane groups, a longer one by the persistent lanes
                     // (both kernels read the length on the device; one of them returns at once)
                     uint32_t skip = 0;
                     if constexpr (!G::kMixed && G::kMode == kPhantom) {
