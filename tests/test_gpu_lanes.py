@@ -163,7 +163,36 @@ def test_axis_parallel_rays_in_wide_scenes(gpu_ctx, G, oracle, half):
     rays[:, 7] = 3e38
     ref = S.trace(rays)
     assert (ref["prim"] != 0xFFFFFFFF).mean() > 0.9
-    G.compare_hits(G.trace(gpu_ctx, tlas, rays), ref, f"scene of +-{half:g}")
+    for persistent in (1, 0):
+        gpu_ctx.set_option(V.OPTION_PERSISTENT, persistent)
+        try:
+            G.compare_hits(G.trace(gpu_ctx, tlas, rays), ref, f"scene of +-{half:g}")
+            got = G.trace(gpu_ctx, tlas, rays, flags=V.TRACE_TERMINATE_ON_FIRST_HIT)
+        finally:
+            gpu_ctx.set_option(V.OPTION_PERSISTENT, 1)
+        assert np.array_equal(got["prim"] == 0xFFFFFFFF, ref["prim"] == 0xFFFFFFFF)
+
+
+@pytest.mark.parametrize("length", [1e-12, 1e15, 1e30, 1e36])
+def test_directions_of_any_length(gpu_ctx, G, oracle, length):
+    """t is in units of the direction's length; the node test keeps its bits down to the least normal
+    numbers (t near 1e-35 for a direction of 1e36). (Components below 1e-20 are taken for 1e-20: the
+    shortest length here keeps all but 1 in 10^8 of them above.)"""
+    import vkhrt_amd as V
+    rng = np.random.default_rng(45)
+    n = 4000
+    tri = rng.uniform(-50.0, 50.0, (n, 1, 3)) + rng.normal(size=(n, 3, 3)) * 0.3
+    S = oracle.Scene()
+    tlas = V.TopLevelAccelerationStructure(gpu_ctx, [_mesh(G, gpu_ctx, S, tri.reshape(-1, 3), np.arange(3 * n).reshape(n, 3))])
+    d = rng.normal(size=(n, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    rays = np.zeros((n, 8), np.float32)
+    rays[:, :3] = tri.mean(1) - d * rng.uniform(0.0, 60.0, (n, 1))
+    rays[:, 4:7] = d * length
+    rays[:, 7] = 3e38
+    ref = S.trace(rays)
+    assert (ref["prim"] != 0xFFFFFFFF).mean() > 0.9
+    G.compare_hits(G.trace(gpu_ctx, tlas, rays), ref, f"directions of {length:g}")
 
 
 def test_zero_distances_of_either_sign_are_equal(gpu_ctx, G, oracle):

@@ -156,6 +156,7 @@ struct vkhrt_tlas {
     int variant = vk::kVarMixed;  // kernel variant without FP64 polish
     uint32_t max_depth = 0;       // deepest BLAS (8-wide levels)
     bool polish_ok = true;        // merge keys and compacted-queue entries can encode every (instance, slot)
+    uint32_t trace_flags = 0;     // kTraceWide
     uint64_t serial = 0;          // unique per TLAS built in this process (graph reuse key)
     float lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};  // world bounds of all instances
     std::vector<uint32_t> records;  // leaf records per instance
@@ -203,8 +204,9 @@ uint64_t blas_id_range(const vkhrt_blas* b) {
 
 // Kernel variant for a TLAS and the polish flag. A TLAS of several BVH modes takes the persistent
 // lanes where they run (`lanes`); voxel instances have no BVH to walk, and leaf slots past the
-// queue encoding keep one thread per ray.
+// queue encoding keep one thread per ray. So do scenes too wide for the lanes' node test.
 int trace_variant(const vkhrt_tlas* t, bool polish, bool lanes) {
+    if (t->trace_flags & vk::kTraceWide) return vk::kVarMixed;
     int v = t->variant;
     if (v == vk::kVarMixed && lanes && t->polish_ok &&
         std::find(t->modes.begin(), t->modes.end(), uint32_t(VKHRT_GEOMETRY_VOXELS)) == t->modes.end())
@@ -1132,6 +1134,10 @@ int vkhrt_tlas_build(vkhrt_context* c, const vkhrt_blas* const* blases, uint32_t
                                                            : vk::kVarPhConst;
             v = (v < 0 || v == vi) ? vi : vk::kVarMixed;
             t->max_depth = std::max(t->max_depth, b->bvh.depth);
+            // the slab test's 2^24 * scale * 1e20 stays below 3.3e38 for scales up to 2^37; a node's exponent
+            // byte is at most one above its parent's
+            for (int k = 0; k < 3; ++k)
+                if (((b->bvh.root.e_imask >> (8 * k)) & 0xffu) > 127u + 36u) t->trace_flags = vk::kTraceWide;
             // the compacted phantom lanes queue (lane, leaf slot) pairs in 32 bits
             if (b->mode == VKHRT_GEOMETRY_PHANTOM_CURVES && b->records >= (1u << vk::kCompactSlotBits))
                 t->polish_ok = false;
@@ -1200,7 +1206,7 @@ int trace_launch(vkhrt_context* c, const vkhrt_tlas* t, const vkhrt_ray* rays, u
     flags &= ~uint32_t(VKHRT_TRACE_ACCURATE_NORMALS);
     // persistent phantom kernels compact intersection work through keys that need polish_ok
     const bool persistent = c->persistent && (t->polish_ok || !is_phantom(t));
-    vk::TraceParams tp{t->dev, t->count, flags, c->status, persistent ? s.work : nullptr, c->refill_min};
+    vk::TraceParams tp{t->dev, t->count, flags | t->trace_flags, c->status, persistent ? s.work : nullptr, c->refill_min};
     tp.work_counts = c->work_counts;
     tp.blocks_per_cu = c->blocks_per_cu;
     tp.xcd_chunk = c->xcd_chunk;
@@ -1304,7 +1310,8 @@ int vkhrt_render(vkhrt_context* c, const vkhrt_tlas* t, const vkhrt_camera* cam,
         std::memcpy(rp.light.v, al->edge_v, 12);
         rp.light.seed = al->seed;
     }
-    rp.tp = vk::TraceParams{t->dev, t->count, (d->flags & VKHRT_RENDER_FP64_POLISH) ? uint32_t(vk::kTraceFp64Polish) : 0u,
+    rp.tp = vk::TraceParams{t->dev, t->count,
+                            ((d->flags & VKHRT_RENDER_FP64_POLISH) ? uint32_t(vk::kTraceFp64Polish) : 0u) | t->trace_flags,
                             c->status, c->persistent && (t->polish_ok || !is_phantom(t)) ? c->counters + 1 : nullptr,
                             c->refill_min};
     rp.tp.blocks_per_cu = c->blocks_per_cu;
@@ -1482,7 +1489,7 @@ int vkhrt_render_batch(vkhrt_context* c, const vkhrt_tlas* t, const vkhrt_view* 
 
     const bool polish = (d->flags & VKHRT_BATCH_FP64_POLISH) && has_phantom(t);
     vk::BatchParams bp{};
-    bp.tp = vk::TraceParams{t->dev, t->count, polish ? uint32_t(vk::kTraceFp64Polish) : 0u, c->status,
+    bp.tp = vk::TraceParams{t->dev, t->count, (polish ? uint32_t(vk::kTraceFp64Polish) : 0u) | t->trace_flags, c->status,
                             c->b_counters, c->refill_min};
     bp.tp.blocks_per_cu = c->blocks_per_cu;
     bp.tp.xcd_chunk = c->xcd_chunk;
@@ -1836,7 +1843,7 @@ int vkhrt_trace_stats(vkhrt_context* c, const vkhrt_tlas* t, const vkhrt_ray* ra
     if (flags & ~VKHRT_TRACE_TERMINATE_ON_FIRST_HIT)
         return fail(c, VKHRT_ERROR_INVALID_ARGUMENT, "trace_stats supports only the any-hit flag");
     if (t->variant == vk::kVarMixed) return fail(c, VKHRT_ERROR_UNSUPPORTED, "trace_stats needs a single-mode TLAS");
-    vk::TraceParams tp{t->dev, t->count, flags, c->status, nullptr, 1u};
+    vk::TraceParams tp{t->dev, t->count, flags | t->trace_flags, c->status, nullptr, 1u};
     hipError_t e = vk::launch_trace_rays(tp, reinterpret_cast<const float*>(rays), count,
                                          reinterpret_cast<vk::HitRec*>(hits), reinterpret_cast<uint2*>(stats),
                                          t->variant, stack_kind_for(c, t), pick(c, stream));

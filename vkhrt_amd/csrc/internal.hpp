@@ -81,6 +81,7 @@ struct HitRec {
 enum TraceFlagsDev {
     kTraceAnyHit = 1u << 0,
     kTraceFp64Polish = 1u << 3,
+    kTraceWide = 1u << 16,  // set from the TLAS: some node is so wide that 2^24 times its scale may overflow
 };
 
 }  // namespace vk

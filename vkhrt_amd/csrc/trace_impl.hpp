@@ -78,6 +78,14 @@ __device__ __forceinline__ bool better(float t, uint32_t inst, uint32_t pid, con
 __device__ __forceinline__ float safe_rcp(float x) { return 1.0f / (fabsf(x) < 1e-20f ? copysignf(1e-20f, x) : x); }
 __device__ __forceinline__ f3 safe_inv(f3 d) { return f3{safe_rcp(d.x), safe_rcp(d.y), safe_rcp(d.z)}; }
 
+// The node test multiplies a node's scale by inv and by 2^24, which overflows for a ray parallel to an
+// axis (inv = 1e20) in nodes wider than 5e13. A TLAS that has such nodes (kTraceWide) is traced one
+// thread per ray, whose walker hands the test 1 / d, tmin and the current limit divided by 2^24: it then
+// runs on t / 2^24. (The persistent lanes do without: a check of each node's scale cost them 0.6 to 1 %,
+// testing on t / 2^24 always 0.7 % of a batch and the bits of t below 2e-31, scaling their rays by a
+// factor held in registers 0.7 % of a frame.)
+__device__ __forceinline__ float t_down(const TraceParams& tp) { return (tp.flags & kTraceWide) ? 1.0f / 16777216.0f : 1.0f; }
+
 // The same address as a global-memory pointer: loads through it are global_load, not flat
 // loads (a flat load also counts against the LDS counter, so waiting for an LDS access would
 // wait for it too). The BLAS arrays are device allocations.
@@ -122,16 +130,15 @@ enum StepResult { kStepMore = 0, kStepDone = 1, kStepHit = 2, kStepError = 3 };
 __device__ __forceinline__ void node_visit(const WideNode* nodes, uint32_t node, f3 o, f3 inv, uint32_t oct,
                                            float tmin, float tcur, uint32_t& hits, uint32_t& pmask,
                                            uint32_t& child_base, uint32_t& imask, uint32_t& pbase) {
-    constexpr float kDown = 1.0f / 16777216.0f;  // the slab test's scale of t, see below
     const bool nx = oct & 1u, ny = oct & 2u, nz = oct & 4u;
     const auto* np = gmem(reinterpret_cast<const uint4*>(nodes + node));
     const uint4 n0 = np[0], n1 = np[1], n2 = np[2], n3 = np[3], n4 = np[4];
     const float sx = __uint_as_float((n0.w & 0xffu) << 23) * inv.x;
     const float sy = __uint_as_float(((n0.w >> 8) & 0xffu) << 23) * inv.y;
     const float sz = __uint_as_float(((n0.w >> 16) & 0xffu) << 23) * inv.z;
-    const float ox24 = (__uint_as_float(n0.x) - o.x) * (inv.x * kDown);
-    const float oy24 = (__uint_as_float(n0.y) - o.y) * (inv.y * kDown);
-    const float oz24 = (__uint_as_float(n0.z) - o.z) * (inv.z * kDown);
+    const float ox = (__uint_as_float(n0.x) - o.x) * inv.x;
+    const float oy = (__uint_as_float(n0.y) - o.y) * inv.y;
+    const float oz = (__uint_as_float(n0.z) - o.z) * inv.z;
     imask = n0.w >> 24;
     child_base = n1.x;
     pbase = n1.y;
@@ -146,15 +153,12 @@ __device__ __forceinline__ void node_visit(const WideNode* nodes, uint32_t node,
     // widened by 8 ulp), so it uses fused multiply-adds. A byte placed in the low half of a 16-bit
     // float is the subnormal q * 2^-24 exactly, and v_fma_mix_f32 reads a 16-bit float operand
     // beside two 32-bit ones: one byte permute prepares two planes, where a conversion each took
-    // two instructions. So the test runs on t / 2^24: the other operands are scaled down to
-    // match, since the scale times 2^24 would overflow for a ray parallel to an axis (inv = 1e20)
-    // in nodes wider than 5e13. (The scaled values lose bits where t < 2e-31 or |d| > 5e30: an error
-    // of 2.4e-38 |d| in distance, far inside the boxes' padding.) About 230 -> 180 VALU instructions per node
-    // test.
+    // two instructions. The factor 2^24 goes into the scale. (About 230 -> 180 VALU instructions per
+    // node test.)
     // Each slot contributes one bit of a slot-order hit mask; the metadata is decoded afterwards
     // for the leaf slots hit only. Empty slots are not excluded: they are no internal child and
     // their metadata byte names no record.
-    const float tmin24 = tmin * kDown, tcur24 = tcur * kDown;
+    const float sx24 = sx * 16777216.0f, sy24 = sy * 16777216.0f, sz24 = sz * 16777216.0f;
     uint32_t lm = 0;
 #pragma unroll
     for (int h = 0; h < 4; ++h) {
@@ -163,11 +167,11 @@ __device__ __forceinline__ void node_visit(const WideNode* nodes, uint32_t node,
         const h2 az = qpair(nzl, nzh, h), bz = qpair(fzl, fzh, h);
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
-            const float t0x = fmaf(float(ax[k]), sx, ox24), t1x = fmaf(float(bx[k]), sx, ox24);
-            const float t0y = fmaf(float(ay[k]), sy, oy24), t1y = fmaf(float(by[k]), sy, oy24);
-            const float t0z = fmaf(float(az[k]), sz, oz24), t1z = fmaf(float(bz[k]), sz, oz24);
-            const float tn = fmaxf(fmaxf(t0x, t0y), fmaxf(t0z, tmin24));
-            const float tf = fminf(fminf(t1x, t1y), fminf(t1z, tcur24)) * 1.00000095f;
+            const float t0x = fmaf(float(ax[k]), sx24, ox), t1x = fmaf(float(bx[k]), sx24, ox);
+            const float t0y = fmaf(float(ay[k]), sy24, oy), t1y = fmaf(float(by[k]), sy24, oy);
+            const float t0z = fmaf(float(az[k]), sz24, oz), t1z = fmaf(float(bz[k]), sz24, oz);
+            const float tn = fmaxf(fmaxf(t0x, t0y), fmaxf(t0z, tmin));
+            const float tf = fminf(fminf(t1x, t1y), fminf(t1z, tcur)) * 1.00000095f;
             lm |= tn <= tf ? 1u << (2 * h + k) : 0u;
         }
     }
@@ -200,10 +204,10 @@ struct Walker {
     int sp;
     bool have_node;
 
-    __device__ __forceinline__ void begin(f3 o_, f3 d_) {
+    __device__ __forceinline__ void begin(f3 o_, f3 d_, float down) {
         o = o_;
         d = d_;
-        inv = safe_inv(d);
+        inv = scl(down, safe_inv(d));
         oct = uint32_t(signbit(d.x)) | (uint32_t(signbit(d.y)) << 1) | (uint32_t(signbit(d.z)) << 2);
         if (MODE == kPhantom) make_frame(o, d, F);
         if (MODE == kDots || MODE == kTriangles) TR = make_tri_ray(d);
@@ -219,7 +223,8 @@ struct Walker {
             if (node >= B.nnodes) return kStepError;  // malformed structure: report, never read out of bounds
             if (STATS) ++st->nodes;
             uint32_t hits, pmask, child_base, imask, pbase;
-            node_visit(B.nodes, node, o, inv, oct, tmin, best.t, hits, pmask, child_base, imask, pbase);
+            node_visit(B.nodes, node, o, inv, oct, tmin * t_down(tp), best.t * t_down(tp), hits, pmask, child_base, imask,
+                       pbase);
             // leaf primitives of this node
             if (pmask && pbase + (32u - __clz(pmask)) > B.nprims) return kStepError;
             while (pmask) {
@@ -355,7 +360,7 @@ __device__ __forceinline__ bool traverse(const BlasDev& B, f3 o, f3 d, float tmi
                                          TravStats* st = nullptr) {
     if (B.nprims == 0) return true;
     Walker<MODE, RMODE, POLISH, ANY, STACK, STATS> W;
-    W.begin(o, d);
+    W.begin(o, d, t_down(tp));
     for (;;) {
         const int r = W.step(B, tmin, inst, best, lds, st, tp, ray_id);
         if (r == kStepMore) continue;
@@ -1647,7 +1652,7 @@ __device__ __forceinline__ void persistent_compact(const TraceParams& tp, WorkCl
 // Waves per SIMD the persistent kernels are held to: the LDS of four 256-thread blocks (36.6-38.7 KB
 // each) fits a CU with stacks of up to 12 entries, so the registers have to stay at 128 there. Left
 // alone the variants take 131-150 and run three waves; held to 128 the primary kernels with deferred
-// polish spill 3 words per lane (one instance), 6 or 7 (several), which cost less: accurate 1080p
+// polish spill 3 words per lane (one instance), 6 to 8 (several), which cost less: accurate 1080p
 // frame 1303 us against 1366, 16M curves 2173 against 2242, batch of 16 views 15.4 ms against 17.1.
 // (A 256x256 frame of 16k curves, all of it tail, takes 188 us against 175.)
 constexpr int lanes_waves(int stack) { return stack <= 12 ? 4 : 1; }
