@@ -173,6 +173,51 @@ def test_axis_parallel_rays_in_wide_scenes(gpu_ctx, G, oracle, half):
         assert np.array_equal(got["prim"] == 0xFFFFFFFF, ref["prim"] == 0xFFFFFFFF)
 
 
+@pytest.mark.parametrize("mode", ["phantom", "lss"])
+def test_wide_scenes_take_their_own_route(gpu_ctx, G, oracle, curves, mode):
+    """Two records 1e14 units away make the scene wide, and the kernels others; what is near gives the same
+    records, statistics, frames (polished, accurate, with an area light) and path-traced images."""
+    import scenes
+    import torch
+    import vkhrt_amd as V
+    if mode == "phantom":
+        near, m = np.asarray(curves, np.float32).reshape(-1, 16), V.GEOMETRY_PHANTOM_CURVES
+        far = np.zeros((2, 4, 4), np.float32)
+        far[:, :, 0] = np.array([[1.0], [-1.0]]) * np.linspace(1e14, 1.1e14, 4)
+        far[:, :, 3] = 0.02
+        far = far.reshape(2, 16)
+    else:
+        near, m = oracle.generate_lss(scenes.lines_from_curves(curves, 4)).reshape(-1, 8), V.GEOMETRY_LSS
+        far = np.array([[1e14, 0, 0, 0.1, 1.1e14, 0, 0, 0.1], [-1e14, 0, 0, 0.1, -1.1e14, 0, 0, 0.1]], np.float32)
+    rays = scenes.targeted_rays(curves, 3000, seed=46, dist=(1.0, 60.0))
+    W, H = 160, 120
+    cam = V.camera_look_at((0.0, 20.0, 45.0), (0.0, 8.0, 0.0), fov_deg=60.0, aspect=W / H)
+    light = V.area_light((0.0, 60.0, 0.0), (20.0, 0.0, 0.0), (0.0, 0.0, 20.0), samples=2, seed=3)
+    polish = V.RENDER_SHADOWS | V.RENDER_FP64_POLISH
+    runs = []
+    for records in (near, np.concatenate([near, far])):
+        tlas = V.TopLevelAccelerationStructure(gpu_ctx, [G.build_blas(gpu_ctx, m, records, per_point=mode == "phantom")])
+        out = [G.trace(gpu_ctx, tlas, rays), G.trace(gpu_ctx, tlas, rays, V.TRACE_FP64_POLISH | V.TRACE_ACCURATE_NORMALS),
+               G.trace(gpu_ctx, tlas, rays, V.TRACE_TERMINATE_ON_FIRST_HIT)["prim"] == 0xFFFFFFFF]
+        for flags, al in ((polish, None), (polish | V.RENDER_ACCURATE_NORMALS, None), (polish, light)):
+            image = torch.zeros(W * H, dtype=torch.int32, device="cuda")
+            gpu_ctx.render(tlas, cam, W, H, image.data_ptr(), flags=flags | V.RENDER_RGBA8, area_light=al, stream=G.stream_ptr())
+            out.append(image.cpu().numpy())
+        image = torch.zeros(W * H, dtype=torch.int32, device="cuda")
+        gpu_ctx.render_batch(tlas, [(cam, W, H, image.data_ptr())], bounces=2, seed=5,
+                             flags=V.BATCH_RGBA8 | V.BATCH_FP64_POLISH, stream=G.stream_ptr())
+        out.append(image.cpu().numpy())
+        r, h = G.dev(rays), torch.zeros(len(rays) * 8, device="cuda")
+        st = torch.zeros(len(rays) * 2, dtype=torch.int32, device="cuda")
+        gpu_ctx.trace_stats(tlas, r.data_ptr(), len(rays), h.data_ptr(), st.data_ptr(), stream=G.stream_ptr())
+        out.append(h.cpu().numpy())
+        gpu_ctx.synchronize(G.stream_ptr())
+        runs.append(out)
+    assert (runs[0][0]["prim"] != 0xFFFFFFFF).mean() > 0.25
+    for k, (a, b) in enumerate(zip(*runs)):
+        assert a.tobytes() == b.tobytes(), k
+
+
 @pytest.mark.parametrize("length", [1e-12, 1e15, 1e30, 1e36])
 def test_directions_of_any_length(gpu_ctx, G, oracle, length):
     """t is in units of the direction's length; the node test keeps its bits down to the least normal
